@@ -593,6 +593,22 @@ typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u4 __attribute__((ext_vector_type(4)));
 typedef float fl4 __attribute__((ext_vector_type(4)));
 
+// Maximum over the lanes l, l^16, l^32, l^48, in every one of them.  The
+// swaps exchange 16-lane rows (1 of a with 0 of b, 3 with 2) and 32-lane
+// halves (the upper of a with the lower of b) of two registers on the VALU;
+// with the same value in both, each lane then holds its own and its
+// partner's.  (A shuffle goes through the LDS pipe and waits there behind
+// the block's tile traffic.  The builtins of these instructions return the
+// first register twice with the compiler at hand, hence the assembly; the
+// s_nop covers the wait states the instruction needs after a VALU write.)
+__device__ inline float max_lk(float v) {
+  float a = v, b = v;
+  asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+  a = b = fmaxf(a, b);
+  asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+  return fmaxf(a, b);
+}
+
 // Block fixed-point split of the 32 values of one K step (8 per lane, in the
 // 4 lanes l, l^16, l^32, l^48 that hold the same row or point): they share
 // one exponent e (2^(e-1) <= max |x| < 2^e) and each value becomes integers
@@ -608,8 +624,7 @@ __device__ inline void split3(const float (&x)[8], bf8& h, bf8& m, bf8& l) {
   float mx = 0.f;
 #pragma unroll
   for (int q = 0; q < 8; ++q) mx = fmaxf(mx, fabsf(x[q]));
-  mx = fmaxf(mx, __shfl_xor(mx, 16));
-  mx = fmaxf(mx, __shfl_xor(mx, 32));
+  mx = max_lk(mx);
   int e;
   (void)frexpf(mx, &e);
   // Adding and removing 1.5 * 2^(e+15) rounds a value of magnitude below 2^e
@@ -682,6 +697,92 @@ __device__ inline unsigned short float_to_bf16(float f) {
   unsigned u = __builtin_bit_cast(unsigned, f);
   u += 0x7fffu + ((u >> 16) & 1u);
   return (unsigned short)(u >> 16);
+}
+
+// Tiled planes (density variants 10 and 11): a plane is a sequence of tiles
+// of 16 points x 32 functions, the tiles of 16 points consecutive over the
+// functions, so that the B operand of one wave's K step (16 points, 32
+// functions) is one contiguous 2 KB run and each of its two loads one
+// contiguous 1 KB: lane (l % 16, l / 16) of the MFMA operand takes functions
+// 8 (l / 16) .. + 7 of point l % 16, the first four from the tile's first
+// half, the others from the second.  BF16 planes hold the eight functions of
+// a lane together.  (In the point-major planes a wave's load touched one line
+// in each of 16 rows m_pad values apart.)
+template <bool TL>
+__device__ inline long long pl_row(int mp, int pt) {
+  return TL ? (long long)(pt >> 4) * (16 * mp) + 4 * (pt & 15) : (long long)pt * mp;
+}
+template <bool TL>
+__device__ inline int pl_fn(int f) {  // f a multiple of 4
+  return TL ? ((f >> 5) << 9) + ((f & 4) << 6) + ((f & 24) << 3) : f;
+}
+__device__ inline long long tl16_row(int mp, int pt) {
+  return (long long)(pt >> 4) * (16 * mp) + 8 * (pt & 15);
+}
+__device__ inline int tl16_fn(int f) { return ((f >> 5) << 9) + ((f & 24) << 4) + (f & 7); }
+// The eight functions from f (a multiple of 8) of a lane's point.
+__device__ inline void load8t(const float* row, int f, float (&x)[8]) {
+  const float* p = row + pl_fn<true>(f);
+  const fl4 a = *reinterpret_cast<const fl4*>(p);
+  const fl4 b = *reinterpret_cast<const fl4*>(p + 256);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    x[q] = a[q];
+    x[4 + q] = b[q];
+  }
+}
+
+// The values of a block of 64 points and 32 functions into the tiled planes:
+// lane l of wave w holds point l and evaluates functions 4 w .. 4 w + 3 (the
+// function records wave-uniform), which are one 16-byte store per plane, 16
+// lanes a contiguous 256 bytes, with no transpose.  Also phi's remainder in
+// BF16 and the function-major phi plane of the Fock kernel (rows of 64
+// points).  Items as in k_eval_pm.
+template <int NV>
+__global__ __launch_bounds__(512) void k_eval_tl(const EvalItem* __restrict__ items,
+                                                 const DevGroup* __restrict__ groups,
+                                                 const int* __restrict__ fnl,
+                                                 const DevFn* __restrict__ bas,
+                                                 const double* __restrict__ px,
+                                                 const double* __restrict__ py,
+                                                 const double* __restrict__ pz,
+                                                 float* __restrict__ vals,
+                                                 float* __restrict__ phiT,
+                                                 unsigned short* __restrict__ lo16) {
+  const EvalItem it = items[blockIdx.x];
+  if (it.group < 0) return;
+  const DevGroup g = groups[it.group];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int p = it.p0 + lane;
+  if (p >= g.npts_pad) return;
+  const int q = g.pt_off + p;
+  const double x = px[q], y = py[q], z = pz[q];
+  const int k = it.k + 4 * wave;
+  const long long plane = (long long)g.m_pad * g.npts_pad;
+  float o[NV][4];
+  unsigned short l[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int f = fnl[g.fn_off + k + j];
+    double v[NV];
+    if (f >= 0) {
+      eval_basis<NV>(bas[f], x, y, z, v);
+    } else {
+#pragma unroll
+      for (int c = 0; c < NV; ++c) v[c] = 0.0;
+    }
+#pragma unroll
+    for (int c = 0; c < NV; ++c) o[c][j] = (float)v[c];
+    l[j] = float_to_bf16((float)(v[0] - (double)(float)v[0]));
+    phiT[g.phi_off + (long long)(k + j) * g.npts_pad + p] = o[0][j];
+  }
+  float* out = vals + g.val_off + pl_row<true>(g.m_pad, p) + pl_fn<true>(k);
+#pragma unroll
+  for (int c = 0; c < NV; ++c)
+    *reinterpret_cast<fl4*>(out + c * plane) = fl4{o[c][0], o[c][1], o[c][2], o[c][3]};
+  *reinterpret_cast<uint2*>(lo16 + g.phi_off + tl16_row(g.m_pad, p) + tl16_fn(k)) =
+      uint2{l[0] | ((unsigned)l[1] << 16), l[2] | ((unsigned)l[3] << 16)};
 }
 
 template <int NV, bool LO = false>
@@ -820,7 +921,13 @@ __device__ inline void radial_hessian(const FnMeta& mt, float vx, float vy, floa
 // (the 32 threads of a block are 32 consecutive lanes of one wave); a fourth
 // piece carries the next 8 bits (units of 2^(e-32)) for the products that
 // need P to 2^-32 of the block maximum.
-template <int NPC>
+// FRAG (the chunked density variants): the pieces in the order the density
+// kernel's A operand takes them, [16-row tile][32-column K block][piece]
+// [lane][8 columns], lane l holding row l % 16, columns 8 (l / 16) .. + 7: a
+// K step's tile of 16 rows is 4 KB in one run (rows m_pad values apart gave
+// half a line per row and step), copied to LDS as it stands and read there
+// by lane without bank conflicts.  A block covers 8 rows of one K block.
+template <int NPC, bool FRAG>
 __device__ __forceinline__ void gather_bf_item(const int bi, const GatherItem* __restrict__ items,
                                                            const DevGroup* __restrict__ groups,
                                                            const DevMol* __restrict__ mols,
@@ -833,8 +940,16 @@ __device__ __forceinline__ void gather_bf_item(const int bi, const GatherItem* _
   const long long psz = (long long)g.m_pad * g.m_pad;
   const bool in = e < psz;  // whole 32-lane blocks are in or out (m_pad % 32 == 0)
   double v = 0.0;
+  int k = 0, j = 0;
   if (in) {
-    const int k = e / g.m_pad, j = e % g.m_pad;
+    if constexpr (FRAG) {
+      const int blk = it.start / 256, nr = g.m_pad / 8;
+      k = 8 * (blk % nr) + (threadIdx.x >> 5);
+      j = 32 * (blk / nr) + (threadIdx.x & 31);
+    } else {
+      k = e / g.m_pad;
+      j = e % g.m_pad;
+    }
     v = density_entry(mols[g.mol], rho, fnl[g.fn_off + k], fnl[g.fn_off + j]);
   }
   double mx = fabs(v);
@@ -848,21 +963,25 @@ __device__ __forceinline__ void gather_bf_item(const int bi, const GatherItem* _
   const double r2 = (r1 - a1) * 256.0;
   const double a2 = rint(r2);
   if (!in) return;
-  __bf16* out = reinterpret_cast<__bf16*>(pgs) + NPC * g.pg_off + e;
+  const long long ps = FRAG ? 512 : psz;
+  __bf16* out = reinterpret_cast<__bf16*>(pgs) + NPC * g.pg_off;
+  out += FRAG ? ((long long)(k >> 4) * (g.m_pad >> 5) + (j >> 5)) * (512 * NPC) +
+                    (j & 24) * 16 + (k & 15) * 8 + (j & 7)
+              : (long long)e;
   out[0] = (__bf16)(float)ldexp(a0, ex - 8);
-  out[psz] = (__bf16)(float)ldexp(a1, ex - 16);
-  out[2 * psz] = (__bf16)(float)ldexp(a2, ex - 24);
-  if (NPC == 4) out[3 * psz] = (__bf16)(float)ldexp(rint((r2 - a2) * 256.0), ex - 32);
+  out[ps] = (__bf16)(float)ldexp(a1, ex - 16);
+  out[2 * ps] = (__bf16)(float)ldexp(a2, ex - 24);
+  if (NPC == 4) out[3 * ps] = (__bf16)(float)ldexp(rint((r2 - a2) * 256.0), ex - 32);
 }
 
-template <int NPC>
+template <int NPC, bool FRAG = false>
 __global__ __launch_bounds__(256) void k_gather_density_bf(const GatherItem* __restrict__ items,
                                                            const DevGroup* __restrict__ groups,
                                                            const DevMol* __restrict__ mols,
                                                            const int* __restrict__ fnl,
                                                            const double* __restrict__ rho,
                                                            unsigned short* __restrict__ pgs) {
-  gather_bf_item<NPC>(blockIdx.x, items, groups, mols, fnl, rho, pgs);
+  gather_bf_item<NPC, FRAG>(blockIdx.x, items, groups, mols, fnl, rho, pgs);
 }
 
 // Density + functional on split-BF16 MFMA: same blocking as k_density (64
@@ -1308,19 +1427,19 @@ __global__ __launch_bounds__(256) void k_split_pm(const DensityItem* __restrict_
   if (p0 >= g.npts_pad) return;  // whole waves (the splits exchange across lanes)
   const int np = g.npts_pad, mp = g.m_pad, pt = p0 + lrow;
   const long long plane = (long long)mp * np;
-  const float* Vp = vals + g.val_off + (long long)pt * mp;
-  const unsigned short* Vl = lo16 + g.phi_off + (long long)pt * mp;
-  unsigned short* Pc = pcs + 4 * g.phi_off + (long long)pt * mp;
+  const float* Vp = vals + g.val_off + pl_row<true>(mp, pt);
+  const unsigned short* Vl = lo16 + g.phi_off + tl16_row(mp, pt);
+  unsigned short* Pc = pcs + 4 * g.phi_off + tl16_row(mp, pt);
   for (int k0 = 0; k0 < mp; k0 += 32) {
     const int kk = k0 + 8 * lk;
     float x[8], xl[8];
-    load8(Vp + kk, x);
-    bf16x8_to_float(*reinterpret_cast<const u4*>(Vl + kk), xl);
+    load8t(Vp, kk, x);
+    bf16x8_to_float(*reinterpret_cast<const u4*>(Vl + tl16_fn(kk)), xl);
     bf8 b4[4];
     split4f(x, xl, b4);
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      *reinterpret_cast<u4*>(Pc + j * plane + kk) = __builtin_bit_cast(u4, b4[j]);
+      *reinterpret_cast<u4*>(Pc + j * plane + tl16_fn(kk)) = __builtin_bit_cast(u4, b4[j]);
   }
 }
 
@@ -1333,7 +1452,20 @@ __global__ __launch_bounds__(256) void k_split_pm(const DensityItem* __restrict_
 // Each block leaves its ten row-dot sums per point in cpart (one slot per
 // chunk) and k_density_cs_finish adds them in chunk order, then evaluates
 // the functional with one lane per point (the density blocks hold each point
-// on four lanes, a quarter of the wave).  (A last-block-finishes form, with
+// on four lanes, a quarter of the wave).
+//
+// What bounds it: the SIMDs' issue.  A K step is about 600 VALU instructions
+// (the split of the B operand) of 4 cycles and 112 MFMA of 16, and the two
+// overlap little on this GPU (two waves a SIMD alternating 384 FMA and 96
+// MFMA take 4.7 ms where the sum is 5.3, fully interleaved 4.1), so the time
+// is near their sum as long as the operands arrive.  The tiled planes and the
+// P_g tiles in operand order are for that: contiguous runs of 1 KB per load
+// instead of 16 rows, whole lines, no LDS bank conflicts, and the split's
+// lane maximum off the LDS pipe.  (H2O)32: 1.40 -> 1.11 ms, 195 atoms 37.5 ->
+// 34.4 ms (point-major planes and row-major P_g before), bitwise the same.
+// Two passes over taller chunks (phi, then the gradient: half the split
+// work, more P_g traffic) took 1.17 and 32.4 ms, s_setprio around the
+// products and other block orders moved it by 1 %.  (A last-block-finishes form, with
 // an agent-scope counter per tile, needs agent-scope fences in every block;
 // on this GPU they write back and invalidate the XCD's L2, which undid the
 // sharing: 9.0 ms against 1.4 ms.)
@@ -1361,9 +1493,8 @@ __global__ __launch_bounds__(256, 2) void k_density_cs(const ChunkItem* __restri
                                                        double* __restrict__ cpart,
                                                        const unsigned short* __restrict__ pcs) {
   constexpr int NS = (NT == 4) ? 10 : 1;
-  constexpr int ROWS = 64, RT = 4, NPC = 4;
-  constexpr int UNITS = NPC * ROWS * 4;  // 16-byte units of one staged P_g tile
-  __shared__ u4 sA[2][UNITS];            // [buf][piece][row][k octet]
+  constexpr int ROWS = 64, RT = 4;
+  __shared__ u4 sA[2][RT][4][64];  // [buf][16-row tile][piece][lane]
   const ChunkItem it = items[blockIdx.x];
   if (it.group < 0) return;  // padding of a short XCD list
   const DevGroup g = groups[it.group];
@@ -1373,51 +1504,46 @@ __global__ __launch_bounds__(256, 2) void k_density_cs(const ChunkItem* __restri
   const bool active = p0 < g.npts_pad;
   const int np = g.npts_pad, mp = g.m_pad, c0 = it.c0;
   const long long plane = (long long)mp * np;
-  const long long psz = (long long)mp * mp;
   const int pt = active ? p0 + lrow : it.p0;  // inactive waves still stage tiles
-  const float* Vp = vals + g.val_off + (long long)pt * mp;
-  const unsigned short* Vl = lo16 + g.phi_off + (long long)pt * mp;
-  const unsigned short* Pp = pg4 + NPC * g.pg_off;
-  // P_g tile of a K step: 16-byte unit c = threadIdx.x + 256 i is piece
-  // c / (4 ROWS), row (c / 4) % ROWS, k octet c % 4, loaded into registers
-  // before the step's products and written to LDS after them.  (Copied
-  // straight into LDS instead, the copy's completion has to be awaited
-  // before the next LDS instruction -- the split's cross-lane exchange --
-  // which left its latency exposed at every step.)  Rows past the group's
-  // functions are never read (their address is clamped to the last row).
-  u4 pa[UNITS / 256];
+  const float* Vp = vals + g.val_off + pl_row<true>(mp, pt);
+  const unsigned short* Vl = lo16 + g.phi_off + tl16_row(mp, pt);
+  const u4* Pp = reinterpret_cast<const u4*>(pg4 + 4 * g.pg_off);
+  const int nrt = min(RT, (mp - c0) / 16);
+  // P_g tiles of a K step (4 KB per 16 rows, in operand order), loaded into
+  // registers before the step's products and written to LDS after them.
+  // (Copied straight into LDS instead, the copy's completion has to be
+  // awaited before the next LDS instruction, which left its latency exposed
+  // at every step.)
+  u4 pa[RT];
   auto gload = [&](int k0) {
 #pragma unroll
-    for (int i = 0; i < UNITS / 256; ++i) {
-      const int c = threadIdx.x + 256 * i;
-      const int sp = c / (4 * ROWS), row = (c >> 2) & (ROWS - 1), oc = c & 3;
-      const int j = min(c0 + row, mp - 1);
-      pa[i] = *reinterpret_cast<const u4*>(Pp + sp * psz + (long long)j * mp + k0 + 8 * oc);
-    }
+    for (int i = 0; i < RT; ++i)
+      if (i < nrt)
+        pa[i] = Pp[((long long)(c0 / 16 + i) * (mp >> 5) + (k0 >> 5)) * 256 + threadIdx.x];
   };
   auto lstore = [&](int b) {
 #pragma unroll
-    for (int i = 0; i < UNITS / 256; ++i) sA[b][threadIdx.x + 256 * i] = pa[i];
+    for (int i = 0; i < RT; ++i)
+      if (i < nrt) (&sA[b][i][0][0])[threadIdx.x] = pa[i];
   };
-  const int nrt = min(RT, (mp - c0) / 16);
   f4 acc[RT][NT];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
     for (int t = 0; t < NT; ++t) acc[rt][t] = f4{0, 0, 0, 0};
-  const unsigned short* Pc = pcs + 4 * g.phi_off + (long long)pt * mp;  // PS
+  const unsigned short* Pc = pcs + 4 * g.phi_off + tl16_row(mp, pt);  // PS
   float xb[NT][8];      // the next step's FP32 values (plane 0 unused with PS)
   u4 xlp = u4{0, 0, 0, 0};
   u4 nb[PS ? 4 : 1];    // the next step's phi pieces (PS)
   if constexpr (PS) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) nb[j] = *reinterpret_cast<const u4*>(Pc + j * plane + 8 * lk);
+    for (int j = 0; j < 4; ++j) nb[j] = *reinterpret_cast<const u4*>(Pc + j * plane + tl16_fn(8 * lk));
   } else {
-    load8(Vp + 8 * lk, xb[0]);
-    xlp = *reinterpret_cast<const u4*>(Vl + 8 * lk);
+    load8t(Vp, 8 * lk, xb[0]);
+    xlp = *reinterpret_cast<const u4*>(Vl + tl16_fn(8 * lk));
   }
 #pragma unroll
-  for (int t = 1; t < NT; ++t) load8(Vp + t * plane + 8 * lk, xb[t]);
+  for (int t = 1; t < NT; ++t) load8t(Vp + t * plane, 8 * lk, xb[t]);
   gload(0);
   lstore(0);
   __syncthreads();
@@ -1440,28 +1566,26 @@ __global__ __launch_bounds__(256, 2) void k_density_cs(const ChunkItem* __restri
       gload(k0 + 32);
       if constexpr (PS) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) nb[j] = *reinterpret_cast<const u4*>(Pc + j * plane + kk + 32);
+        for (int j = 0; j < 4; ++j) nb[j] = *reinterpret_cast<const u4*>(Pc + j * plane + tl16_fn(kk + 32));
       } else {
-        load8(Vp + kk + 32, xb[0]);
-        xlp = *reinterpret_cast<const u4*>(Vl + kk + 32);
+        load8t(Vp, kk + 32, xb[0]);
+        xlp = *reinterpret_cast<const u4*>(Vl + tl16_fn(kk + 32));
       }
 #pragma unroll
-      for (int t = 1; t < NT; ++t) load8(Vp + t * plane + kk + 32, xb[t]);
+      for (int t = 1; t < NT; ++t) load8t(Vp + t * plane, kk + 32, xb[t]);
     }
     if (active) {
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
         if (rt < nrt) {
-          const int u = (16 * rt + lrow) * 4 + lk;
-          const bf8 ah = __builtin_bit_cast(bf8, sA[buf][u]);
-          const bf8 am = __builtin_bit_cast(bf8, sA[buf][ROWS * 4 + u]);
-          const bf8 al = __builtin_bit_cast(bf8, sA[buf][2 * ROWS * 4 + u]);
-          const bf8 a4[4] = {ah, am, al, __builtin_bit_cast(bf8, sA[buf][3 * ROWS * 4 + u])};
+          bf8 a4[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) a4[j] = __builtin_bit_cast(bf8, sA[buf][rt][j][lane]);
           f4 hi, lo;
           mma10(a4, b4, hi, lo);
           acc[rt][0] += hi + lo;
 #pragma unroll
-          for (int t = 1; t < NT; ++t) acc[rt][t] += mma6(ah, am, al, bh[t], bm[t], bl[t]);
+          for (int t = 1; t < NT; ++t) acc[rt][t] += mma6(a4[0], a4[1], a4[2], bh[t], bm[t], bl[t]);
         }
       }
     }
@@ -1476,14 +1600,16 @@ __global__ __launch_bounds__(256, 2) void k_density_cs(const ChunkItem* __restri
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt)
         if (rt < nrt)
-          *reinterpret_cast<fl4*>(ybuf + g.phi_off + (long long)pt * mp + c0 + 16 * rt + 4 * lk) =
+          *reinterpret_cast<fl4*>(ybuf + g.phi_off + pl_row<true>(mp, pt) +
+                                  pl_fn<true>(c0 + 16 * rt + 4 * lk)) =
               fl4{acc[rt][0][0], acc[rt][0][1], acc[rt][0][2], acc[rt][0][3]};
     }
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
       if (rt >= nrt) continue;
-      const float* vj = Vp + c0 + 16 * rt + 4 * lk;  // functions j .. j+3 of this point
-      const fl4 vlo = bf16x4_to_float(Vl + c0 + 16 * rt + 4 * lk);
+      const int j = c0 + 16 * rt + 4 * lk;
+      const float* vj = Vp + pl_fn<true>(j);  // functions j .. j+3 of this point
+      const fl4 vlo = bf16x4_to_float(Vl + tl16_fn(j));
       if constexpr (NT == 4) {
         fl4 v[10];
 #pragma unroll
@@ -1911,8 +2037,7 @@ __device__ inline void split4f(const float (&hi)[8], const float (&lo)[8], bf8 (
   float mx = 0.f;
 #pragma unroll
   for (int q = 0; q < 8; ++q) mx = fmaxf(mx, fabsf(hi[q]));
-  mx = fmaxf(mx, __shfl_xor(mx, 16));
-  mx = fmaxf(mx, __shfl_xor(mx, 32));
+  mx = max_lk(mx);
   int e;
   (void)frexpf(mx, &e);
   const float c0 = ldexpf(1.5f, e + 15), c1 = ldexpf(1.5f, e + 7), c2 = ldexpf(1.5f, e - 1),
@@ -2480,6 +2605,7 @@ __global__ __launch_bounds__(256, 2) void k_force_bf(const DensityItem* __restri
 // Split-BF16 forces from the Y = P_g phi the density kernel left in ybuf
 // (point-major, exact FP32 sums): the same per-function sums as k_force_bf,
 // in the same lane and wave order, without recomputing the product.
+template <bool TL>
 __global__ __launch_bounds__(256) void k_force_y(const DensityItem* __restrict__ items,
                                                  const DevGroup* __restrict__ groups,
                                                  const float* __restrict__ ybuf,
@@ -2495,7 +2621,7 @@ __global__ __launch_bounds__(256) void k_force_y(const DensityItem* __restrict__
   const bool active = p0 < g.npts_pad;  // uniform over the wave
   const int np = g.npts_pad, mp = g.m_pad;
   const long long plane = (long long)mp * np;
-  const long long prow = (long long)(active ? p0 + lrow : 0) * mp;
+  const long long prow = pl_row<TL>(mp, active ? p0 + lrow : 0);
   const float* Vp = vals + g.val_off + prow;
   const float* Yp = ybuf + g.phi_off + prow;
   const double f = active ? factor[g.pt_off + p0 + lrow] : 0.0;
@@ -2507,7 +2633,7 @@ __global__ __launch_bounds__(256) void k_force_y(const DensityItem* __restrict__
       fl4 y = fl4{0, 0, 0, 0};
       fl4 v[3] = {fl4{0, 0, 0, 0}, fl4{0, 0, 0, 0}, fl4{0, 0, 0, 0}};
       if (active && rt < nrt) {
-        const int j = c0 + 16 * rt + 4 * lk;  // functions j .. j+3 of this point
+        const int j = pl_fn<TL>(c0 + 16 * rt + 4 * lk);  // functions j .. j+3 of this point
         y = *reinterpret_cast<const fl4*>(Yp + j);
 #pragma unroll
         for (int a = 0; a < 3; ++a) v[a] = *reinterpret_cast<const fl4*>(Vp + j + (a + 1) * plane);
@@ -2939,7 +3065,7 @@ __global__ __launch_bounds__(256, 2) void k_build_persist(PersistArgs* pargs, in
     int* tdone = ddone + a.ngroups;
     if (it >= a.n5) break;
     if (it < a.n0) {
-      gather_bf_item<4>(it, a.gitems, a.groups, a.mols, a.fnl, rho, a.pg);
+      gather_bf_item<4, false>(it, a.gitems, a.groups, a.mols, a.fnl, rho, a.pg);
       persist_signal(&gdone[a.gitems[it].group]);
     } else if (it < a.n1) {
       const int d = it - a.n0, g = a.ditems[d].group;
@@ -4671,7 +4797,11 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
     } else {
       float* v = static_cast<float*>(dg->vals);
       if (dg->npm > 0) {
-        if (dg->lo && dg->gga)
+        if (dg->chunked)
+          hipLaunchKernelGGL(dg->gga ? k_eval_tl<10> : k_eval_tl<4>, dim3(dg->npm), dim3(512), 0,
+                             s, dg->pmitems, dg->groups, dg->fnl, dg->bas, dg->px, dg->py, dg->pz,
+                             v, dg->phiT, dg->lo16);
+        else if (dg->lo && dg->gga)
           hipLaunchKernelGGL((k_eval_pm<10, true>), dim3(dg->npm), dim3(512), 0, s,
                              dg->pmitems, dg->groups, dg->fnl, dg->bas, dg->px, dg->py, dg->pz, v,
                              dg->phiT, dg->lo16);
@@ -5316,8 +5446,9 @@ static void launch_density_bf(DeviceGrid& g, hipStream_t s, const double* d_rho,
     const bool four = g.density_variant == 8 || g.chunked;
     if (g.ngather > 0) {
       if (four)
-        hipLaunchKernelGGL(k_gather_density_bf<4>, dim3(g.ngather), dim3(256), 0, s, g.gitems,
-                           g.groups, g.mols, g.fnl, rho, pg3);
+        hipLaunchKernelGGL((g.chunked ? k_gather_density_bf<4, true> : k_gather_density_bf<4, false>),
+                           dim3(g.ngather), dim3(256), 0, s, g.gitems, g.groups, g.mols, g.fnl,
+                           rho, pg3);
       else
         hipLaunchKernelGGL(k_gather_density_bf<3>, dim3(g.ngather), dim3(256), 0, s, g.gitems,
                            g.groups, g.mols, g.fnl, rho, pg3);
@@ -5483,7 +5614,8 @@ static void launch_forces(DeviceGrid& g, hipStream_t s, double* d_forces) {
                            g.ybuf + (sp == 1 ? g.phi_elems : 0), g.fmeta, g.shells, g.tsh, g.bas,
                            g.px, g.py, g.pz, factor, g.gpart);
       else if (ystore_forces(g))
-        hipLaunchKernelGGL(k_force_y, dim3(g.nforce), dim3(256), 0, s, g.citems, g.groups,
+        hipLaunchKernelGGL(g.chunked ? k_force_y<true> : k_force_y<false>, dim3(g.nforce),
+                           dim3(256), 0, s, g.citems, g.groups,
                            g.ybuf + (sp == 1 ? g.phi_elems : 0),
                            static_cast<const float*>(g.vals), factor, g.gpart);
       else

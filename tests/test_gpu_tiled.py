@@ -1,0 +1,49 @@
+"""Tiled value planes and operand-ordered P_g of the chunked split-BF16
+density (variants 10 and 11), on the GPU, at the sizes where the layouts have
+edges: groups of one 32-function block, row counts that end inside a chunk,
+point counts that are not multiples of 64.
+
+The tiled layout holds the values of the point-major planes, P_g the same
+pieces, so every product is variant 8's; the FP64 epilogue sums differ in
+grouping only: 1e-10 on Exc, N, F and the forces, as for the chunked form's
+other comparisons.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SAME = 1e-10
+
+
+def _molecule(name):
+    from lio_amd import systems
+    if name == "water":
+        return systems.config0()
+    n, iexch = name
+    Z, pos = systems.random_molecule_ang(n, 50 + n)
+    return systems.make_system("mol%d" % n, Z, pos, seed=n, iexch=iexch)
+
+
+@pytest.mark.parametrize("grid_type", [0, 2])
+@pytest.mark.parametrize("name", ["water", (2, 9), (5, 9), (9, 9), (14, 3), (22, 9)])
+def test_tiled_layout_equals_point_major(name, grid_type):
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from lio_amd import g2g
+    s = _molecule(name)
+    out = {}
+    for variant in (8, 10, 11):
+        ctx = g2g.Context(s, precision="bf16x6")
+        ctx.set_schedule(density_variant=variant)
+        ctx.build_grid(grid_type)
+        F = np.zeros(s.M * (s.M + 1) // 2)
+        E, f, info = ctx.solve_forces(fock=F)
+        out[variant] = (E, info["electrons"], F, f)
+        ctx.close()
+    print("case", name, grid_type, out[10][0], out[10][0] - out[8][0], flush=True)
+    for a, b in zip(out[8], out[10]):
+        assert np.max(np.abs(np.asarray(a) - np.asarray(b))) <= SAME
+    for a, b in zip(out[10], out[11]):
+        assert np.array_equal(a, b)

@@ -2,16 +2,18 @@
 //
 // Grid build (once per geometry, like the reference's cached GPU groups,
 // g2g/cuda/iteration.cu:792-881):
-//   k_eval_basis       phi, grad phi and the Hessian of every significant basis
+//   k_eval_fm          phi, grad phi and the Hessian of every significant basis
 //                      function at every point of its group, written once to
-//                      HBM as planes [value][function][point] (points
-//                      contiguous, coalesced).  HBM-bound.
+//                      HBM as planes [value][16-point tile][function][16
+//                      points].  HBM-bound.
 // Per XC Fock build (one solve):
 //   k_gather_density   packed rho -> dense symmetric block P_g per group
-//   k_density          Y_t^T = P_g Phi_t^T for t = phi, d/dx, d/dy, d/dz on
-//                      FP64 MFMA (16x16x4), 64 points per block; row-dot
-//                      epilogue -> rho, grad rho, Hessian of rho -> PBE/LDA
-//                      -> factor_p = w_p v_p and per-block (Exc, N)
+//   k_density_dc       Y = P_g phi and the gradients' forms on FP64 MFMA
+//                      (16x16x4), one block per 64 points and 64 functions;
+//                      row-dot epilogue -> the block's share of rho, grad
+//                      rho, Hessian of rho
+//   k_density_cs_finish  the chunks' shares added, PBE/LDA
+//                      -> factor_p = w_p v_p and per-tile (Exc, N)
 //   k_fock             F_g tile (64 x 64) over a 512-point slice,
 //                      phi^T diag(factor) phi on FP64 MFMA, one partial/slice
 //   k_fock_group       sums the slices of each tile in fixed order
@@ -262,6 +264,56 @@ __global__ __launch_bounds__(256) void k_eval_basis(const EvalItem* __restrict__
   }
 }
 
+// Tiled planes of the FP64 and FP32 modes: a plane is the 16-point tiles of
+// the group, each m_pad functions x 16 points (points contiguous).  A wave's
+// operand of four functions and 16 points is one contiguous run (512 bytes in
+// FP64), consecutive functions follow each other, and a function's 16 points
+// are one line for the Fock kernel.  (Planes of m_pad x npts_pad put the rows
+// of a wave's operand npts_pad values apart.)
+__device__ inline long long fm_row(int mp, int p) {
+  return (long long)(p >> 4) * (16 * mp) + (p & 15);
+}
+
+// The values of 64 points and 16 functions: lane l of wave w holds point l and
+// evaluates functions 4 w .. 4 w + 3 (the function records wave-uniform).
+constexpr int kFmFns = 16;
+template <int NV, class T>
+__global__ __launch_bounds__(256) void k_eval_fm(const EvalItem* __restrict__ items,
+                                                 const DevGroup* __restrict__ groups,
+                                                 const int* __restrict__ fnl,
+                                                 const DevFn* __restrict__ bas,
+                                                 const double* __restrict__ px,
+                                                 const double* __restrict__ py,
+                                                 const double* __restrict__ pz,
+                                                 T* __restrict__ vals) {
+  const EvalItem it = items[blockIdx.x];
+  if (it.group < 0) return;
+  const DevGroup g = groups[it.group];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int p = it.p0 + lane;
+  if (p >= g.npts_pad) return;
+  const int q = g.pt_off + p;
+  const double x = px[q], y = py[q], z = pz[q];
+  const long long plane = (long long)g.m_pad * g.npts_pad;
+  T* row = vals + g.val_off + fm_row(g.m_pad, p);
+#pragma unroll
+  for (int j = 0; j < kFmFns / 4; ++j) {
+    const int k = it.k + 4 * wave + j;
+    const int f = fnl[g.fn_off + k];
+    double v[NV];
+    if (f >= 0) {
+      eval_basis<NV>(bas[f], x, y, z, v);
+    } else {
+#pragma unroll
+      for (int c = 0; c < NV; ++c) v[c] = 0.0;
+    }
+    T* out = row + 16 * k;
+#pragma unroll
+    for (int c = 0; c < NV; ++c) out[c * plane] = (T)v[c];
+  }
+}
+
 // ---------------------------------------------------------------------------
 // density blocks P_g[k][j] = P(f_k, f_j) with the true symmetric P
 // ---------------------------------------------------------------------------
@@ -275,6 +327,9 @@ __device__ inline double density_entry(const DevMol& mol, const double* __restri
   return lo != hi ? 0.5 * v : v;
 }
 
+// FP32: rows.  FP64: operand order, [16-row tile][8 columns][lane][2], lane l
+// holding row l % 16 and columns l / 16 and l / 16 + 4 of the eight: the two A
+// operands of a lane are one 16-byte load and a wave's load one 1 KB run.
 template <class T>
 __global__ __launch_bounds__(256) void k_gather_density(const GatherItem* __restrict__ items,
                                                         const DevGroup* __restrict__ groups,
@@ -286,7 +341,15 @@ __global__ __launch_bounds__(256) void k_gather_density(const GatherItem* __rest
   const DevGroup g = groups[it.group];
   const int e = it.start + threadIdx.x;
   if (e >= g.m_pad * g.m_pad) return;
-  const int k = e / g.m_pad, j = e % g.m_pad;
+  int k, j;
+  if constexpr (sizeof(T) == 8) {
+    const int u = e >> 7, nk8 = g.m_pad >> 3, l = (e >> 1) & 63;
+    k = 16 * (u / nk8) + (l & 15);
+    j = 8 * (u % nk8) + 4 * (e & 1) + (l >> 4);
+  } else {
+    k = e / g.m_pad;
+    j = e % g.m_pad;
+  }
   const double v = density_entry(mols[g.mol], rho, fnl[g.fn_off + k], fnl[g.fn_off + j]);
   pg[g.pg_off + e] = (T)v;
 }
@@ -346,7 +409,7 @@ __device__ inline void point_stage(const double* s, int q, int iexch, int spin,
 }
 
 // ---------------------------------------------------------------------------
-// density + functional: 64 points per block, 16 per wave
+// density + functional (FP32 mode): 64 points per block, 16 per wave
 // ---------------------------------------------------------------------------
 // Wave w owns points p0 = 64 b + 16 w (the 16 columns of its MFMA tiles) and
 // walks the functions in chunks of 64 (4 row tiles).  For each row tile rt
@@ -386,7 +449,7 @@ __global__ __launch_bounds__(256, 2) void k_density(const DensityItem* __restric
       for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
         for (int t = 0; t < NT; ++t) acc[rt][t] = typename Mma<T>::acc{0, 0, 0, 0};
-      const T* Bk = V + (long long)lk * np + p0 + lrow;   // Phi_t[k][p]
+      const T* Bk = V + fm_row(mp, p0 + lrow) + 16 * lk;   // Phi_t[k][p]
       const T* Ak = Pm + (long long)lk * mp + c0 + lrow;  // P[k][j] = P[j][k]
       // operands of step k0 in (a, b); the next step's are loaded before the
       // MFMAs of this one so the loads overlap the matrix pipe
@@ -400,7 +463,7 @@ __global__ __launch_bounds__(256, 2) void k_density(const DensityItem* __restric
         const bool more = k0 + 4 < mp;
         const long long kb = (long long)(more ? k0 + 4 : k0);
 #pragma unroll
-        for (int t = 0; t < NT; ++t) bn[t] = Bk[t * plane + kb * np];
+        for (int t = 0; t < NT; ++t) bn[t] = Bk[t * plane + kb * 16];
 #pragma unroll
         for (int rt = 0; rt < 4; ++rt) an[rt] = (rt < nrt) ? Ak[kb * mp + 16 * rt] : T(0);
 #pragma unroll
@@ -421,7 +484,7 @@ __global__ __launch_bounds__(256, 2) void k_density(const DensityItem* __restric
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int j = c0 + 16 * rt + Mma<T>::row(lk, i);
-          const T* vj = V + (long long)j * np + p0 + lrow;
+          const T* vj = V + fm_row(mp, p0 + lrow) + 16 * j;
           if constexpr (NT == 4) {
             double v[10];
 #pragma unroll
@@ -522,13 +585,13 @@ __global__ __launch_bounds__(256, 2) void k_fock(const FockItem* __restrict__ it
     V4 A[4], B[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      A[r] = (r < nri) ? *reinterpret_cast<const V4*>(V + (long long)(i0 + 16 * r + lrow) * np + p)
+      A[r] = (r < nri) ? *reinterpret_cast<const V4*>(V + fm_row(mp, p) + 16 * (i0 + 16 * r + lrow))
                        : V4{0, 0, 0, 0};
       if (diag)  // the same function rows on both sides: one load
         B[r] = A[r] * f;
       else
         B[r] = (r < nrj)
-                   ? *reinterpret_cast<const V4*>(V + (long long)(j0 + 16 * r + lrow) * np + p) * f
+                   ? *reinterpret_cast<const V4*>(V + fm_row(mp, p) + 16 * (j0 + 16 * r + lrow)) * f
                    : V4{0, 0, 0, 0};
     }
 #pragma unroll
@@ -1693,6 +1756,174 @@ __global__ __launch_bounds__(256) void k_density_cs_finish(const ChunkItem* __re
   }
 }
 
+// ---------------------------------------------------------------------------
+// FP64 density row-dot sums, one (64-point tile, 64-function chunk) per block
+// ---------------------------------------------------------------------------
+// With Y = P phi and the gradients' forms d_a phi^T P d_b phi, P symmetric: let
+// U_a[i] = sum over the 16-row blocks before i's of P d_a phi, plus half the
+// product with i's own (symmetric) diagonal block; then
+//   d_a phi^T P d_b phi = d_a phi . U_b + d_b phi . U_a,
+// so the three gradient products need only the blocks up to the diagonal:
+// 2 + 3 n m^2 flops instead of 8.  A block's K loop runs over slabs of 16
+// functions: before the chunk all four products, within it each row tile up
+// to its diagonal block, past it only phi's.  Wave w owns 16 points; the P_g
+// slab (operand order) goes through LDS once per block, the planes' operands
+// come straight into registers one slab ahead.  The ten sums per point go to
+// cpart and k_density_cs_finish adds the chunks and evaluates the functional.
+//
+// What bounds it: the FP64 unit for large groups (the matrix products keep it
+// busy 69 % of the time at 60 atoms, the epilogue's FMAs, which it shares with
+// them, another 7 %), HBM for small ones ((H2O)32: 9.1 GB at 5.1 TB/s, the
+// epilogue's ten planes and the K loop's four).  Against one block per tile
+// walking the chunks with four full products: (H2O)32 2.47 -> 1.83 ms, 60
+// atoms 8.9 -> 5.6 ms, 45 atoms LDA 0.89 -> 0.60 ms.  Taking the diagonal
+// blocks' share of the epilogue from the K loop's operands moves 6.5 GB
+// instead but needs the sums beside 128 accumulator and 64 operand registers:
+// 1.80 and 5.7 ms with them in LDS, 2.4 ms spilled; single-buffered operands
+// 1.94 ms, two waves per 16 points and four waves a SIMD 2.16 ms.
+template <int NT>
+__global__ __launch_bounds__(256, 2) void k_density_dc(const ChunkItem* __restrict__ items,
+                                                       const DevGroup* __restrict__ groups,
+                                                       const double* __restrict__ pg,
+                                                       const double* __restrict__ vals,
+                                                       double* __restrict__ cpart) {
+  constexpr int NS = (NT == 4) ? 10 : 1;
+  constexpr int RT = 4;
+  typedef double d2 __attribute__((ext_vector_type(2)));
+  __shared__ d2 sA[2][RT * 128];  // [buf][16-row tile][8-column half][lane]
+  const ChunkItem it = items[blockIdx.x];
+  if (it.group < 0) return;  // padding of a short XCD list
+  const DevGroup g = groups[it.group];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lrow = lane & 15, lk = lane >> 4;
+  const int p0 = it.p0 + 16 * wave;
+  const bool active = p0 < g.npts_pad;
+  const int mp = g.m_pad, nk = mp >> 4;
+  const int r0 = it.c0 >> 4, nrt = min(RT, nk - r0);
+  const long long plane = (long long)mp * g.npts_pad;
+  // wave-uniform pointers and a 32-bit lane offset: no address arithmetic on
+  // the VALU, which FP64 MFMA shares
+  const double* V = vals + g.val_off + (long long)((active ? p0 : it.p0) >> 4) * (16 * mp);
+  const unsigned vo = 16 * lk + lrow;
+  const d2* Pp = reinterpret_cast<const d2*>(pg + g.pg_off) + (long long)r0 * nk * 128;
+  d4 acc[RT][NT];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[rt][t] = d4{0.0, 0.0, 0.0, 0.0};
+  d2 pa[2];
+  auto gload = [&](int kt) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int rt = min(2 * i + (wave >> 1), nrt - 1);
+      pa[i] = (Pp + (rt * nk + kt) * 128)[threadIdx.x & 127u];
+    }
+  };
+  auto lstore = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) sA[b][threadIdx.x + 256 * i] = pa[i];
+  };
+  const int kg = NT == 4 ? r0 + nrt : 0;  // slabs with gradient products
+  double bx[NT][4], by[NT][4];            // operands of this slab and the next
+  auto bload = [&](int kt, double (&b)[NT][4]) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) b[0][q] = (V + 256 * kt + 64 * q)[vo];
+    if (kt < kg) {
+#pragma unroll
+      for (int t = 1; t < NT; ++t)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) b[t][q] = (V + t * plane + 256 * kt + 64 * q)[vo];
+    }
+  };
+  auto slab = [&](int kt, const double (&b)[NT][4], double (&bn)[NT][4]) {
+    const int nx = min(kt + 1, nk - 1);
+    gload(nx);
+    if (active) {
+      bload(nx, bn);
+      const int buf = kt & 1, d = kt - r0;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        d2 a[RT];
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) a[rt] = sA[buf][rt * 128 + h * 64 + lane];
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+          if (rt >= nrt) continue;
+#pragma unroll
+          for (int q = 0; q < 2; ++q) Mma<double>::op(a[rt][q], b[0][2 * h + q], acc[rt][0]);
+          if (NT == 4 && d <= rt) {
+            const double w = d == rt ? 0.5 : 1.0;
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+              const double aw = w * a[rt][q];
+#pragma unroll
+              for (int t = 1; t < NT; ++t) Mma<double>::op(aw, b[t][2 * h + q], acc[rt][t]);
+            }
+          }
+        }
+      }
+    }
+    lstore((kt + 1) & 1);
+    __syncthreads();
+  };
+  if (active) bload(0, bx);
+  gload(0);
+  lstore(0);
+  __syncthreads();
+  for (int kt = 0; kt < nk; kt += 2) {
+    slab(kt, bx, by);
+    if (kt + 1 < nk) slab(kt + 1, by, bx);
+  }
+  if (!active) return;
+  double s[NS], h[6];
+#pragma unroll
+  for (int k = 0; k < NS; ++k) s[k] = 0.0;
+#pragma unroll
+  for (int k = 0; k < 6; ++k) h[k] = 0.0;
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    if (rt >= nrt) continue;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      // item i is function lk + 4 i of the row tile
+      const double* vj = V + 16 * (it.c0 + 16 * rt + 4 * i);
+      double v[NS];
+#pragma unroll
+      for (int q = 0; q < NS; ++q) v[q] = (vj + q * plane)[vo];
+      const double y0 = acc[rt][0][i];
+#pragma unroll
+      for (int q = 0; q < NS; ++q) s[q] += v[q] * y0;
+      if constexpr (NT == 4) {
+        const double ux = acc[rt][1][i], uy = acc[rt][2][i], uz = acc[rt][3][i];
+        h[0] += v[1] * ux;
+        h[1] += v[2] * uy;
+        h[2] += v[3] * uz;
+        h[3] += v[1] * uy + v[2] * ux;
+        h[4] += v[1] * uz + v[3] * ux;
+        h[5] += v[2] * uz + v[3] * uy;
+      }
+    }
+  }
+  if constexpr (NT == 4) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      s[4 + k] += 2.0 * h[k];
+      s[7 + k] += h[3 + k];
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < NS; ++k) {  // the 4 lane groups holding the same point
+    s[k] += __shfl_xor(s[k], 16);
+    s[k] += __shfl_xor(s[k], 32);
+  }
+  if (lk == 0) {
+    double* my = cpart + (long long)(it.pbase + it.c0 / kFnChunk) * NS * kDensPts + 16 * wave + lrow;
+#pragma unroll
+    for (int k = 0; k < NS; ++k) my[k * kDensPts] = s[k];
+  }
+}
+
 // Density + functional on split-BF16 MFMA, row-split form for groups of
 // more than 64 functions: a block owns 16 points and its four waves split the
 // function row tiles (wave w takes tiles w, w + 4, ..., RTW of them a pass).
@@ -2438,7 +2669,7 @@ __device__ inline void force_rows(const double (&w)[12], int lrow, double (*slot
   }
 }
 
-// FP64 / FP32 values (planes [value][function][point]).
+// FP64 / FP32 values (tiled planes; P_g as k_gather_density leaves it).
 template <class T>
 __global__ __launch_bounds__(256, 2) void k_force(const DensityItem* __restrict__ items,
                                                   const DevGroup* __restrict__ groups,
@@ -2465,13 +2696,20 @@ __global__ __launch_bounds__(256, 2) void k_force(const DensityItem* __restrict_
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt) acc[rt] = typename Mma<T>::acc{0, 0, 0, 0};
     if (active) {
-      const T* Bk = V + (long long)lk * np + p0 + lrow;   // phi[k][p]
-      const T* Ak = Pm + (long long)lk * mp + c0 + lrow;  // P[k][j] = P[j][k]
+      const T* Bk = V + fm_row(mp, p0 + lrow) + 16 * lk;  // phi[k][p]
       for (int k0 = 0; k0 < mp; k0 += 4) {
-        const T b = Bk[(long long)k0 * np];
+        const T b = Bk[16 * k0];
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt)
-          if (rt < nrt) Mma<T>::op(Ak[(long long)k0 * mp + 16 * rt], b, acc[rt]);
+        for (int rt = 0; rt < 4; ++rt) {
+          if (rt >= nrt) continue;
+          T a;  // P[j][k], symmetric
+          if constexpr (sizeof(T) == 8)
+            a = Pm[((long long)(c0 / 16 + rt) * (mp >> 3) + (k0 >> 3)) * 128 + 2 * lane +
+                   ((k0 >> 2) & 1)];
+          else
+            a = Pm[(long long)(k0 + lk) * mp + c0 + lrow + 16 * rt];
+          Mma<T>::op(a, b, acc[rt]);
+        }
       }
     }
 #pragma unroll
@@ -2481,7 +2719,7 @@ __global__ __launch_bounds__(256, 2) void k_force(const DensityItem* __restrict_
         const int jj = 16 * rt + Mma<T>::row(lk, i);
         double c[3] = {0.0, 0.0, 0.0};
         if (active && rt < nrt) {
-          const T* vj = V + (long long)(c0 + jj) * np + p0 + lrow;
+          const T* vj = V + fm_row(mp, p0 + lrow) + 16 * (c0 + jj);
           const double y = f * (double)acc[rt][i];
 #pragma unroll
           for (int a = 0; a < 3; ++a) c[a] = y * (double)vj[(a + 1) * plane];
@@ -4166,6 +4404,7 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
   // 11: 10 with phi's four pieces split once per grid
   dg->chunked = prec == Precision::BF16X6 && tuning_.density_variant >= 10;
   dg->presplit = prec == Precision::BF16X6 && tuning_.density_variant == 11;
+  const bool chunks = dg->chunked || prec == Precision::FP64;
   // in-kernel evaluation keeps no value planes (phi alone, function-major,
   // for the Fock kernel); variant 8 one more plane (phi's remainder)
   dg->nval = dg->inkernel ? 0 : (dg->gga && !dg->radial) ? 10 : 4;
@@ -4372,8 +4611,10 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
   // kernel on 16-point blocks (listed first), the rest 64-point blocks
   const bool rowsplit = bf && (tuning_.density_variant == 3 || tuning_.density_variant == 4);
   std::vector<DensityItem> ditems, dsmall, citems;
-  // the function-major evaluation runs unless the point-major one does
-  const bool fm_eval = !bf || dg->inkernel, pm_eval = bf && !dg->inkernel;
+  // the function-major evaluation (phi alone) runs for the in-kernel variants,
+  // the tile evaluations (64 points x pm_fns functions) otherwise
+  const bool fm_eval = dg->inkernel, pm_eval = !dg->inkernel;
+  const int pm_fns = bf ? kPmFns : kFmFns;
   {  // the lists' lengths first: millions of items for large molecules
     size_t ne = 0, ng = 0, npm = 0, nt = 0;
     for (int g = 0; g < G; ++g) {
@@ -4383,7 +4624,7 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
       if (fm_eval) ne += (size_t)d.m_pad * ((d.npts_pad + kEvalSpan - 1) / kEvalSpan);
       ng += ((size_t)d.m_pad * d.m_pad + 255) / 256;
       if (pm_eval)
-        npm += (size_t)((d.npts_pad + kPmPts - 1) / kPmPts) * ((d.m_pad + kPmFns - 1) / kPmFns);
+        npm += (size_t)((d.npts_pad + kPmPts - 1) / kPmPts) * ((d.m_pad + pm_fns - 1) / pm_fns);
     }
     citems.reserve(nt);
     dsmall.reserve(nt);
@@ -4405,7 +4646,7 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
     for (int e0 = 0; e0 < d.m_pad * d.m_pad; e0 += 256) gitems.push_back(GatherItem{g, e0});
     if (pm_eval)
       for (int p0 = 0; p0 < d.npts_pad; p0 += kPmPts)
-        for (int k0 = 0; k0 < d.m_pad; k0 += kPmFns, ++pm_next)
+        for (int k0 = 0; k0 < d.m_pad; k0 += pm_fns, ++pm_next)
           pmitems[kXcds * (pm_next % pm_len) + pm_next / pm_len] = EvalItem{g, k0, p0, 0};
     if (dg->radial)
       for (int e0 = 0; e0 < d.nsh_pad * d.npts_pad; e0 += kEvalSpan)
@@ -4426,7 +4667,7 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
       if (groups[ditems[i].group].mol == k) eidx.push_back(i);
     hmol[k].ee = (int)eidx.size();
   }
-  // variants 10, 11: every point tile's row chunks.  Block b runs on XCD
+  // FP64 and variants 10, 11: every point tile's row chunks.  Block b runs on XCD
   // b % kXcds, so the list is the XCDs' lists interleaved: each tile (heavy
   // groups first) goes whole to the XCD with the least work so far, its
   // chunks consecutive there, and the short lists are padded with empty
@@ -4435,7 +4676,7 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
   // slower.
   std::vector<ChunkItem> chitems, finitems;
   long long npart = 0;
-  if (dg->chunked) {
+  if (chunks) {
     std::vector<std::vector<ChunkItem>> lane(kXcds);
     std::vector<long long> load(kXcds, 0);
     for (int i = 0; i < (int)ditems.size(); ++i) {
@@ -4776,21 +5017,13 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
   if (dg->neval > 0 || dg->npm > 0) {
     const dim3 grid(dg->neval), block(kEvalPts);
     if (prec == Precision::FP64) {
-      double* v = static_cast<double*>(dg->vals);
-      if (dg->gga)
-        hipLaunchKernelGGL((k_eval_basis<10, double>), grid, block, 0, s, dg->eitems, dg->groups,
-                           dg->fnl, dg->bas, dg->px, dg->py, dg->pz, v, 0);
-      else
-        hipLaunchKernelGGL((k_eval_basis<4, double>), grid, block, 0, s, dg->eitems, dg->groups,
-                           dg->fnl, dg->bas, dg->px, dg->py, dg->pz, v, 0);
+      hipLaunchKernelGGL((dg->gga ? k_eval_fm<10, double> : k_eval_fm<4, double>), dim3(dg->npm),
+                         dim3(256), 0, s, dg->pmitems, dg->groups, dg->fnl, dg->bas, dg->px, dg->py,
+                         dg->pz, static_cast<double*>(dg->vals));
     } else if (prec == Precision::FP32) {
-      float* v = static_cast<float*>(dg->vals);
-      if (dg->gga)
-        hipLaunchKernelGGL((k_eval_basis<10, float>), grid, block, 0, s, dg->eitems, dg->groups,
-                           dg->fnl, dg->bas, dg->px, dg->py, dg->pz, v, 0);
-      else
-        hipLaunchKernelGGL((k_eval_basis<4, float>), grid, block, 0, s, dg->eitems, dg->groups,
-                           dg->fnl, dg->bas, dg->px, dg->py, dg->pz, v, 0);
+      hipLaunchKernelGGL((dg->gga ? k_eval_fm<10, float> : k_eval_fm<4, float>), dim3(dg->npm),
+                         dim3(256), 0, s, dg->pmitems, dg->groups, dg->fnl, dg->bas, dg->px, dg->py,
+                         dg->pz, static_cast<float*>(dg->vals));
     } else if (dg->inkernel) {  // phi alone, function-major, for the Fock kernel
       hipLaunchKernelGGL((k_eval_basis<1, float>), grid, block, 0, s, dg->eitems, dg->groups,
                          dg->fnl, dg->bas, dg->px, dg->py, dg->pz, dg->phiT, 1);
@@ -5388,26 +5621,40 @@ static void mark(hipEvent_t* ev, int k, hipStream_t s) {
 // Gather and density + functional launches of one spin.  spin 0 closed
 // shell, 1 the alpha pass (P_g from the first packed block into pg), 2 the
 // beta pass (the second block into pg2).
-template <class T>
-static void launch_density(DeviceGrid& g, hipStream_t s, const double* d_rho, int spin,
-                           hipEvent_t* ev) {
-  T* pg = static_cast<T*>(spin == 2 ? g.pg2 : g.pg);
+static void launch_density_finish(DeviceGrid& g, hipStream_t s, int spin) {
+  if (g.nfin <= 0) return;
+  hipLaunchKernelGGL(g.gga ? k_density_cs_finish<4> : k_density_cs_finish<1>,
+                     dim3((g.nfin + 3) / 4), dim3(256), 0, s, g.finitems, g.nfin, g.groups, g.pw,
+                     g.factor, g.epart, g.iexch, spin, g.factor_b, g.sums, g.npts_pad, g.cpart);
+}
+
+static void launch_density_fp64(DeviceGrid& g, hipStream_t s, const double* d_rho, int spin,
+                                hipEvent_t* ev) {
+  double* pg = static_cast<double*>(spin == 2 ? g.pg2 : g.pg);
   const double* rho = spin == 2 ? d_rho + g.packed : d_rho;
-  const T* vals = static_cast<const T*>(g.vals);
   if (g.ngather > 0)
-    hipLaunchKernelGGL(k_gather_density<T>, dim3(g.ngather), dim3(256), 0, s, g.gitems, g.groups,
-                       g.mols, g.fnl, rho, pg);
+    hipLaunchKernelGGL(k_gather_density<double>, dim3(g.ngather), dim3(256), 0, s, g.gitems,
+                       g.groups, g.mols, g.fnl, rho, pg);
   if (spin < 2) mark(ev, 1, s);
-  if (g.ndensity > 0) {
-    if (g.gga)
-      hipLaunchKernelGGL((k_density<4, T>), dim3(g.ndensity), dim3(256), 0, s, g.ditems, g.groups,
-                         pg, vals, g.pw, g.factor, g.epart, g.iexch, spin, g.factor_b, g.sums,
-                         g.npts_pad);
-    else
-      hipLaunchKernelGGL((k_density<1, T>), dim3(g.ndensity), dim3(256), 0, s, g.ditems, g.groups,
-                         pg, vals, g.pw, g.factor, g.epart, g.iexch, spin, g.factor_b, g.sums,
-                         g.npts_pad);
-  }
+  if (g.nchunk > 0)
+    hipLaunchKernelGGL(g.gga ? k_density_dc<4> : k_density_dc<1>, dim3(g.nchunk), dim3(256), 0, s,
+                       g.chitems, g.groups, pg, static_cast<const double*>(g.vals), g.cpart);
+  launch_density_finish(g, s, spin);
+  XCQ_HIP(hipGetLastError());
+}
+
+static void launch_density_fp32(DeviceGrid& g, hipStream_t s, const double* d_rho, int spin,
+                                hipEvent_t* ev) {
+  float* pg = static_cast<float*>(spin == 2 ? g.pg2 : g.pg);
+  const double* rho = spin == 2 ? d_rho + g.packed : d_rho;
+  if (g.ngather > 0)
+    hipLaunchKernelGGL(k_gather_density<float>, dim3(g.ngather), dim3(256), 0, s, g.gitems,
+                       g.groups, g.mols, g.fnl, rho, pg);
+  if (spin < 2) mark(ev, 1, s);
+  if (g.ndensity > 0)
+    hipLaunchKernelGGL((g.gga ? k_density<4, float> : k_density<1, float>), dim3(g.ndensity),
+                       dim3(256), 0, s, g.ditems, g.groups, pg, static_cast<const float*>(g.vals),
+                       g.pw, g.factor, g.epart, g.iexch, spin, g.factor_b, g.sums, g.npts_pad);
   XCQ_HIP(hipGetLastError());
 }
 
@@ -5457,30 +5704,11 @@ static void launch_density_bf(DeviceGrid& g, hipStream_t s, const double* d_rho,
     float* y = yb ? yb + (spin == 2 ? g.phi_elems : 0) : nullptr;
 
     if (g.chunked && g.nchunk > 0) {
-      const dim3 fgrid((g.nfin + 3) / 4);
-      if (g.gga) {
-        if (g.presplit)
-          hipLaunchKernelGGL((k_density_cs<4, true>), dim3(g.nchunk), dim3(256), 0, s, g.chitems,
-                             g.groups, pg3, vals, y, g.lo16, g.cpart, g.pcs);
-        else
-          hipLaunchKernelGGL((k_density_cs<4, false>), dim3(g.nchunk), dim3(256), 0, s, g.chitems,
-                             g.groups, pg3, vals, y, g.lo16, g.cpart, g.pcs);
-        if (g.nfin > 0)
-          hipLaunchKernelGGL(k_density_cs_finish<4>, fgrid, dim3(256), 0, s, g.finitems, g.nfin,
-                             g.groups, g.pw, g.factor, g.epart, g.iexch, spin, g.factor_b, g.sums,
-                             g.npts_pad, g.cpart);
-      } else {
-        if (g.presplit)
-          hipLaunchKernelGGL((k_density_cs<1, true>), dim3(g.nchunk), dim3(256), 0, s, g.chitems,
-                             g.groups, pg3, vals, y, g.lo16, g.cpart, g.pcs);
-        else
-          hipLaunchKernelGGL((k_density_cs<1, false>), dim3(g.nchunk), dim3(256), 0, s, g.chitems,
-                             g.groups, pg3, vals, y, g.lo16, g.cpart, g.pcs);
-        if (g.nfin > 0)
-          hipLaunchKernelGGL(k_density_cs_finish<1>, fgrid, dim3(256), 0, s, g.finitems, g.nfin,
-                             g.groups, g.pw, g.factor, g.epart, g.iexch, spin, g.factor_b, g.sums,
-                             g.npts_pad, g.cpart);
-      }
+      const auto kernel = g.gga ? (g.presplit ? k_density_cs<4, true> : k_density_cs<4, false>)
+                                : (g.presplit ? k_density_cs<1, true> : k_density_cs<1, false>);
+      hipLaunchKernelGGL(kernel, dim3(g.nchunk), dim3(256), 0, s, g.chitems, g.groups, pg3, vals, y,
+                         g.lo16, g.cpart, g.pcs);
+      launch_density_finish(g, s, spin);
     } else if (g.ndensity > 0) {
 #define XCQ_LO(NT, L)                                                                           \
   hipLaunchKernelGGL((k_density_bf2<NT, 64, false, L>), dim3(g.ndensity), dim3(256), 0, s,        \
@@ -5673,9 +5901,9 @@ static void launch_all(DeviceGrid& g, hipStream_t s, const double* d_rho, double
   for (int sp = 0; sp < nspin; ++sp) {
     const int spin = g.open ? sp + 1 : 0;
     if (g.prec == Precision::FP64)
-      launch_density<double>(g, s, d_rho, spin, ev);
+      launch_density_fp64(g, s, d_rho, spin, ev);
     else if (g.prec == Precision::FP32)
-      launch_density<float>(g, s, d_rho, spin, ev);
+      launch_density_fp32(g, s, d_rho, spin, ev);
     else
       launch_density_bf(g, s, d_rho, spin, ev, ystore ? g.ybuf : nullptr);
   }

@@ -47,3 +47,36 @@ def test_tiled_layout_equals_point_major(name, grid_type):
         assert np.max(np.abs(np.asarray(a) - np.asarray(b))) <= SAME
     for a, b in zip(out[10], out[11]):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("grid_type", [0, 2])
+@pytest.mark.parametrize("name", ["water", (2, 9), (5, 9), (9, 9), (14, 3), (22, 9)])
+def test_fp64_chunks_against_the_oracle(name, grid_type):
+    """FP64 density in (point tile, 64-function chunk) blocks with the
+    gradient forms up to the diagonal, at row counts of one to several chunks
+    (and parts of them).  Oracle and library differ by FP64 round-off of sums
+    of at most 1e5 terms of order one: 1e-10."""
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import os
+    import sys
+    sys.path.insert(0, os.path.join(os.path.dirname(__file__), "..", "oracle"))
+    from pyxc import Oracle
+    from lio_amd import g2g
+    import dataclasses
+    s = dataclasses.replace(_molecule(name), grid_type=grid_type)
+    o = Oracle()
+    o.setup(s)
+    Eo, Fo, _ = o.solve()
+    ctx = g2g.Context(s)
+    ctx.build_grid()
+    F = np.zeros(s.M * (s.M + 1) // 2)
+    E, f, info = ctx.solve_forces(fock=F)
+    fo = o.solve_forces()
+    ctx.close()
+    fo = fo[1] if isinstance(fo, tuple) else fo
+    print("case", name, grid_type, E - Eo, np.max(np.abs(F - Fo)), flush=True)
+    assert abs(E - Eo) <= SAME and abs(info["electrons"] - o.electrons()) <= SAME
+    assert np.max(np.abs(F - Fo)) <= SAME
+    assert np.max(np.abs(f - np.asarray(fo).reshape(f.shape))) <= SAME

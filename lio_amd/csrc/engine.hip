@@ -327,9 +327,9 @@ __device__ inline double density_entry(const DevMol& mol, const double* __restri
   return lo != hi ? 0.5 * v : v;
 }
 
-// FP32: rows.  FP64: operand order, [16-row tile][8 columns][lane][2], lane l
-// holding row l % 16 and columns l / 16 and l / 16 + 4 of the eight: the two A
-// operands of a lane are one 16-byte load and a wave's load one 1 KB run.
+// In operand order, [16-row tile][8 columns][lane][2], lane l holding row
+// l % 16 and columns l / 16 and l / 16 + 4 of the eight: the two A operands of
+// a lane are one load and a wave's load one run (1 KB in FP64).
 template <class T>
 __global__ __launch_bounds__(256) void k_gather_density(const GatherItem* __restrict__ items,
                                                         const DevGroup* __restrict__ groups,
@@ -341,15 +341,8 @@ __global__ __launch_bounds__(256) void k_gather_density(const GatherItem* __rest
   const DevGroup g = groups[it.group];
   const int e = it.start + threadIdx.x;
   if (e >= g.m_pad * g.m_pad) return;
-  int k, j;
-  if constexpr (sizeof(T) == 8) {
-    const int u = e >> 7, nk8 = g.m_pad >> 3, l = (e >> 1) & 63;
-    k = 16 * (u / nk8) + (l & 15);
-    j = 8 * (u % nk8) + 4 * (e & 1) + (l >> 4);
-  } else {
-    k = e / g.m_pad;
-    j = e % g.m_pad;
-  }
+  const int u = e >> 7, nk8 = g.m_pad >> 3, l = (e >> 1) & 63;
+  const int k = 16 * (u / nk8) + (l & 15), j = 8 * (u % nk8) + 4 * (e & 1) + (l >> 4);
   const double v = density_entry(mols[g.mol], rho, fnl[g.fn_off + k], fnl[g.fn_off + j]);
   pg[g.pg_off + e] = (T)v;
 }
@@ -406,128 +399,6 @@ __device__ inline void point_stage(const double* s, int q, int iexch, int spin,
   factor[q] = w * y2a;
   e_w = (dens * w) * (ex + ec);
   n_w = dens * w;
-}
-
-// ---------------------------------------------------------------------------
-// density + functional (FP32 mode): 64 points per block, 16 per wave
-// ---------------------------------------------------------------------------
-// Wave w owns points p0 = 64 b + 16 w (the 16 columns of its MFMA tiles) and
-// walks the functions in chunks of 64 (4 row tiles).  For each row tile rt
-// and derivative t it accumulates (Y_t)^T[j][p] = sum_k P[j][k] Phi_t[k][p];
-// lane l then holds, for point p0 + l%16, the four functions
-// j = 16 rt + l/16 + 4 i (i = item) of all NT derivatives, and contracts them
-// with the values of those functions at that point (10 row-dot partials).
-template <int NT, class T>
-__global__ __launch_bounds__(256, 2) void k_density(const DensityItem* __restrict__ items,
-                                                 const DevGroup* __restrict__ groups,
-                                                 const T* __restrict__ pg,
-                                                 const T* __restrict__ vals,
-                                                 const double* __restrict__ pw,
-                                                 double* __restrict__ factor,
-                                                 double* __restrict__ epart, int iexch,
-                                                 int spin, double* __restrict__ factor_b,
-                                                 double* __restrict__ sums, long long sstride) {
-  __shared__ double sE[4][2];
-  constexpr int NS = (NT == 4) ? 10 : 1;
-  const DensityItem it = items[blockIdx.x];
-  const DevGroup g = groups[it.group];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int lrow = lane & 15, lk = lane >> 4;
-  const int p0 = it.p0 + 16 * wave;
-  double e_w = 0.0, n_w = 0.0;
-  if (p0 < g.npts_pad) {
-    const int np = g.npts_pad, mp = g.m_pad;
-    const long long plane = (long long)mp * np;
-    const T* V = vals + g.val_off;
-    const T* Pm = pg + g.pg_off;
-    double s[NS];
-    for (int k = 0; k < NS; ++k) s[k] = 0.0;
-    for (int c0 = 0; c0 < mp; c0 += kFnChunk) {
-      const int nrt = min(4, (mp - c0) / 16);
-      typename Mma<T>::acc acc[4][NT];
-#pragma unroll
-      for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-        for (int t = 0; t < NT; ++t) acc[rt][t] = typename Mma<T>::acc{0, 0, 0, 0};
-      const T* Bk = V + fm_row(mp, p0 + lrow) + 16 * lk;   // Phi_t[k][p]
-      const T* Ak = Pm + (long long)lk * mp + c0 + lrow;  // P[k][j] = P[j][k]
-      // operands of step k0 in (a, b); the next step's are loaded before the
-      // MFMAs of this one so the loads overlap the matrix pipe
-      T a[4], b[NT];
-#pragma unroll
-      for (int t = 0; t < NT; ++t) b[t] = Bk[t * plane];
-#pragma unroll
-      for (int rt = 0; rt < 4; ++rt) a[rt] = (rt < nrt) ? Ak[16 * rt] : T(0);
-      for (int k0 = 0; k0 < mp; k0 += 4) {
-        T an[4], bn[NT];
-        const bool more = k0 + 4 < mp;
-        const long long kb = (long long)(more ? k0 + 4 : k0);
-#pragma unroll
-        for (int t = 0; t < NT; ++t) bn[t] = Bk[t * plane + kb * 16];
-#pragma unroll
-        for (int rt = 0; rt < 4; ++rt) an[rt] = (rt < nrt) ? Ak[kb * mp + 16 * rt] : T(0);
-#pragma unroll
-        for (int rt = 0; rt < 4; ++rt) {
-          if (rt < nrt) {
-#pragma unroll
-            for (int t = 0; t < NT; ++t) Mma<T>::op(a[rt], b[t], acc[rt][t]);
-          }
-        }
-#pragma unroll
-        for (int t = 0; t < NT; ++t) b[t] = bn[t];
-#pragma unroll
-        for (int rt = 0; rt < 4; ++rt) a[rt] = an[rt];
-      }
-#pragma unroll
-      for (int rt = 0; rt < 4; ++rt) {
-        if (rt >= nrt) continue;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int j = c0 + 16 * rt + Mma<T>::row(lk, i);
-          const T* vj = V + fm_row(mp, p0 + lrow) + 16 * j;
-          if constexpr (NT == 4) {
-            double v[10];
-#pragma unroll
-            for (int q = 0; q < 10; ++q) v[q] = (double)vj[q * plane];
-            const double y0 = acc[rt][0][i], yx = acc[rt][1][i], yy = acc[rt][2][i],
-                         yz = acc[rt][3][i];
-            s[0] += v[0] * y0;
-            s[1] += v[1] * y0;
-            s[2] += v[2] * y0;
-            s[3] += v[3] * y0;
-            s[4] += v[4] * y0 + v[1] * yx;
-            s[5] += v[5] * y0 + v[2] * yy;
-            s[6] += v[6] * y0 + v[3] * yz;
-            s[7] += v[7] * y0 + v[1] * yy;
-            s[8] += v[8] * y0 + v[1] * yz;
-            s[9] += v[9] * y0 + v[2] * yz;
-          } else {
-            s[0] += (double)vj[0] * (double)acc[rt][0][i];
-          }
-        }
-      }
-    }
-    for (int k = 0; k < NS; ++k) {  // the 4 lane groups holding the same point
-      s[k] += __shfl_xor(s[k], 16);
-      s[k] += __shfl_xor(s[k], 32);
-    }
-    if (lk == 0)
-      point_stage<NT>(s, g.pt_off + p0 + lrow, iexch, spin, pw, factor, factor_b, sums, sstride,
-                      e_w, n_w);
-    for (int o = 8; o >= 1; o >>= 1) {
-      e_w += __shfl_xor(e_w, o);
-      n_w += __shfl_xor(n_w, o);
-    }
-  }
-  if (lane == 0) {
-    sE[wave][0] = e_w;
-    sE[wave][1] = n_w;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    epart[2 * blockIdx.x] = ((sE[0][0] + sE[1][0]) + sE[2][0]) + sE[3][0];
-    epart[2 * blockIdx.x + 1] = ((sE[0][1] + sE[1][1]) + sE[2][1]) + sE[3][1];
-  }
 }
 
 // Item i of an accumulator with a runtime index (selects, no scratch).
@@ -1757,7 +1628,8 @@ __global__ __launch_bounds__(256) void k_density_cs_finish(const ChunkItem* __re
 }
 
 // ---------------------------------------------------------------------------
-// FP64 density row-dot sums, one (64-point tile, 64-function chunk) per block
+// FP64 and FP32 density row-dot sums, one (64-point tile, 64-function chunk) per
+// block
 // ---------------------------------------------------------------------------
 // With Y = P phi and the gradients' forms d_a phi^T P d_b phi, P symmetric: let
 // U_a[i] = sum over the 16-row blocks before i's of P d_a phi, plus half the
@@ -1768,7 +1640,8 @@ __global__ __launch_bounds__(256) void k_density_cs_finish(const ChunkItem* __re
 // functions: before the chunk all four products, within it each row tile up
 // to its diagonal block, past it only phi's.  Wave w owns 16 points; the P_g
 // slab (operand order) goes through LDS once per block, the planes' operands
-// come straight into registers one slab ahead.  The ten sums per point go to
+// come straight into registers one slab ahead.  (FP32 keeps the four full
+// products, whose roundings its results are made of.)  The ten sums per point go to
 // cpart and k_density_cs_finish adds the chunks and evaluates the functional.
 //
 // What bounds it: the FP64 unit for large groups (the matrix products keep it
@@ -1781,16 +1654,18 @@ __global__ __launch_bounds__(256) void k_density_cs_finish(const ChunkItem* __re
 // instead but needs the sums beside 128 accumulator and 64 operand registers:
 // 1.80 and 5.7 ms with them in LDS, 2.4 ms spilled; single-buffered operands
 // 1.94 ms, two waves per 16 points and four waves a SIMD 2.16 ms.
-template <int NT>
+template <int NT, class T>
 __global__ __launch_bounds__(256, 2) void k_density_dc(const ChunkItem* __restrict__ items,
                                                        const DevGroup* __restrict__ groups,
-                                                       const double* __restrict__ pg,
-                                                       const double* __restrict__ vals,
+                                                       const T* __restrict__ pg,
+                                                       const T* __restrict__ vals,
                                                        double* __restrict__ cpart) {
   constexpr int NS = (NT == 4) ? 10 : 1;
   constexpr int RT = 4;
-  typedef double d2 __attribute__((ext_vector_type(2)));
-  __shared__ d2 sA[2][RT * 128];  // [buf][16-row tile][8-column half][lane]
+  constexpr bool TRI = sizeof(T) == 8;
+  typedef typename Mma<T>::acc A4;
+  typedef T T2 __attribute__((ext_vector_type(2)));
+  __shared__ T2 sA[2][RT * 128];  // [buf][16-row tile][8-column half][lane]
   const ChunkItem it = items[blockIdx.x];
   if (it.group < 0) return;  // padding of a short XCD list
   const DevGroup g = groups[it.group];
@@ -1804,15 +1679,15 @@ __global__ __launch_bounds__(256, 2) void k_density_dc(const ChunkItem* __restri
   const long long plane = (long long)mp * g.npts_pad;
   // wave-uniform pointers and a 32-bit lane offset: no address arithmetic on
   // the VALU, which FP64 MFMA shares
-  const double* V = vals + g.val_off + (long long)((active ? p0 : it.p0) >> 4) * (16 * mp);
-  const unsigned vo = 16 * lk + lrow;
-  const d2* Pp = reinterpret_cast<const d2*>(pg + g.pg_off) + (long long)r0 * nk * 128;
-  d4 acc[RT][NT];
+  const T* V = vals + g.val_off + (long long)((active ? p0 : it.p0) >> 4) * (16 * mp);
+  const unsigned vo = 16 * lk + lrow, ve = 16 * Mma<T>::row(lk, 0) + lrow;
+  const T2* Pp = reinterpret_cast<const T2*>(pg + g.pg_off) + (long long)r0 * nk * 128;
+  A4 acc[RT][NT];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-    for (int t = 0; t < NT; ++t) acc[rt][t] = d4{0.0, 0.0, 0.0, 0.0};
-  d2 pa[2];
+    for (int t = 0; t < NT; ++t) acc[rt][t] = A4{0, 0, 0, 0};
+  T2 pa[2];
   auto gload = [&](int kt) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -1824,9 +1699,9 @@ __global__ __launch_bounds__(256, 2) void k_density_dc(const ChunkItem* __restri
 #pragma unroll
     for (int i = 0; i < 2; ++i) sA[b][threadIdx.x + 256 * i] = pa[i];
   };
-  const int kg = NT == 4 ? r0 + nrt : 0;  // slabs with gradient products
-  double bx[NT][4], by[NT][4];            // operands of this slab and the next
-  auto bload = [&](int kt, double (&b)[NT][4]) {
+  const int kg = NT == 4 ? (TRI ? r0 + nrt : nk) : 0;  // slabs with gradient products
+  T bx[NT][4], by[NT][4];  // operands of this slab and the next
+  auto bload = [&](int kt, T (&b)[NT][4]) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) b[0][q] = (V + 256 * kt + 64 * q)[vo];
     if (kt < kg) {
@@ -1836,7 +1711,7 @@ __global__ __launch_bounds__(256, 2) void k_density_dc(const ChunkItem* __restri
         for (int q = 0; q < 4; ++q) b[t][q] = (V + t * plane + 256 * kt + 64 * q)[vo];
     }
   };
-  auto slab = [&](int kt, const double (&b)[NT][4], double (&bn)[NT][4]) {
+  auto slab = [&](int kt, const T (&b)[NT][4], T (&bn)[NT][4]) {
     const int nx = min(kt + 1, nk - 1);
     gload(nx);
     if (active) {
@@ -1844,21 +1719,21 @@ __global__ __launch_bounds__(256, 2) void k_density_dc(const ChunkItem* __restri
       const int buf = kt & 1, d = kt - r0;
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        d2 a[RT];
+        T2 a[RT];
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) a[rt] = sA[buf][rt * 128 + h * 64 + lane];
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
           if (rt >= nrt) continue;
 #pragma unroll
-          for (int q = 0; q < 2; ++q) Mma<double>::op(a[rt][q], b[0][2 * h + q], acc[rt][0]);
-          if (NT == 4 && d <= rt) {
-            const double w = d == rt ? 0.5 : 1.0;
+          for (int q = 0; q < 2; ++q) Mma<T>::op(a[rt][q], b[0][2 * h + q], acc[rt][0]);
+          if (NT == 4 && (!TRI || d <= rt)) {
+            const T w = TRI && d == rt ? T(0.5) : T(1);
 #pragma unroll
             for (int q = 0; q < 2; ++q) {
-              const double aw = w * a[rt][q];
+              const T aw = TRI ? w * a[rt][q] : a[rt][q];
 #pragma unroll
-              for (int t = 1; t < NT; ++t) Mma<double>::op(aw, b[t][2 * h + q], acc[rt][t]);
+              for (int t = 1; t < NT; ++t) Mma<T>::op(aw, b[t][2 * h + q], acc[rt][t]);
             }
           }
         }
@@ -1886,11 +1761,11 @@ __global__ __launch_bounds__(256, 2) void k_density_dc(const ChunkItem* __restri
     if (rt >= nrt) continue;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      // item i is function lk + 4 i of the row tile
-      const double* vj = V + 16 * (it.c0 + 16 * rt + 4 * i);
+      // item i is function lk + 4 i of the row tile in FP64, 4 lk + i in FP32
+      const T* vj = V + 16 * (it.c0 + 16 * rt + Mma<T>::row(0, i));
       double v[NS];
 #pragma unroll
-      for (int q = 0; q < NS; ++q) v[q] = (vj + q * plane)[vo];
+      for (int q = 0; q < NS; ++q) v[q] = (double)(vj + q * plane)[ve];
       const double y0 = acc[rt][0][i];
 #pragma unroll
       for (int q = 0; q < NS; ++q) s[q] += v[q] * y0;
@@ -1899,16 +1774,21 @@ __global__ __launch_bounds__(256, 2) void k_density_dc(const ChunkItem* __restri
         h[0] += v[1] * ux;
         h[1] += v[2] * uy;
         h[2] += v[3] * uz;
-        h[3] += v[1] * uy + v[2] * ux;
-        h[4] += v[1] * uz + v[3] * ux;
-        h[5] += v[2] * uz + v[3] * uy;
+        h[3] += v[1] * uy;
+        h[4] += v[1] * uz;
+        h[5] += v[2] * uz;
+        if constexpr (TRI) {
+          h[3] += v[2] * ux;
+          h[4] += v[3] * ux;
+          h[5] += v[3] * uy;
+        }
       }
     }
   }
   if constexpr (NT == 4) {
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-      s[4 + k] += 2.0 * h[k];
+      s[4 + k] += (TRI ? 2.0 : 1.0) * h[k];
       s[7 + k] += h[3 + k];
     }
   }
@@ -2702,12 +2582,8 @@ __global__ __launch_bounds__(256, 2) void k_force(const DensityItem* __restrict_
 #pragma unroll
         for (int rt = 0; rt < 4; ++rt) {
           if (rt >= nrt) continue;
-          T a;  // P[j][k], symmetric
-          if constexpr (sizeof(T) == 8)
-            a = Pm[((long long)(c0 / 16 + rt) * (mp >> 3) + (k0 >> 3)) * 128 + 2 * lane +
-                   ((k0 >> 2) & 1)];
-          else
-            a = Pm[(long long)(k0 + lk) * mp + c0 + lrow + 16 * rt];
+          const T a = Pm[((long long)(c0 / 16 + rt) * (mp >> 3) + (k0 >> 3)) * 128 + 2 * lane +
+                         ((k0 >> 2) & 1)];
           Mma<T>::op(a, b, acc[rt]);
         }
       }
@@ -4404,7 +4280,7 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
   // 11: 10 with phi's four pieces split once per grid
   dg->chunked = prec == Precision::BF16X6 && tuning_.density_variant >= 10;
   dg->presplit = prec == Precision::BF16X6 && tuning_.density_variant == 11;
-  const bool chunks = dg->chunked || prec == Precision::FP64;
+  const bool chunks = dg->chunked || !(prec == Precision::BF16X6);
   // in-kernel evaluation keeps no value planes (phi alone, function-major,
   // for the Fock kernel); variant 8 one more plane (phi's remainder)
   dg->nval = dg->inkernel ? 0 : (dg->gga && !dg->radial) ? 10 : 4;
@@ -4667,7 +4543,7 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
       if (groups[ditems[i].group].mol == k) eidx.push_back(i);
     hmol[k].ee = (int)eidx.size();
   }
-  // FP64 and variants 10, 11: every point tile's row chunks.  Block b runs on XCD
+  // FP64, FP32 and variants 10, 11: every point tile's row chunks.  Block b runs on XCD
   // b % kXcds, so the list is the XCDs' lists interleaved: each tile (heavy
   // groups first) goes whole to the XCD with the least work so far, its
   // chunks consecutive there, and the short lists are padded with empty
@@ -5628,33 +5504,20 @@ static void launch_density_finish(DeviceGrid& g, hipStream_t s, int spin) {
                      g.factor, g.epart, g.iexch, spin, g.factor_b, g.sums, g.npts_pad, g.cpart);
 }
 
-static void launch_density_fp64(DeviceGrid& g, hipStream_t s, const double* d_rho, int spin,
-                                hipEvent_t* ev) {
-  double* pg = static_cast<double*>(spin == 2 ? g.pg2 : g.pg);
+template <class T>
+static void launch_density(DeviceGrid& g, hipStream_t s, const double* d_rho, int spin,
+                           hipEvent_t* ev) {
+  T* pg = static_cast<T*>(spin == 2 ? g.pg2 : g.pg);
   const double* rho = spin == 2 ? d_rho + g.packed : d_rho;
   if (g.ngather > 0)
-    hipLaunchKernelGGL(k_gather_density<double>, dim3(g.ngather), dim3(256), 0, s, g.gitems,
-                       g.groups, g.mols, g.fnl, rho, pg);
+    hipLaunchKernelGGL(k_gather_density<T>, dim3(g.ngather), dim3(256), 0, s, g.gitems, g.groups,
+                       g.mols, g.fnl, rho, pg);
   if (spin < 2) mark(ev, 1, s);
   if (g.nchunk > 0)
-    hipLaunchKernelGGL(g.gga ? k_density_dc<4> : k_density_dc<1>, dim3(g.nchunk), dim3(256), 0, s,
-                       g.chitems, g.groups, pg, static_cast<const double*>(g.vals), g.cpart);
+    hipLaunchKernelGGL((g.gga ? k_density_dc<4, T> : k_density_dc<1, T>), dim3(g.nchunk),
+                       dim3(256), 0, s, g.chitems, g.groups, pg, static_cast<const T*>(g.vals),
+                       g.cpart);
   launch_density_finish(g, s, spin);
-  XCQ_HIP(hipGetLastError());
-}
-
-static void launch_density_fp32(DeviceGrid& g, hipStream_t s, const double* d_rho, int spin,
-                                hipEvent_t* ev) {
-  float* pg = static_cast<float*>(spin == 2 ? g.pg2 : g.pg);
-  const double* rho = spin == 2 ? d_rho + g.packed : d_rho;
-  if (g.ngather > 0)
-    hipLaunchKernelGGL(k_gather_density<float>, dim3(g.ngather), dim3(256), 0, s, g.gitems,
-                       g.groups, g.mols, g.fnl, rho, pg);
-  if (spin < 2) mark(ev, 1, s);
-  if (g.ndensity > 0)
-    hipLaunchKernelGGL((g.gga ? k_density<4, float> : k_density<1, float>), dim3(g.ndensity),
-                       dim3(256), 0, s, g.ditems, g.groups, pg, static_cast<const float*>(g.vals),
-                       g.pw, g.factor, g.epart, g.iexch, spin, g.factor_b, g.sums, g.npts_pad);
   XCQ_HIP(hipGetLastError());
 }
 
@@ -5901,9 +5764,9 @@ static void launch_all(DeviceGrid& g, hipStream_t s, const double* d_rho, double
   for (int sp = 0; sp < nspin; ++sp) {
     const int spin = g.open ? sp + 1 : 0;
     if (g.prec == Precision::FP64)
-      launch_density_fp64(g, s, d_rho, spin, ev);
+      launch_density<double>(g, s, d_rho, spin, ev);
     else if (g.prec == Precision::FP32)
-      launch_density_fp32(g, s, d_rho, spin, ev);
+      launch_density<float>(g, s, d_rho, spin, ev);
     else
       launch_density_bf(g, s, d_rho, spin, ev, ystore ? g.ybuf : nullptr);
   }

@@ -1659,6 +1659,7 @@ __global__ __launch_bounds__(256, 2) void k_density_dc(const ChunkItem* __restri
                                                        const DevGroup* __restrict__ groups,
                                                        const T* __restrict__ pg,
                                                        const T* __restrict__ vals,
+                                                       T* __restrict__ ybuf,
                                                        double* __restrict__ cpart) {
   constexpr int NS = (NT == 4) ? 10 : 1;
   constexpr int RT = 4;
@@ -1751,6 +1752,15 @@ __global__ __launch_bounds__(256, 2) void k_density_dc(const ChunkItem* __restri
     if (kt + 1 < nk) slab(kt + 1, by, bx);
   }
   if (!active) return;
+  if (ybuf) {  // Y for the force pass, in the planes' layout (one plane per group)
+    T* Y = ybuf + g.val_off / (NT == 4 ? 10 : 4) + (V - (vals + g.val_off));
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+      if (rt < nrt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          (Y + 16 * (it.c0 + 16 * rt + Mma<T>::row(0, i)))[ve] = acc[rt][0][i];
+  }
   double s[NS], h[6];
 #pragma unroll
   for (int k = 0; k < NS; ++k) s[k] = 0.0;
@@ -2502,21 +2512,6 @@ __global__ __launch_bounds__(256, 2) void k_density_ev(const DensityItem* __rest
 // functions of each nucleus (ascending) over the groups holding them
 // (ascending), so the forces are as reproducible as the energy.
 
-// Adds c over the 16 lanes of a lane group (one function, 16 points) and
-// stores the sum of wave w at sG[w][jj] from the lane group's first lane.
-__device__ inline void force_lanes(double (&c)[3], int lrow, double* slot) {
-#pragma unroll
-  for (int o = 1; o < 16; o <<= 1) {
-#pragma unroll
-    for (int a = 0; a < 3; ++a) c[a] += __shfl_xor(c[a], o);
-  }
-  if (lrow == 0) {
-    slot[0] = c[0];
-    slot[1] = c[1];
-    slot[2] = c[2];
-  }
-}
-
 // Sums w[3 i + a] (four functions i, three components a) over the 16 lanes
 // of a row (the 16 points of a wave's tile) in a fixed order: two halving
 // exchanges (xor 8, then 4) leave each lane three partial sums of one
@@ -2549,25 +2544,33 @@ __device__ inline void force_rows(const double (&w)[12], int lrow, double (*slot
   }
 }
 
-// FP64 / FP32 values (tiled planes; P_g as k_gather_density leaves it).
-template <class T>
+// FP64 / FP32 values (tiled planes).  YS: Y from the density kernel's buffer
+// (8 or 4 bytes per point and function written and read again instead of
+// 2 n m^2 flops: HBM-bound); else recomputed from P_g as k_gather_density
+// leaves it, the same operations in the same order, for callers that allow no
+// allocation (or where none is left).  The sums are the same bit for bit.
+template <class T, bool YS>
 __global__ __launch_bounds__(256, 2) void k_force(const DensityItem* __restrict__ items,
                                                   const DevGroup* __restrict__ groups,
                                                   const T* __restrict__ pg,
-                                                  const T* __restrict__ vals,
+                                                  const T* __restrict__ vals, int nval,
                                                   const double* __restrict__ factor,
                                                   double* __restrict__ gpart) {
   __shared__ double sG[4][kFnChunk][3];
   const DensityItem it = items[blockIdx.x];
   const DevGroup g = groups[it.group];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lrow = lane & 15, lk = lane >> 4;
   const int p0 = it.p0 + 16 * wave;
   const bool active = p0 < g.npts_pad;  // uniform over the wave
-  const int np = g.npts_pad, mp = g.m_pad;
-  const long long plane = (long long)mp * np;
-  const T* V = vals + g.val_off;
+  const int mp = g.m_pad;
+  const long long plane = (long long)mp * g.npts_pad;
+  const long long tile = (long long)((active ? p0 : 0) >> 4) * (16 * mp);
+  const T* V = vals + g.val_off + tile;
+  const T* Yp = YS ? pg + g.val_off / nval + tile : nullptr;
   const T* Pm = pg + g.pg_off;
+  const unsigned ve = 16 * Mma<T>::row(lk, 0) + lrow;
   const double f = active ? factor[g.pt_off + p0 + lrow] : 0.0;
   double* out = gpart + g.force_off + (long long)(it.p0 / kDensPts) * mp * 3;
   for (int c0 = 0; c0 < mp; c0 += kFnChunk) {
@@ -2576,32 +2579,41 @@ __global__ __launch_bounds__(256, 2) void k_force(const DensityItem* __restrict_
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt) acc[rt] = typename Mma<T>::acc{0, 0, 0, 0};
     if (active) {
-      const T* Bk = V + fm_row(mp, p0 + lrow) + 16 * lk;  // phi[k][p]
-      for (int k0 = 0; k0 < mp; k0 += 4) {
-        const T b = Bk[16 * k0];
+      if constexpr (YS) {
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt) {
-          if (rt >= nrt) continue;
-          const T a = Pm[((long long)(c0 / 16 + rt) * (mp >> 3) + (k0 >> 3)) * 128 + 2 * lane +
-                         ((k0 >> 2) & 1)];
-          Mma<T>::op(a, b, acc[rt]);
+        for (int rt = 0; rt < 4; ++rt)
+          if (rt < nrt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              acc[rt][i] = (Yp + 16 * (c0 + 16 * rt + Mma<T>::row(0, i)))[ve];
+      } else {
+        const T* Bk = V + 16 * lk + lrow;  // phi[k][p]
+        for (int k0 = 0; k0 < mp; k0 += 4) {
+          const T b = Bk[16 * k0];
+#pragma unroll
+          for (int rt = 0; rt < 4; ++rt) {
+            if (rt >= nrt) continue;
+            const T a = Pm[((long long)(c0 / 16 + rt) * (mp >> 3) + (k0 >> 3)) * 128 + 2 * lane +
+                           ((k0 >> 2) & 1)];
+            Mma<T>::op(a, b, acc[rt]);
+          }
         }
       }
     }
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt) {
+      double w[12];
+      int jj[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int jj = 16 * rt + Mma<T>::row(lk, i);
-        double c[3] = {0.0, 0.0, 0.0};
-        if (active && rt < nrt) {
-          const T* vj = V + fm_row(mp, p0 + lrow) + 16 * (c0 + jj);
-          const double y = f * (double)acc[rt][i];
+        jj[i] = 16 * rt + Mma<T>::row(lk, i);
+        const T* vj = V + 16 * (c0 + 16 * rt + Mma<T>::row(0, i));
+        const double y = f * (double)acc[rt][i];
 #pragma unroll
-          for (int a = 0; a < 3; ++a) c[a] = y * (double)vj[(a + 1) * plane];
-        }
-        force_lanes(c, lrow, sG[wave][jj]);
+        for (int a = 0; a < 3; ++a)
+          w[3 * i + a] = active && rt < nrt ? y * (double)(vj + (a + 1) * plane)[ve] : 0.0;
       }
+      force_rows(w, lrow, sG[wave], jj);
     }
     __syncthreads();
     if (threadIdx.x < 3 * kFnChunk) {
@@ -3971,9 +3983,19 @@ struct DeviceGrid {
   EvalItem* pmitems = nullptr;  // point-major evaluation blocks (split-BF16)
   int npm = 0;
   float* phiT = nullptr;          // function-major phi (split-BF16 Fock operand)
-  float* ybuf = nullptr;          // Y = P_g phi per point (split-BF16 forces), point-major;
-                                  // allocated at the first forces build (not in the arena)
+  void* ybuf = nullptr;           // Y = P_g phi per point and function (force pass), in the
+                                  // planes' layout and type; allocated at the first forces
+                                  // build (not in the arena)
   size_t ybuf_cap = 0;            // its bytes
+  bool y_denied = false;          // no memory for it: FP64 and FP32 forces recompute Y
+  // values of Y per spin
+  long long yelems() const {
+    return prec == Precision::BF16X6 ? phi_elems : val_elems / nval;
+  }
+  size_t ybytes() const {
+    return (size_t)(open ? 2 : 1) * (size_t)yelems() *
+           (prec == Precision::FP64 ? sizeof(double) : sizeof(float));
+  }
   DensityItem* ditems = nullptr;
   FockItem* fitems = nullptr;
   int2* gtiles = nullptr;
@@ -4146,6 +4168,19 @@ static size_t pool_alloc(void** p, size_t want, size_t need, hipStream_t s, int 
   (void)hipGetLastError();
   XCQ_HIP(hipMallocAsync(p, need, s));
   return need;
+}
+
+// Device memory a new allocation could have: free, or cached unused in the
+// stream-ordered pool.
+static size_t obtainable_bytes(int device) {
+  size_t free_b = 0, total_b = 0;
+  XCQ_HIP(hipMemGetInfo(&free_b, &total_b));
+  hipMemPool_t pool;
+  uint64_t reserved = 0, used = 0;
+  XCQ_HIP(hipDeviceGetDefaultMemPool(&pool, device));
+  XCQ_HIP(hipMemPoolGetAttribute(pool, hipMemPoolAttrReservedMemCurrent, &reserved));
+  XCQ_HIP(hipMemPoolGetAttribute(pool, hipMemPoolAttrUsedMemCurrent, &used));
+  return free_b + (reserved > used ? reserved - used : 0);
 }
 
 // Returns an arena to the slab it came from (after the stream's work on it
@@ -4729,17 +4764,8 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
     // headroom (12.5 %, 25 % for a grid that outgrew its arena) so that the
     // grids of the next steps of a moving molecule fit the same arena
     const size_t want = dg->arena_bytes + (reclaim ? dg->arena_bytes / 4 : dg->arena_bytes / 8);
-    size_t free_b = 0, total_b = 0;
+    const size_t free_b = obtainable_bytes(device_);
     const bool slab = g_slab[device_].active();
-    XCQ_HIP(hipMemGetInfo(&free_b, &total_b));
-    {  // memory freed into the pool is available again
-      hipMemPool_t pool;
-      uint64_t reserved = 0, used = 0;
-      XCQ_HIP(hipDeviceGetDefaultMemPool(&pool, device_));
-      XCQ_HIP(hipMemPoolGetAttribute(pool, hipMemPoolAttrReservedMemCurrent, &reserved));
-      XCQ_HIP(hipMemPoolGetAttribute(pool, hipMemPoolAttrUsedMemCurrent, &used));
-      if (reserved > used) free_b += reserved - used;
-    }
     if (!slab && dg->arena_bytes > free_b + reclaim) {
       const size_t need = dg->arena_bytes;
       throw std::runtime_error("g2g: grid needs " + std::to_string(need >> 20) +
@@ -4769,7 +4795,7 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
   Carver carve{dg->arena};
   plan(carve);
   // the previous grid's Y buffer serves this one when large enough
-  if (old.g && old.g->ybuf && old.g->ybuf_cap >= (size_t)(dg->open ? 2 : 1) * fo * sizeof(float)) {
+  if (old.g && old.g->ybuf && old.g->ybuf_cap >= dg->ybytes()) {
     dg->ybuf = old.g->ybuf;
     dg->ybuf_cap = old.g->ybuf_cap;
     old.g->ybuf = nullptr;
@@ -5506,7 +5532,7 @@ static void launch_density_finish(DeviceGrid& g, hipStream_t s, int spin) {
 
 template <class T>
 static void launch_density(DeviceGrid& g, hipStream_t s, const double* d_rho, int spin,
-                           hipEvent_t* ev) {
+                           hipEvent_t* ev, void* yb) {
   T* pg = static_cast<T*>(spin == 2 ? g.pg2 : g.pg);
   const double* rho = spin == 2 ? d_rho + g.packed : d_rho;
   if (g.ngather > 0)
@@ -5516,7 +5542,7 @@ static void launch_density(DeviceGrid& g, hipStream_t s, const double* d_rho, in
   if (g.nchunk > 0)
     hipLaunchKernelGGL((g.gga ? k_density_dc<4, T> : k_density_dc<1, T>), dim3(g.nchunk),
                        dim3(256), 0, s, g.chitems, g.groups, pg, static_cast<const T*>(g.vals),
-                       g.cpart);
+                       yb ? static_cast<T*>(yb) + (spin == 2 ? g.yelems() : 0) : nullptr, g.cpart);
   launch_density_finish(g, s, spin);
   XCQ_HIP(hipGetLastError());
 }
@@ -5681,9 +5707,23 @@ static void launch_fock(DeviceGrid& g, hipStream_t s, const double* factor) {
 // Closed-shell split-BF16 builds whose density kernel is k_density_bf2
 // (variants 1, 2, 5) leave Y for the forces in ybuf.
 static bool ystore_forces(const DeviceGrid& g) {
+  if (g.prec != Precision::BF16X6) return g.ybuf != nullptr;  // both spins when open
   if (g.inkernel || g.lo) return g.ybuf != nullptr;  // both spins when open
   return g.prec == Precision::BF16X6 && !g.open && g.ybuf &&
          (g.density_variant == 1 || g.density_variant == 2 || g.density_variant == 5);
+}
+
+template <class T>
+static void launch_force_planes(DeviceGrid& g, hipStream_t s, const void* pg, int sp,
+                                const double* factor) {
+  const T* vals = static_cast<const T*>(g.vals);
+  if (ystore_forces(g))
+    hipLaunchKernelGGL((k_force<T, true>), dim3(g.nforce), dim3(256), 0, s, g.citems, g.groups,
+                       static_cast<const T*>(g.ybuf) + (sp == 1 ? g.yelems() : 0), vals, g.nval,
+                       factor, g.gpart);
+  else
+    hipLaunchKernelGGL((k_force<T, false>), dim3(g.nforce), dim3(256), 0, s, g.citems, g.groups,
+                       static_cast<const T*>(pg), vals, g.nval, factor, g.gpart);
 }
 
 static void launch_forces(DeviceGrid& g, hipStream_t s, double* d_forces) {
@@ -5693,21 +5733,17 @@ static void launch_forces(DeviceGrid& g, hipStream_t s, double* d_forces) {
     const double* factor = sp == 1 ? g.factor_b : g.factor;
     if (g.nforce > 0) {
       if (g.prec == Precision::FP64)
-        hipLaunchKernelGGL(k_force<double>, dim3(g.nforce), dim3(256), 0, s, g.citems, g.groups,
-                           static_cast<const double*>(pg), static_cast<const double*>(g.vals),
-                           factor, g.gpart);
+        launch_force_planes<double>(g, s, pg, sp, factor);
       else if (g.prec == Precision::FP32)
-        hipLaunchKernelGGL(k_force<float>, dim3(g.nforce), dim3(256), 0, s, g.citems, g.groups,
-                           static_cast<const float*>(pg), static_cast<const float*>(g.vals),
-                           factor, g.gpart);
+        launch_force_planes<float>(g, s, pg, sp, factor);
       else if (g.inkernel)
         hipLaunchKernelGGL(k_force_ev, dim3(g.nforce), dim3(256), 0, s, g.citems, g.groups,
-                           g.ybuf + (sp == 1 ? g.phi_elems : 0), g.fmeta, g.shells, g.tsh, g.bas,
+                           static_cast<const float*>(g.ybuf) + (sp == 1 ? g.phi_elems : 0), g.fmeta, g.shells, g.tsh, g.bas,
                            g.px, g.py, g.pz, factor, g.gpart);
       else if (ystore_forces(g))
         hipLaunchKernelGGL(g.chunked ? k_force_y<true> : k_force_y<false>, dim3(g.nforce),
                            dim3(256), 0, s, g.citems, g.groups,
-                           g.ybuf + (sp == 1 ? g.phi_elems : 0),
+                           static_cast<const float*>(g.ybuf) + (sp == 1 ? g.phi_elems : 0),
                            static_cast<const float*>(g.vals), factor, g.gpart);
       else
         hipLaunchKernelGGL(k_force_bf, dim3(g.nforce), dim3(256), 0, s, g.citems, g.groups,
@@ -5740,7 +5776,7 @@ static void launch_all(DeviceGrid& g, hipStream_t s, const double* d_rho, double
     // not a memset, so the pair can be captured in a graph); the HIP-event
     // phases then read: expand = clearing, density = the whole build
     const PersistArgs& pa = g.pargs;
-    float* yb = d_forces && ystore_forces(g) ? g.ybuf : nullptr;
+    float* yb = d_forces && ystore_forces(g) ? static_cast<float*>(g.ybuf) : nullptr;
     hipLaunchKernelGGL(k_fill_int, dim3((g.nsync + 255) / 256), dim3(256), 0, s, pa.sync, g.nsync,
                        0);
     mark(ev, 1, s);
@@ -5764,11 +5800,11 @@ static void launch_all(DeviceGrid& g, hipStream_t s, const double* d_rho, double
   for (int sp = 0; sp < nspin; ++sp) {
     const int spin = g.open ? sp + 1 : 0;
     if (g.prec == Precision::FP64)
-      launch_density<double>(g, s, d_rho, spin, ev);
+      launch_density<double>(g, s, d_rho, spin, ev, ystore ? g.ybuf : nullptr);
     else if (g.prec == Precision::FP32)
-      launch_density<float>(g, s, d_rho, spin, ev);
+      launch_density<float>(g, s, d_rho, spin, ev, ystore ? g.ybuf : nullptr);
     else
-      launch_density_bf(g, s, d_rho, spin, ev, ystore ? g.ybuf : nullptr);
+      launch_density_bf(g, s, d_rho, spin, ev, ystore ? static_cast<float*>(g.ybuf) : nullptr);
   }
   mark(ev, 2, s);
   for (int sp = 0; d_fock && sp < nspin; ++sp) {
@@ -5790,15 +5826,24 @@ static void launch_all(DeviceGrid& g, hipStream_t s, const double* d_rho, double
   mark(ev, 4, s);
 }
 
-// The split-BF16 force passes read Y = P_g phi, which the density kernel
-// leaves in a buffer of its own (one FP32 value per padded point and function,
-// per spin): allocated at the first forces build of a grid, from the device
-// slab when one is reserved, else from the stream-ordered pool.
+// The force passes read Y = P_g phi, which the density kernel leaves in a
+// buffer of its own (one value per padded point and function, per spin),
+// allocated at the first forces build of a grid: for split-BF16 from the
+// device slab when one is reserved, else from the stream-ordered pool.  FP64
+// and FP32 can recompute Y (the same bits), so they take the buffer (12.5 %
+// headroom for the grids of the next steps of a moving molecule) only from
+// plenty, at most an eighth of the obtainable memory and never from a slab:
+// no later grid is refused because of it.
 static void ensure_ybuf(DeviceGrid& g, hipStream_t s, int device) {
-  if (g.prec != Precision::BF16X6 || g.ybuf) return;
-  const size_t bytes = (size_t)(g.open ? 2 : 1) * g.phi_elems * sizeof(float) + 256;
+  if (g.ybuf || g.y_denied) return;
+  const bool must = g.prec == Precision::BF16X6;
+  const size_t need = g.ybytes() + 256, bytes = must ? need : need + need / 8;
   Slab& sl = g_slab[device];
   void* p = nullptr;
+  if (!must && (sl.active() || bytes > obtainable_bytes(device) / 8)) {
+    g.y_denied = true;
+    return;
+  }
   if (sl.active()) {
     p = sl.take(bytes);
     if (!p)
@@ -5808,7 +5853,7 @@ static void ensure_ybuf(DeviceGrid& g, hipStream_t s, int device) {
   } else {
     g.ybuf_cap = pool_alloc(&p, bytes, bytes, s, device);
   }
-  g.ybuf = static_cast<float*>(p);
+  g.ybuf = p;
 }
 
 SolveResult Engine::solve_device(const double* d_rho, double* d_fock, bool want_energy,
@@ -5867,7 +5912,7 @@ SolveResult Engine::solve_device_static(const double* d_rho, double* d_fock, dou
                              " MiB (use the allocating entry point)");
   float* y = static_cast<float*>(scratch_address(device_));
   XCQ_HIP(hipSetDevice(device_));
-  float* own = g.ybuf;  // the grid's own buffer (if any) is left untouched
+  void* own = g.ybuf;  // the grid's own buffer (if any) is left untouched
   g.ybuf = y;
   try {
     launch_all(g, (hipStream_t)stream_, d_rho, d_fock, reinterpret_cast<hipEvent_t*>(events_),

@@ -80,3 +80,32 @@ def test_fp64_chunks_against_the_oracle(name, grid_type):
     assert abs(E - Eo) <= SAME and abs(info["electrons"] - o.electrons()) <= SAME
     assert np.max(np.abs(F - Fo)) <= SAME
     assert np.max(np.abs(f - np.asarray(fo).reshape(f.shape))) <= SAME
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("opened", [False, True])
+def test_forces_from_stored_y_equal_recomputed(precision, opened):
+    """FP64 and FP32 forces with Y = P phi left by the density kernel and with
+    Y recomputed (the entry point that allocates nothing, before a Y buffer
+    exists): the same operations, so bitwise the same, at group sizes of one
+    row tile to several chunks."""
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from lio_amd import g2g, systems
+    mols = [_molecule(n) for n in ((2, 9), (5, 9), (22, 9))]
+    if opened:
+        mols = [systems.open_shell(m) for m in mols]
+    b = g2g.Batch(mols, precision=precision)
+    rho = torch.from_numpy(b.packed_density()).cuda()
+    F = torch.zeros_like(rho)
+    f = torch.zeros((2, 3 * int(b.atoms()[-1])), dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    b.solve_forces_static(rho.data_ptr(), F.data_ptr(), f[0].data_ptr())
+    b.energies()
+    b.solve_forces(rho.data_ptr(), F.data_ptr(), f[1].data_ptr())
+    b.energies()
+    torch.cuda.synchronize()
+    b.close()
+    assert float(f[0].abs().max()) > 0.0
+    assert torch.equal(f[0], f[1])

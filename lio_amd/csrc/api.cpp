@@ -543,7 +543,10 @@ int xcq_batch_load_ms(xcq_batch* b, double ms[4]) {
 }
 
 static xcq::Tuning schedule(xcq::Tuning t, int fock_slice, int density_variant) {
-  if (fock_slice > 0) t.fock_slice = fock_slice;
+  if (fock_slice > 0) {
+    t.fock_slice = fock_slice;
+    t.default_slice = false;
+  }
   if (density_variant >= 0) t.density_variant = density_variant;
   return t;
 }
@@ -622,6 +625,7 @@ int xcq_batch_tune(xcq_batch* b, const double* d_rho, double* d_fock, int reps, 
     for (int c = 0; c < ncand; ++c) {
       xcq::Tuning t = b->engine->tuning();
       t.fock_slice = slices[c];
+      t.default_slice = false;
       if (variants) t.density_variant = variants[c];
       b->engine->set_tuning(t);
       load_batch(b);
@@ -640,6 +644,7 @@ int xcq_batch_tune(xcq_batch* b, const double* d_rho, double* d_fock, int reps, 
     }
     xcq::Tuning t = b->engine->tuning();
     t.fock_slice = slices[ibest];
+    t.default_slice = false;
     if (variants) t.density_variant = variants[ibest];
     b->engine->set_tuning(t);
     load_batch(b);

@@ -408,79 +408,123 @@ __device__ inline double pick(const A& v, int i) {
 }
 
 // ---------------------------------------------------------------------------
-// Fock: one block (4 waves) per (group, tile pair, 512-point slice)
+// Fock (FP64, FP32): one block (4 waves) per (group, tile pair, point slice)
 // ---------------------------------------------------------------------------
-// out[i][j] = sum_p phi_i(p) factor_p phi_j(p) for i in tile ti, j in tile tj.
-// Wave w takes the points pb + [128 w, 128 w + 128) of the slice; the four
-// partial tiles are added through LDS in wave order (fixed, reproducible).
-// The K order is permuted so that the four K slots a lane feeds to four
-// consecutive MFMAs are four consecutive points: one 32-byte load per lane
-// and operand row instead of four scattered 8-byte loads.
+// out[i][j] = sum_p phi_i(p) factor_p phi_j(p) for i in tile ti, j in tile tj,
+// p in the slice.  Wave (a, b) owns the 32 x 32 quarter of rows 32 a and
+// columns 32 b (the quarter below the diagonal of a diagonal pair is left
+// zero: nothing reads it).  The rows of 16 points at a time (contiguous in the
+// tiled planes) go through LDS, the columns' already multiplied by the factor,
+// loaded one step ahead; a row's 16-byte units are permuted by its number so
+// that the operand reads, 16 rows of one unit, meet no bank twice.  Lane group
+// l / 16 feeds points 4 (l / 16) + s to MFMA s.  The quarters need 32
+// accumulator registers instead of the 128 of whole tiles split by points, so
+// several blocks share a SIMD and cover each other's loads (the whole-tile
+// form waited for memory 58 % of the time), and no partial tiles are added
+// through LDS: (H2O)32 FP64 0.55 -> 0.39 ms, FP32 0.39 -> 0.28, 60 atoms FP64
+// 1.74 -> 1.29 ms, one water 36 -> 24 us (with the slices of
+// Tuning::slice_for).
+// Block b takes item order[b], as k_fock_bf.
 template <class T>
-__global__ __launch_bounds__(256, 2) void k_fock(const FockItem* __restrict__ items,
+__global__ __launch_bounds__(256, 4) void k_fock(const FockItem* __restrict__ items,
                                                  const DevGroup* __restrict__ groups,
                                                  const T* __restrict__ vals,
                                                  const double* __restrict__ factor,
-                                                 double* __restrict__ fpart) {
+                                                 double* __restrict__ fpart,
+                                                 const int* __restrict__ order) {
   typedef typename Mma<T>::acc A4;
-  typedef T V4 __attribute__((ext_vector_type(4)));
+  constexpr int U = 16 / sizeof(T);          // values per 16-byte unit
+  constexpr int UPR = 16 / U;                // units of a row of 16 points
+  constexpr int NU = kFnChunk * UPR / 256;   // units a thread stages per side
+  typedef T TU __attribute__((ext_vector_type(U)));
   // FP32 products are summed over at most 32 points in the matrix unit and
   // then added into FP64; FP64 accumulates in place.
   constexpr bool kFlush = sizeof(T) == 4;
-  __shared__ double sF[kFnChunk * kFnChunk];
-  const FockItem it = items[blockIdx.x];
+  __shared__ TU sA[2][kFnChunk * UPR], sB[2][kFnChunk * UPR];
+  const int item = order[blockIdx.x];
+  if (item < 0) return;  // padding of a short XCD list
+  const FockItem it = items[item];
   const DevGroup g = groups[it.group];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lrow = lane & 15, lk = lane >> 4;
+  const int lane = threadIdx.x & 63, lrow = lane & 15, lk = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int np = g.npts_pad, mp = g.m_pad;
   const int i0 = kFnChunk * it.ti, j0 = kFnChunk * it.tj;
-  const int nri = min(4, (mp - i0) / 16), nrj = min(4, (mp - j0) / 16);
+  const int wi = 2 * (wave >> 1), wj = 2 * (wave & 1);  // first row and column tile
   const bool diag = it.ti == it.tj;
-  const int slen = g.slen;
-  const int pb = it.slice * slen + wave * (slen / 4);
-  const int pe = min(pb + slen / 4, np);
+  const int nri = diag && wi > wj ? 0 : min(2, (mp - i0) / 16 - wi);
+  const int nrj = min(2, (mp - j0) / 16 - wj);
+  const int pb = it.slice * g.slen, pe = min(pb + g.slen, np);
   const T* V = vals + g.val_off;
   const double* fac = factor + g.pt_off;
-  A4 acc[4][4];
-  d4 dacc[4][4];
+  // this thread's units: row f = t / UPR + 256 / UPR i, unit u = t % UPR
+  const int u = threadIdx.x & (UPR - 1), f0 = threadIdx.x / UPR;
+  TU ra[NU], rb[NU];
+  double rf[U];
+  auto gload = [&](int p) {
+    const T* Vt = V + (long long)(p >> 4) * (16 * mp);
 #pragma unroll
-  for (int a = 0; a < 4; ++a)
+    for (int i = 0; i < NU; ++i) {
+      const int f = f0 + i * (256 / UPR);
+      ra[i] = *reinterpret_cast<const TU*>(Vt + 16 * min(i0 + f, mp - 1) + U * u);
+      if (!diag) rb[i] = *reinterpret_cast<const TU*>(Vt + 16 * min(j0 + f, mp - 1) + U * u);
+    }
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
+    for (int q = 0; q < U; ++q) rf[q] = fac[p + U * u + q];
+  };
+  auto lstore = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < NU; ++i) {
+      const int f = f0 + i * (256 / UPR), x = f * UPR + (u ^ (f & (UPR - 1)));
+      TU y = diag ? ra[i] : rb[i];
+#pragma unroll
+      for (int q = 0; q < U; ++q) y[q] *= (T)rf[q];
+      sA[b][x] = ra[i];
+      sB[b][x] = y;
+    }
+  };
+  // the four points of this lane's group in row f
+  auto row4 = [&](const TU* s, int f, T (&o)[4]) {
+#pragma unroll
+    for (int h = 0; h < 4 / U; ++h) {
+      const TU x = s[f * UPR + ((lk * (4 / U) + h) ^ (f & (UPR - 1)))];
+#pragma unroll
+      for (int q = 0; q < U; ++q) o[U * h + q] = x[q];
+    }
+  };
+  A4 acc[2][2];
+  d4 dacc[2][2];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
       acc[a][b] = A4{0, 0, 0, 0};
       dacc[a][b] = d4{0.0, 0.0, 0.0, 0.0};
     }
-  int step = 0;
-  for (int p = pb + 4 * lk; p < pe; p += 16, ++step) {
-    const d4 fd = *reinterpret_cast<const d4*>(fac + p);
-    const V4 f = V4{(T)fd[0], (T)fd[1], (T)fd[2], (T)fd[3]};
-    V4 A[4], B[4];
+  gload(pb);
+  lstore(0);
+  __syncthreads();
+  for (int p = pb, buf = 0, step = 0; p < pe; p += 16, buf ^= 1, ++step) {
+    const bool more = p + 16 < pe;
+    if (more) gload(p + 16);
+    T A[2][4], B[2][4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      A[r] = (r < nri) ? *reinterpret_cast<const V4*>(V + fm_row(mp, p) + 16 * (i0 + 16 * r + lrow))
-                       : V4{0, 0, 0, 0};
-      if (diag)  // the same function rows on both sides: one load
-        B[r] = A[r] * f;
-      else
-        B[r] = (r < nrj)
-                   ? *reinterpret_cast<const V4*>(V + fm_row(mp, p) + 16 * (j0 + 16 * r + lrow)) * f
-                   : V4{0, 0, 0, 0};
+    for (int r = 0; r < 2; ++r) {
+      if (r < nri) row4(sA[buf], 16 * (wi + r) + lrow, A[r]);
+      if (r < nrj) row4(sB[buf], 16 * (wj + r) + lrow, B[r]);
     }
 #pragma unroll
     for (int s = 0; s < 4; ++s)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        if (r < nri) {
+      for (int r = 0; r < 2; ++r)
 #pragma unroll
-          for (int c = 0; c < 4; ++c)
-            if (c < nrj) Mma<T>::op(A[r][s], B[c][s], acc[r][c]);
-        }
-      }
+        for (int c = 0; c < 2; ++c)
+          if (r < nri && c < nrj) Mma<T>::op(A[r][s], B[c][s], acc[r][c]);
     if constexpr (kFlush) {
-      if ((step & 1) == 1 || p + 16 >= pe) {
+      if ((step & 1) == 1 || !more) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
+        for (int r = 0; r < 2; ++r)
 #pragma unroll
-          for (int c = 0; c < 4; ++c)
+          for (int c = 0; c < 2; ++c)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
               dacc[r][c][i] += (double)acc[r][c][i];
@@ -488,24 +532,19 @@ __global__ __launch_bounds__(256, 2) void k_fock(const FockItem* __restrict__ it
             }
       }
     }
-  }
-  for (int w = 0; w < 4; ++w) {
-    if (wave == w) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int e = (16 * r + Mma<T>::row(lk, i)) * kFnChunk + 16 * c + lrow;
-            const double x = kFlush ? dacc[r][c][i] : (double)acc[r][c][i];
-            sF[e] = (w == 0) ? x : sF[e] + x;
-          }
-    }
+    if (more) lstore(buf ^ 1);
     __syncthreads();
   }
-  double* out = fpart + (long long)blockIdx.x * kFnChunk * kFnChunk;
-  for (int e = threadIdx.x; e < kFnChunk * kFnChunk; e += 256) out[e] = sF[e];
+  double* out = fpart + (long long)item * kFnChunk * kFnChunk;
+#pragma unroll
+  for (int r = 0; r < 2; ++r)
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (i0 + 16 * (wi + r) < mp && c < nrj)  // k_fock_group reads the group's rows only
+          out[(16 * (wi + r) + Mma<T>::row(lk, i)) * kFnChunk + 16 * (wj + c) + lrow] =
+              kFlush ? dacc[r][c][i] : (double)acc[r][c][i];
 }
 
 // ---------------------------------------------------------------------------
@@ -4034,7 +4073,7 @@ struct DeviceGrid {
   int nchunk = 0;
   double* cpart = nullptr;        // per (point tile, chunk): 10 x 64 row-dot sums
   ChunkItem* finitems = nullptr;  // per point tile (k_density_cs_finish)
-  int* forder = nullptr;          // split-BF16 Fock blocks: item per block (XCD-interleaved)
+  int* forder = nullptr;          // Fock blocks: item per block (XCD-interleaved)
   int nfock_order = 0;
   int nfin = 0;
   unsigned short* lo16 = nullptr; // phi's remainder in BF16, point-major (phi_elems)
@@ -4413,11 +4452,11 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
     d.pt_off = (int)pt;
     d.fn_off = (int)fnl.size();
     d.ntile = (d.m_pad + kFnChunk - 1) / kFnChunk;
-    d.nslice = (d.npts_pad + tuning_.slice_for(d.m_pad) - 1) / tuning_.slice_for(d.m_pad);
+    d.slen = tuning_.slice_for(d.m_pad, bf);
+    d.nslice = (d.npts_pad + d.slen - 1) / d.slen;
     d.val_off = vo;
     d.pg_off = po;
     d.fock_base = fock_base;
-    d.slen = tuning_.slice_for(d.m_pad);
     d.phi_off = fo;
     d.force_off = go;
     go += (long long)(d.npts_pad + kDensPts - 1) / kDensPts * d.m_pad * 3;
@@ -4606,10 +4645,10 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
       for (size_t j = 0; j < lane[x].size(); ++j) chitems[j * kXcds + x] = lane[x][j];
   }
   dg->nchunk = (int)chitems.size();
-  // split-BF16 Fock blocks: the tile pairs of each (group, slice), heavy
-  // groups first, go whole to the XCD with the fewest blocks so far
+  // Fock blocks: the tile pairs of each (group, slice), heavy groups first, go
+  // whole to the XCD with the fewest blocks so far
   std::vector<int> forder;
-  if (bf) {
+  {
     std::vector<std::vector<int>> lane(kXcds);
     for (int g : order) {
       const DevGroup& d = groups[g];
@@ -5688,11 +5727,11 @@ static void launch_density_bf(DeviceGrid& g, hipStream_t s, const double* d_rho,
 static void launch_fock(DeviceGrid& g, hipStream_t s, const double* factor) {
   if (g.nfock <= 0) return;
   if (g.prec == Precision::FP64)
-    hipLaunchKernelGGL(k_fock<double>, dim3(g.nfock), dim3(256), 0, s, g.fitems, g.groups,
-                       static_cast<const double*>(g.vals), factor, g.fpart);
+    hipLaunchKernelGGL(k_fock<double>, dim3(g.nfock_order), dim3(256), 0, s, g.fitems, g.groups,
+                       static_cast<const double*>(g.vals), factor, g.fpart, g.forder);
   else if (g.prec == Precision::FP32)
-    hipLaunchKernelGGL(k_fock<float>, dim3(g.nfock), dim3(256), 0, s, g.fitems, g.groups,
-                       static_cast<const float*>(g.vals), factor, g.fpart);
+    hipLaunchKernelGGL(k_fock<float>, dim3(g.nfock_order), dim3(256), 0, s, g.fitems, g.groups,
+                       static_cast<const float*>(g.vals), factor, g.fpart, g.forder);
   else
     hipLaunchKernelGGL(k_fock_bf, dim3(g.nfock_order), dim3(256), 0, s, g.fitems, g.groups,
                        g.phiT, factor, g.fpart, g.forder);

@@ -219,10 +219,18 @@ struct Tuning {
   int density_variant = 10;
   int persistent = 0;
   std::vector<int> bucket_mhi, bucket_slice;
-  int slice_for(int m_pad) const {
+  // No slice was asked for: FP64 and FP32 groups take 256 points up to 128
+  // functions (one to three blocks a slice, whose 64 steps of a 1024-point
+  // slice would run alone: one water 24 us against 61, 25 atoms 215 against
+  // 251), 512 up to 384 ((H2O)32 389 us against 418 with 256 and 406 with 1024
+  // throughout) and fock_slice above (100 atoms 2.71 ms against 2.80 with 512).
+  // Split-BF16's slices also decide where its FP32 sums end: always fock_slice.
+  bool default_slice = true;
+  int slice_for(int m_pad, bool split_bf16) const {
     for (size_t i = 0; i < bucket_mhi.size(); ++i)
       if (m_pad <= bucket_mhi[i]) return bucket_slice[i];
-    return fock_slice;
+    if (!default_slice || split_bf16) return fock_slice;
+    return m_pad <= 128 ? 256 : m_pad <= 384 ? 512 : fock_slice;
   }
 };
 

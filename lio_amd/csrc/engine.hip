@@ -63,7 +63,7 @@ constexpr int kRowSplitMin = 64; // split-BF16 row-split density above this m_pa
 constexpr int kFnChunk = 64;     // functions per density pass / Fock tile side
 constexpr int kXcds = 8;         // MI355X: XCDs, each with its own L2 (block b runs on b % 8)
 constexpr int kSliceDefault = 1024;  // points per Fock slice (split-K over blocks)
-constexpr int kPackMapMax = 16384;  // groups per molecule the packing kernel maps in LDS
+constexpr int kPackMapMax = 8192;  // groups per molecule the packing kernel maps in LDS (64 KB)
 constexpr int kEvalPts = 256;    // threads per evaluation block
 constexpr int kEvalSpan = 4096;  // points (or elements) one evaluation block covers
 
@@ -2908,62 +2908,67 @@ __global__ __launch_bounds__(256) void k_force_ev(const DensityItem* __restrict_
 // accumulate: add onto gsum (the second spin of an open shell).
 // One thread per (group, element), blockIdx.x the group; the loads of
 // several blocks are in flight together, the sum stays in block order.
+// (Four threads per element, each a quarter of the blocks by turns, added in
+// thread order: a sphere's 73 blocks are 19 loads in a row, not 73.)
 __global__ __launch_bounds__(256) void k_force_group(const DevGroup* __restrict__ groups,
                                                      const double* __restrict__ gpart,
                                                      double* __restrict__ gsum, int accumulate) {
+  __shared__ double sq[4][64];
   const DevGroup g = groups[blockIdx.x];
-  const int e = blockIdx.y * 256 + threadIdx.x;
-  if (e >= 3 * g.m_pad) return;
+  const int q = threadIdx.x >> 6, l = threadIdx.x & 63;
+  const int e = blockIdx.y * 64 + l;
+  if ((int)blockIdx.y * 64 >= 3 * g.m_pad) return;  // whole blocks
   const int nblk = (g.npts_pad + kDensPts - 1) / kDensPts;
   const long long stride = 3LL * g.m_pad;
-  const double* src = gpart + g.force_off + e;
   double s = 0.0;
+  if (e < 3 * g.m_pad) {
+    const double* src = gpart + g.force_off + e;
 #pragma unroll 8
-  for (int b = 0; b < nblk; ++b) s += src[b * stride];
+    for (int b = q; b < nblk; b += 4) s += src[b * stride];
+  }
+  sq[q][l] = s;
+  __syncthreads();
+  if (q != 0 || e >= 3 * g.m_pad) return;
+  s = ((sq[0][l] + sq[1][l]) + sq[2][l]) + sq[3][l];
   double* dst = gsum + 3LL * g.fn_off + e;
   *dst = accumulate ? *dst + s : s;
 }
 
-// Per batch function I, the sum of its group sums over the groups holding it
-// (ascending group order); one thread per function.
-__global__ __launch_bounds__(256) void k_force_fn(const int* __restrict__ memb_off,
-                                                  const int2* __restrict__ memb,
-                                                  const DevGroup* __restrict__ groups,
-                                                  const double* __restrict__ gsum, int M,
-                                                  double* __restrict__ fsum) {
-  const int I = blockIdx.x * blockDim.x + threadIdx.x;
-  if (I >= M) return;
-  double s[3] = {0.0, 0.0, 0.0};
-  for (int k = memb_off[I]; k < memb_off[I + 1]; ++k) {
-    const int2 u = memb[k];
-    const double* gs = gsum + 3LL * (groups[u.x].fn_off + u.y);
-    s[0] += gs[0];
-    s[1] += gs[1];
-    s[2] += gs[2];
-  }
-  fsum[3LL * I] = s[0];
-  fsum[3LL * I + 1] = s[1];
-  fsum[3LL * I + 2] = s[2];
-}
-
 // Force on batch atom A (atom-major out[3 A + a]) = -2 sum over A's functions
-// (ascending) of their function sums.
-__global__ __launch_bounds__(64) void k_force_atom(const int* __restrict__ afn_off,
-                                                   const int* __restrict__ afn,
-                                                   const double* __restrict__ fsum, int natom,
-                                                   double* __restrict__ out) {
-  const int A = blockIdx.x * blockDim.x + threadIdx.x;
-  if (A >= natom) return;
+// and the groups holding them of their group sums.  One block per atom: wave w
+// takes A's functions w, w + 4, ..., its lanes the groups of each by turns
+// (membf: the function's place in the group sums), then a butterfly over the
+// lanes and the waves in order.  (A thread per function walking its groups
+// took 42 us at (H2O)32.)
+__global__ __launch_bounds__(256) void k_force_atom(const int* __restrict__ afn_off,
+                                                    const int* __restrict__ afn,
+                                                    const int* __restrict__ memb_off,
+                                                    const int* __restrict__ membf,
+                                                    const double* __restrict__ gsum,
+                                                    double* __restrict__ out) {
+  __shared__ double sw[4][3];
+  const int A = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   double s[3] = {0.0, 0.0, 0.0};
-  for (int q = afn_off[A]; q < afn_off[A + 1]; ++q) {
-    const double* fs = fsum + 3LL * afn[q];
-    s[0] += fs[0];
-    s[1] += fs[1];
-    s[2] += fs[2];
+  for (int q = afn_off[A] + wave; q < afn_off[A + 1]; q += 4) {
+    const int f = afn[q];
+    for (int k = memb_off[f] + lane; k < memb_off[f + 1]; k += 64) {
+      const double* gs = gsum + 3LL * membf[k];
+      s[0] += gs[0];
+      s[1] += gs[1];
+      s[2] += gs[2];
+    }
   }
-  out[3 * A + 0] = -2.0 * s[0];
-  out[3 * A + 1] = -2.0 * s[1];
-  out[3 * A + 2] = -2.0 * s[2];
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1)
+#pragma unroll
+    for (int a = 0; a < 3; ++a) s[a] += __shfl_xor(s[a], o);
+  if (lane == 0)
+    for (int a = 0; a < 3; ++a) sw[wave][a] = s[a];
+  __syncthreads();
+  if (threadIdx.x < 3) {
+    const int a = threadIdx.x;
+    out[3 * A + a] = -2.0 * (((sw[0][a] + sw[1][a]) + sw[2][a]) + sw[3][a]);
+  }
 }
 
 // F_g tile (ti, tj) = sum over slices, in slice order.  Block b of a tile
@@ -3002,37 +3007,66 @@ __global__ __launch_bounds__(256) void k_fock_group(const DevGroup* __restrict__
 // functions, in ascending group order.  memb holds, per function, its
 // (group, local index) pairs sorted by group.  I (blockIdx.y) and J are
 // batch function indices; J runs over the rest of I's molecule.  The block
-// first maps each group of I's molecule to I's local index in it (-1 where
-// I is absent) in LDS; each thread then walks J's list alone, in ascending
-// group order, so the sum is the same as a merge of the two lists.
-__global__ void k_fock_pack(const int* __restrict__ memb_off, const int2* __restrict__ memb,
-                            const DevGroup* __restrict__ groups, const DevMol* __restrict__ mols,
-                            const int* __restrict__ fn_mol, const double* __restrict__ fg,
-                            double* __restrict__ F) {
-  extern __shared__ int smap[];
+// first maps each group of I's molecule to I's row of its F_g in LDS (-1 where
+// I is absent; a group lists its functions ascending, so J's local index is
+// not below I's).  kPackLanes lanes then share J's list, each every
+// kPackLanes-th entry, and a butterfly adds them: the walk is a few loads deep
+// instead of one or two per group (latency bounds it: (H2O)32 42 -> 26 us,
+// one water 16 -> 6, 195 atoms 660 -> 400 with one thread per J and the
+// group looked up for every entry).
+constexpr int kPackLanes = 8, kPackCols = 256 / kPackLanes;
+__global__ __launch_bounds__(256) void k_fock_pack(const int* __restrict__ memb_off,
+                                                   const int2* __restrict__ memb,
+                                                   const DevGroup* __restrict__ groups,
+                                                   const DevMol* __restrict__ mols,
+                                                   const int* __restrict__ fn_mol,
+                                                   const double* __restrict__ fg,
+                                                   double* __restrict__ F) {
+  extern __shared__ long long srow[];
   const int I = blockIdx.y;
   const DevMol mol = mols[fn_mol[I]];
-  for (int q = threadIdx.x; q < mol.ng; q += blockDim.x) smap[q] = -1;
+  const int j0 = blockIdx.x * kPackCols;
+  if (j0 >= mol.M || mol.fn_base + j0 + kPackCols <= I) return;  // whole blocks
+  const int J = mol.fn_base + j0 + threadIdx.x / kPackLanes;
+  const bool in = J < mol.fn_base + mol.M && J >= I;
+  const int l = threadIdx.x % kPackLanes;
+  const int b0 = in ? memb_off[J] : 0, be = in ? memb_off[J + 1] : 0;
+  for (int q = threadIdx.x; q < mol.ng; q += 256) srow[q] = -1;
   __syncthreads();
-  for (int a = memb_off[I] + threadIdx.x; a < memb_off[I + 1]; a += blockDim.x) {
+  for (int a = memb_off[I] + threadIdx.x; a < memb_off[I + 1]; a += 256) {
     const int2 u = memb[a];
-    smap[u.x - mol.g0] = u.y;
+    srow[u.x - mol.g0] = groups[u.x].pg_off + (long long)u.y * groups[u.x].m_pad;
   }
   __syncthreads();
-  const int J = mol.fn_base + blockIdx.x * blockDim.x + threadIdx.x;
-  if (J >= mol.fn_base + mol.M || J < I) return;
   double s = 0.0;
-  for (int b = memb_off[J]; b < memb_off[J + 1]; ++b) {
+#pragma unroll 4
+  for (int b = b0 + l; b < be; b += kPackLanes) {
     const int2 v = memb[b];
-    const int ui = smap[v.x - mol.g0];
-    if (ui >= 0) {
-      const DevGroup g = groups[v.x];
-      const int li = min(ui, v.y), lj = max(ui, v.y);
-      s += fg[g.pg_off + (long long)li * g.m_pad + lj];
-    }
+    const long long r = srow[v.x - mol.g0];
+    if (r >= 0) s += fg[r + v.y];
   }
-  F[mol.rho_off + packed_index(I - mol.fn_base, J - mol.fn_base, mol.M)] = s;
+#pragma unroll
+  for (int o = 1; o < kPackLanes; o <<= 1) s += __shfl_xor(s, o);
+  if (in && l == 0)
+    F[mol.rho_off + packed_index(I - mol.fn_base, J - mol.fn_base, mol.M)] = s;
 }
+
+// The sum of k_fock_pack in one thread: entry i of J's list belongs to lane
+// i % kPackLanes, the lanes added as the butterfly does.
+struct PackSum {
+  double s[kPackLanes] = {};
+  __device__ inline void add(int i, double x) {
+#pragma unroll
+    for (int k = 0; k < kPackLanes; ++k) s[k] += (i % kPackLanes) == k ? x : 0.0;
+  }
+  __device__ inline double total() {
+#pragma unroll
+    for (int o = 1; o < kPackLanes; o <<= 1)
+#pragma unroll
+      for (int k = 0; k < kPackLanes; k += 2 * o) s[k] += s[k + o];
+    return s[0];
+  }
+};
 
 // The same by merging the two sorted lists, for molecules with more groups
 // than the LDS map holds.
@@ -3046,7 +3080,8 @@ __global__ void k_fock_pack_merge(const int* __restrict__ memb_off, const int2* 
   if (J >= mol.fn_base + mol.M || J < I) return;
   int a = memb_off[I], ae = memb_off[I + 1];
   int b = memb_off[J], be = memb_off[J + 1];
-  double s = 0.0;
+  const int b0 = b;
+  PackSum s;
   while (a < ae && b < be) {
     const int2 u = memb[a], v = memb[b];
     if (u.x < v.x) {
@@ -3056,12 +3091,12 @@ __global__ void k_fock_pack_merge(const int* __restrict__ memb_off, const int2* 
     } else {
       const DevGroup g = groups[u.x];
       const int li = min(u.y, v.y), lj = max(u.y, v.y);
-      s += fg[g.pg_off + (long long)li * g.m_pad + lj];
+      s.add(b - b0, fg[g.pg_off + (long long)li * g.m_pad + lj]);
       ++a;
       ++b;
     }
   }
-  F[mol.rho_off + packed_index(I - mol.fn_base, J - mol.fn_base, mol.M)] = s;
+  F[mol.rho_off + packed_index(I - mol.fn_base, J - mol.fn_base, mol.M)] = s.total();
 }
 
 // Fixed-order reduction of the per-block (Exc, N) pairs of each molecule
@@ -3073,9 +3108,11 @@ __global__ __launch_bounds__(1024) void k_energy(const double* __restrict__ epar
   __shared__ double se[1024], sn[1024];
   const DevMol mol = mols[blockIdx.x];
   double e = 0.0, c = 0.0;
+#pragma unroll 4
   for (int i = mol.eb + threadIdx.x; i < mol.ee; i += 1024) {
-    e += epart[2 * eidx[i]];
-    c += epart[2 * eidx[i] + 1];
+    const double2 x = reinterpret_cast<const double2*>(epart)[eidx[i]];
+    e += x.x;
+    c += x.y;
   }
   se[threadIdx.x] = e;
   sn[threadIdx.x] = c;
@@ -3265,7 +3302,7 @@ __global__ __launch_bounds__(256, 2) void k_build_persist(PersistArgs* pargs, in
       if (J < mol.fn_base + mol.M && J >= I) {
         int u0 = a.memb_off[I], ue = a.memb_off[I + 1];
         int v0 = a.memb_off[J], ve = a.memb_off[J + 1];
-        double sum = 0.0;
+        PackSum sum;
         while (u0 < ue && v0 < ve) {
           const int2 u = a.memb[u0], v = a.memb[v0];
           if (u.x < v.x) {
@@ -3275,12 +3312,12 @@ __global__ __launch_bounds__(256, 2) void k_build_persist(PersistArgs* pargs, in
           } else {
             const DevGroup gg = a.groups[u.x];
             const int li = min(u.y, v.y), lj = max(u.y, v.y);
-            sum += a.fg[gg.pg_off + (long long)li * gg.m_pad + lj];
+            sum.add(v0 - a.memb_off[J], a.fg[gg.pg_off + (long long)li * gg.m_pad + lj]);
             ++u0;
             ++v0;
           }
         }
-        F[mol.rho_off + packed_index(I - mol.fn_base, J - mol.fn_base, mol.M)] = sum;
+        F[mol.rho_off + packed_index(I - mol.fn_base, J - mol.fn_base, mol.M)] = sum.total();
       }
     } else {
       // energies: the 1024-lane fixed-order reduction of the phase launch,
@@ -4059,7 +4096,7 @@ struct DeviceGrid {
   DensityItem* citems = nullptr;  // force blocks
   double* gpart = nullptr;        // per block and function (3)
   double* gsum = nullptr;         // per group and function (3)
-  double* fsum = nullptr;         // per batch function (3): its groups' sums
+  int* membf = nullptr;           // per memb entry: the function's row of gsum
   int* afn_off = nullptr;         // functions of each batch atom
   int* afn = nullptr;
   double* fout = nullptr;         // forces, natom x 3 (atom-major)
@@ -4728,6 +4765,8 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
     memb.insert(memb.end(), membership[f].begin(), membership[f].end());
   }
   moff[M] = (int)memb.size();
+  std::vector<int> membf(memb.size());
+  for (size_t k = 0; k < memb.size(); ++k) membf[k] = groups[memb[k].x].fn_off + memb[k].y;
 
   auto plan = [&](Carver& c) {
     dg->bas = c.take<DevFn>(M);
@@ -4761,7 +4800,7 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
     dg->citems = c.take<DensityItem>(citems.size());
     dg->gpart = c.take<double>(go);
     dg->gsum = c.take<double>(3 * fnl.size());
-    dg->fsum = c.take<double>(3 * (size_t)M + 3);
+    dg->membf = c.take<int>(memb.size() + 1);
     dg->afn_off = c.take<int>(afn_off.size());
     dg->afn = c.take<int>(afn.size());
     dg->fout = c.take<double>(3 * (size_t)dg->natom);
@@ -4875,6 +4914,7 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
   up(dg->pw, hw.data(), hw.size() * sizeof(double));
   up(dg->memb_off, moff.data(), moff.size() * sizeof(int));
   up(dg->memb, memb.data(), memb.size() * sizeof(int2));
+  up(dg->membf, membf.data(), membf.size() * sizeof(int));
   up(dg->mols, hmol.data(), hmol.size() * sizeof(DevMol));
   up(dg->fn_mol, fn_mol.data(), fn_mol.size() * sizeof(int));
   up(dg->eidx, eidx.data(), eidx.size() * sizeof(int));
@@ -5790,15 +5830,12 @@ static void launch_forces(DeviceGrid& g, hipStream_t s, double* d_forces) {
                            static_cast<const float*>(g.vals), factor, g.gpart);
     }
     if (g.ngroups > 0)
-      hipLaunchKernelGGL(k_force_group, dim3(g.ngroups, (3 * g.max_mpad + 255) / 256), dim3(256),
+      hipLaunchKernelGGL(k_force_group, dim3(g.ngroups, (3 * g.max_mpad + 63) / 64), dim3(256),
                          0, s, g.groups, g.gpart, g.gsum, sp);
   }
-  if (g.M > 0)
-    hipLaunchKernelGGL(k_force_fn, dim3((g.M + 255) / 256), dim3(256), 0, s, g.memb_off, g.memb,
-                       g.groups, g.gsum, g.M, g.fsum);
   if (g.natom > 0)
-    hipLaunchKernelGGL(k_force_atom, dim3((g.natom + 63) / 64), dim3(64), 0, s, g.afn_off, g.afn,
-                       g.fsum, g.natom, d_forces);
+    hipLaunchKernelGGL(k_force_atom, dim3(g.natom), dim3(256), 0, s, g.afn_off, g.afn, g.memb_off,
+                       g.membf, g.gsum, d_forces);
   XCQ_HIP(hipGetLastError());
 }
 
@@ -5850,8 +5887,8 @@ static void launch_all(DeviceGrid& g, hipStream_t s, const double* d_rho, double
     launch_fock(g, s, sp == 1 ? g.factor_b : g.factor);
     if (sp == 0) mark(ev, 3, s);
     if (g.max_ng <= kPackMapMax)
-      hipLaunchKernelGGL(k_fock_pack, dim3((g.max_M + 127) / 128, g.M), dim3(128),
-                         (size_t)g.max_ng * sizeof(int), s, g.memb_off, g.memb, g.groups, g.mols,
+      hipLaunchKernelGGL(k_fock_pack, dim3((g.max_M + kPackCols - 1) / kPackCols, g.M), dim3(256),
+                         (size_t)g.max_ng * sizeof(long long), s, g.memb_off, g.memb, g.groups, g.mols,
                          g.fn_mol, g.fg, d_fock + sp * g.packed);
     else
       hipLaunchKernelGGL(k_fock_pack_merge, dim3((g.max_M + 127) / 128, g.M), dim3(128), 0, s,

@@ -274,11 +274,41 @@ __device__ inline long long fm_row(int mp, int p) {
   return (long long)(p >> 4) * (16 * mp) + (p & 15);
 }
 
+// Block b of a tile evaluation: the groups heavy first (order), of each its
+// tiles of 64 points, of each its blocks of FNS functions, laid end to end
+// (first[i]: the first of group order[i]; first[ng]: the total); XCD b % 8 takes
+// the (b % 8)-th eighth, so that a tile's function blocks, neighbours in
+// memory, are written through one L2.  Found by bisection: a list of them is
+// half a million entries at 195 atoms, made and uploaded at every rebuild (a
+// loop over the function blocks instead cost the registers of a third of the
+// waves: 11.3 ms against 8.3).
+struct TileBlock {
+  int group, p0, k;
+};
+template <int FNS>
+__device__ inline TileBlock tile_block(const int* __restrict__ first, const int* __restrict__ order,
+                                       int ng, const DevGroup* __restrict__ groups) {
+  const int total = first[ng], len = (total + kXcds - 1) / kXcds;
+  const int b = (int)(blockIdx.x % kXcds) * len + (int)(blockIdx.x / kXcds);
+  if (b >= total) return {-1, 0, 0};
+  int lo = 0, hi = ng;  // first[lo] <= b < first[hi]
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (first[mid] <= b)
+      lo = mid;
+    else
+      hi = mid;
+  }
+  const int g = order[lo], nb = (groups[g].m_pad + FNS - 1) / FNS, r = b - first[lo];
+  return {g, 64 * (r / nb), FNS * (r % nb)};
+}
+
 // The values of 64 points and 16 functions: lane l of wave w holds point l and
 // evaluates functions 4 w .. 4 w + 3 (the function records wave-uniform).
 constexpr int kFmFns = 16;
 template <int NV, class T>
-__global__ __launch_bounds__(256) void k_eval_fm(const EvalItem* __restrict__ items,
+__global__ __launch_bounds__(256) void k_eval_fm(const int* __restrict__ first,
+                                                 const int* __restrict__ order, int ng,
                                                  const DevGroup* __restrict__ groups,
                                                  const int* __restrict__ fnl,
                                                  const DevFn* __restrict__ bas,
@@ -286,7 +316,7 @@ __global__ __launch_bounds__(256) void k_eval_fm(const EvalItem* __restrict__ it
                                                  const double* __restrict__ py,
                                                  const double* __restrict__ pz,
                                                  T* __restrict__ vals) {
-  const EvalItem it = items[blockIdx.x];
+  const TileBlock it = tile_block<kFmFns>(first, order, ng, groups);
   if (it.group < 0) return;
   const DevGroup g = groups[it.group];
   const int lane = threadIdx.x & 63;
@@ -331,20 +361,18 @@ __device__ inline double density_entry(const DevMol& mol, const double* __restri
 // l % 16 and columns l / 16 and l / 16 + 4 of the eight: the two A operands of
 // a lane are one load and a wave's load one run (1 KB in FP64).
 template <class T>
-__global__ __launch_bounds__(256) void k_gather_density(const GatherItem* __restrict__ items,
-                                                        const DevGroup* __restrict__ groups,
+__global__ __launch_bounds__(256) void k_gather_density(const DevGroup* __restrict__ groups,
                                                         const DevMol* __restrict__ mols,
                                                         const int* __restrict__ fnl,
                                                         const double* __restrict__ rho,
                                                         T* __restrict__ pg) {
-  const GatherItem it = items[blockIdx.x];
-  const DevGroup g = groups[it.group];
-  const int e = it.start + threadIdx.x;
-  if (e >= g.m_pad * g.m_pad) return;
-  const int u = e >> 7, nk8 = g.m_pad >> 3, l = (e >> 1) & 63;
-  const int k = 16 * (u / nk8) + (l & 15), j = 8 * (u % nk8) + 4 * (e & 1) + (l >> 4);
-  const double v = density_entry(mols[g.mol], rho, fnl[g.fn_off + k], fnl[g.fn_off + j]);
-  pg[g.pg_off + e] = (T)v;
+  const DevGroup g = groups[blockIdx.x];
+  const DevMol mol = mols[g.mol];
+  for (int e = blockIdx.y * 256 + threadIdx.x; e < g.m_pad * g.m_pad; e += 256 * gridDim.y) {
+    const int u = e >> 7, nk8 = g.m_pad >> 3, l = (e >> 1) & 63;
+    const int k = 16 * (u / nk8) + (l & 15), j = 8 * (u % nk8) + 4 * (e & 1) + (l >> 4);
+    pg[g.pg_off + e] = (T)density_entry(mol, rho, fnl[g.fn_off + k], fnl[g.fn_off + j]);
+  }
 }
 
 // Functional stage of a density launch for point q from its row-dot sums s
@@ -710,9 +738,10 @@ __device__ inline void load8t(const float* row, int f, float (&x)[8]) {
 // function records wave-uniform), which are one 16-byte store per plane, 16
 // lanes a contiguous 256 bytes, with no transpose.  Also phi's remainder in
 // BF16 and the function-major phi plane of the Fock kernel (rows of 64
-// points).  Items as in k_eval_pm.
+// points).
 template <int NV>
-__global__ __launch_bounds__(512) void k_eval_tl(const EvalItem* __restrict__ items,
+__global__ __launch_bounds__(512) void k_eval_tl(const int* __restrict__ first,
+                                                 const int* __restrict__ order, int ng,
                                                  const DevGroup* __restrict__ groups,
                                                  const int* __restrict__ fnl,
                                                  const DevFn* __restrict__ bas,
@@ -722,7 +751,7 @@ __global__ __launch_bounds__(512) void k_eval_tl(const EvalItem* __restrict__ it
                                                  float* __restrict__ vals,
                                                  float* __restrict__ phiT,
                                                  unsigned short* __restrict__ lo16) {
-  const EvalItem it = items[blockIdx.x];
+  const TileBlock it = tile_block<kPmFns>(first, order, ng, groups);
   if (it.group < 0) return;
   const DevGroup g = groups[it.group];
   const int lane = threadIdx.x & 63;
@@ -731,8 +760,8 @@ __global__ __launch_bounds__(512) void k_eval_tl(const EvalItem* __restrict__ it
   if (p >= g.npts_pad) return;
   const int q = g.pt_off + p;
   const double x = px[q], y = py[q], z = pz[q];
-  const int k = it.k + 4 * wave;
   const long long plane = (long long)g.m_pad * g.npts_pad;
+  const int k = it.k + 4 * wave;
   float o[NV][4];
   unsigned short l[4];
 #pragma unroll
@@ -759,7 +788,8 @@ __global__ __launch_bounds__(512) void k_eval_tl(const EvalItem* __restrict__ it
 }
 
 template <int NV, bool LO = false>
-__global__ __launch_bounds__(512) void k_eval_pm(const EvalItem* __restrict__ items,
+__global__ __launch_bounds__(512) void k_eval_pm(const int* __restrict__ first,
+                                                 const int* __restrict__ order, int ng,
                                                  const DevGroup* __restrict__ groups,
                                                  const int* __restrict__ fnl,
                                                  const DevFn* __restrict__ bas,
@@ -771,7 +801,7 @@ __global__ __launch_bounds__(512) void k_eval_pm(const EvalItem* __restrict__ it
                                                  unsigned short* __restrict__ lo16) {
   constexpr int NP = NV + (LO ? 1 : 0), FW = kPmFns / 8;  // functions per wave
   __shared__ float sT[2][kPmFns][kPmPts + 1];
-  const EvalItem it = items[blockIdx.x];
+  const TileBlock it = tile_block<kPmFns>(first, order, ng, groups);
   if (it.group < 0) return;
   const DevGroup g = groups[it.group];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -901,13 +931,12 @@ __device__ inline void radial_hessian(const FnMeta& mt, float vx, float vy, floa
 // half a line per row and step), copied to LDS as it stands and read there
 // by lane without bank conflicts.  A block covers 8 rows of one K block.
 template <int NPC, bool FRAG>
-__device__ __forceinline__ void gather_bf_item(const int bi, const GatherItem* __restrict__ items,
+__device__ __forceinline__ void gather_bf_item(const GatherItem it,
                                                            const DevGroup* __restrict__ groups,
                                                            const DevMol* __restrict__ mols,
                                                            const int* __restrict__ fnl,
                                                            const double* __restrict__ rho,
                                                            unsigned short* __restrict__ pgs) {
-  const GatherItem it = items[bi];
   const DevGroup g = groups[it.group];
   const int e = it.start + threadIdx.x;
   const long long psz = (long long)g.m_pad * g.m_pad;
@@ -948,13 +977,14 @@ __device__ __forceinline__ void gather_bf_item(const int bi, const GatherItem* _
 }
 
 template <int NPC, bool FRAG = false>
-__global__ __launch_bounds__(256) void k_gather_density_bf(const GatherItem* __restrict__ items,
-                                                           const DevGroup* __restrict__ groups,
+__global__ __launch_bounds__(256) void k_gather_density_bf(const DevGroup* __restrict__ groups,
                                                            const DevMol* __restrict__ mols,
                                                            const int* __restrict__ fnl,
                                                            const double* __restrict__ rho,
                                                            unsigned short* __restrict__ pgs) {
-  gather_bf_item<NPC, FRAG>(blockIdx.x, items, groups, mols, fnl, rho, pgs);
+  const int mp = groups[blockIdx.x].m_pad;
+  for (int e0 = blockIdx.y * 256; e0 < mp * mp; e0 += 256 * gridDim.y)
+    gather_bf_item<NPC, FRAG>(GatherItem{(int)blockIdx.x, e0}, groups, mols, fnl, rho, pgs);
 }
 
 // Density + functional on split-BF16 MFMA: same blocking as k_density (64
@@ -3267,7 +3297,7 @@ __global__ __launch_bounds__(256, 2) void k_build_persist(PersistArgs* pargs, in
     int* tdone = ddone + a.ngroups;
     if (it >= a.n5) break;
     if (it < a.n0) {
-      gather_bf_item<4, false>(it, a.gitems, a.groups, a.mols, a.fnl, rho, a.pg);
+      gather_bf_item<4, false>(a.gitems[it], a.groups, a.mols, a.fnl, rho, a.pg);
       persist_signal(&gdone[a.gitems[it].group]);
     } else if (it < a.n1) {
       const int d = it - a.n0, g = a.ditems[d].group;
@@ -4043,7 +4073,7 @@ struct DeviceGrid {
   int* fn_mol = nullptr;
   int* eidx = nullptr;
   bool gga = true;
-  int ngroups = 0, neval = 0, ngather = 0, ndensity = 0, nfock = 0, ngroup_tiles = 0;
+  int ngroups = 0, neval = 0, ndensity = 0, nfock = 0, ngroup_tiles = 0;
   int nforce = 0;                        // force blocks (64 points each)
   long long npts_pad = 0, val_elems = 0, pg_elems = 0;
   char* arena = nullptr;
@@ -4055,15 +4085,20 @@ struct DeviceGrid {
   DevFn* bas = nullptr;
   DevGroup* groups = nullptr;
   EvalItem* eitems = nullptr;
-  GatherItem* gitems = nullptr;
-  EvalItem* pmitems = nullptr;  // point-major evaluation blocks (split-BF16)
-  int npm = 0;
+  GatherItem* gitems = nullptr;  // P_g expansion blocks of the persistent build
+  int *tfirst = nullptr, *torder = nullptr;  // tile evaluation blocks (tile_block)
+  int ntile = 0;
   float* phiT = nullptr;          // function-major phi (split-BF16 Fock operand)
   void* ybuf = nullptr;           // Y = P_g phi per point and function (force pass), in the
                                   // planes' layout and type; allocated at the first forces
                                   // build (not in the arena)
   size_t ybuf_cap = 0;            // its bytes
   bool y_denied = false;          // no memory for it: FP64 and FP32 forces recompute Y
+  // P_g expansion: up to 256 blocks per group, each looping
+  dim3 gather_grid() const {
+    return dim3((unsigned)ngroups, (unsigned)std::max(
+                                       1LL, std::min(256LL, ((long long)max_mpad * max_mpad + 255) / 256)));
+  }
   // values of Y per spin
   long long yelems() const {
     return prec == Precision::BF16X6 ? phi_elems : val_elems / nval;
@@ -4591,50 +4626,40 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
   std::stable_sort(order.begin(), order.end(),
                    [&](int a, int b) { return groups[a].m_pad > groups[b].m_pad; });
   std::vector<EvalItem> eitems;
+  const bool persist = tuning_.persistent != 0 && bf && dg->density_variant == 8 && !dg->open;
   std::vector<GatherItem> gitems, ritems;
-  std::vector<EvalItem> pmitems;
-  size_t pm_len = 0;
   // split-BF16 variant 3: groups of more than 64 functions run the row-split
   // kernel on 16-point blocks (listed first), the rest 64-point blocks
   const bool rowsplit = bf && (tuning_.density_variant == 3 || tuning_.density_variant == 4);
   std::vector<DensityItem> ditems, dsmall, citems;
   // the function-major evaluation (phi alone) runs for the in-kernel variants,
-  // the tile evaluations (64 points x pm_fns functions) otherwise
-  const bool fm_eval = dg->inkernel, pm_eval = !dg->inkernel;
-  const int pm_fns = bf ? kPmFns : kFmFns;
+  // the tile evaluations (64 points x tile_fns functions) otherwise
+  const bool fm_eval = dg->inkernel;
+  const int tile_fns = bf ? kPmFns : kFmFns;
+  std::vector<int> tfirst(1, 0);  // tile evaluation: each group's first block, in order
   {  // the lists' lengths first: millions of items for large molecules
-    size_t ne = 0, ng = 0, npm = 0, nt = 0;
+    size_t ne = 0, ng = 0, nt = 0;
     for (int g = 0; g < G; ++g) {
       const DevGroup& d = groups[g];
       const size_t tiles = (d.npts_pad + kDensPts - 1) / kDensPts;
       nt += tiles;
       if (fm_eval) ne += (size_t)d.m_pad * ((d.npts_pad + kEvalSpan - 1) / kEvalSpan);
-      ng += ((size_t)d.m_pad * d.m_pad + 255) / 256;
-      if (pm_eval)
-        npm += (size_t)((d.npts_pad + kPmPts - 1) / kPmPts) * ((d.m_pad + pm_fns - 1) / pm_fns);
+      if (persist) ng += ((size_t)d.m_pad * d.m_pad + 255) / 256;
     }
     citems.reserve(nt);
     dsmall.reserve(nt);
     eitems.reserve(ne);
     gitems.reserve(ng);
-    // the point-major items XCD-interleaved: block b runs on XCD b % 8 and
-    // takes item b / 8 of the list's (b % 8)-th eighth, so the function
-    // chunks of one point tile, the rows of the same points, are written
-    // through one L2 (items of group -1 pad the eighths)
-    pm_len = (npm + kXcds - 1) / kXcds;
-    pmitems.assign(kXcds * pm_len, EvalItem{-1, 0, 0, 0});
   }
-  size_t pm_next = 0;
   for (int g : order) {
     const DevGroup& d = groups[g];
     for (int p0 = 0; p0 < d.npts_pad; p0 += kDensPts) citems.push_back(DensityItem{g, p0});
     for (int k = 0; fm_eval && k < d.m_pad; ++k)
       for (int p0 = 0; p0 < d.npts_pad; p0 += kEvalSpan) eitems.push_back(EvalItem{g, k, p0, 0});
-    for (int e0 = 0; e0 < d.m_pad * d.m_pad; e0 += 256) gitems.push_back(GatherItem{g, e0});
-    if (pm_eval)
-      for (int p0 = 0; p0 < d.npts_pad; p0 += kPmPts)
-        for (int k0 = 0; k0 < d.m_pad; k0 += pm_fns, ++pm_next)
-          pmitems[kXcds * (pm_next % pm_len) + pm_next / pm_len] = EvalItem{g, k0, p0, 0};
+    for (int e0 = 0; persist && e0 < d.m_pad * d.m_pad; e0 += 256)
+      gitems.push_back(GatherItem{g, e0});
+    tfirst.push_back(tfirst.back() + (d.npts_pad + kDensPts - 1) / kDensPts *
+                                         ((d.m_pad + tile_fns - 1) / tile_fns));
     if (dg->radial)
       for (int e0 = 0; e0 < d.nsh_pad * d.npts_pad; e0 += kEvalSpan)
         ritems.push_back(GatherItem{g, e0});
@@ -4721,7 +4746,7 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
   // persistent build: per-group item counts, each group's first tile pair,
   // the packing items and the queue orders of the Fock and tile-sum items
   // (groups in the density order, heavy first)
-  dg->persistent = tuning_.persistent != 0 && bf && dg->density_variant == 8 && !dg->open;
+  dg->persistent = persist;
   std::vector<int> gneed, dneed, tbase, fperm, tperm;
   std::vector<int2> pitems;
   if (dg->persistent) {
@@ -4752,8 +4777,7 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
     dg->persist_blocks = 2 * std::max(1, cus);
   }
   dg->neval = (int)eitems.size();
-  dg->ngather = (int)gitems.size();
-  dg->npm = (int)pmitems.size();
+  dg->ntile = dg->inkernel ? 0 : (tfirst.back() + kXcds - 1) / kXcds * kXcds;
   dg->nrad = (int)ritems.size();
   dg->ndensity = (int)ditems.size();
   dg->nforce = (int)citems.size();
@@ -4773,7 +4797,8 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
     dg->groups = c.take<DevGroup>(G);
     dg->eitems = c.take<EvalItem>(eitems.size());
     dg->gitems = c.take<GatherItem>(gitems.size());
-    dg->pmitems = c.take<EvalItem>(pmitems.size());
+    dg->tfirst = c.take<int>(tfirst.size());
+    dg->torder = c.take<int>(order.size());
     dg->phiT = c.take<float>(fo);
     dg->ditems = c.take<DensityItem>(ditems.size());
     dg->fitems = c.take<FockItem>(fitems.size());
@@ -4903,7 +4928,8 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
   up(dg->groups, groups.data(), groups.size() * sizeof(DevGroup));
   up(dg->eitems, eitems.data(), eitems.size() * sizeof(EvalItem));
   up(dg->gitems, gitems.data(), gitems.size() * sizeof(GatherItem));
-  up(dg->pmitems, pmitems.data(), pmitems.size() * sizeof(EvalItem));
+  up(dg->tfirst, tfirst.data(), tfirst.size() * sizeof(int));
+  up(dg->torder, order.data(), order.size() * sizeof(int));
   up(dg->ditems, ditems.data(), ditems.size() * sizeof(DensityItem));
   up(dg->fitems, fitems.data(), fitems.size() * sizeof(FockItem));
   up(dg->gtiles, gtiles.data(), gtiles.size() * sizeof(int2));
@@ -4995,40 +5021,29 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
   hipEvent_t* ev = reinterpret_cast<hipEvent_t*>(events_);
   const double t_eval = wall();
   XCQ_HIP(hipEventRecord(ev[6], s));
-  if (dg->neval > 0 || dg->npm > 0) {
-    const dim3 grid(dg->neval), block(kEvalPts);
+  if (dg->neval > 0 || dg->ntile > 0) {
+    const dim3 grid(dg->neval), block(kEvalPts), tgrid(std::max(1, dg->ntile));
     if (prec == Precision::FP64) {
-      hipLaunchKernelGGL((dg->gga ? k_eval_fm<10, double> : k_eval_fm<4, double>), dim3(dg->npm),
-                         dim3(256), 0, s, dg->pmitems, dg->groups, dg->fnl, dg->bas, dg->px, dg->py,
+      hipLaunchKernelGGL((dg->gga ? k_eval_fm<10, double> : k_eval_fm<4, double>), tgrid,
+                         dim3(256), 0, s, dg->tfirst, dg->torder, G, dg->groups, dg->fnl, dg->bas, dg->px, dg->py,
                          dg->pz, static_cast<double*>(dg->vals));
     } else if (prec == Precision::FP32) {
-      hipLaunchKernelGGL((dg->gga ? k_eval_fm<10, float> : k_eval_fm<4, float>), dim3(dg->npm),
-                         dim3(256), 0, s, dg->pmitems, dg->groups, dg->fnl, dg->bas, dg->px, dg->py,
+      hipLaunchKernelGGL((dg->gga ? k_eval_fm<10, float> : k_eval_fm<4, float>), tgrid,
+                         dim3(256), 0, s, dg->tfirst, dg->torder, G, dg->groups, dg->fnl, dg->bas, dg->px, dg->py,
                          dg->pz, static_cast<float*>(dg->vals));
     } else if (dg->inkernel) {  // phi alone, function-major, for the Fock kernel
       hipLaunchKernelGGL((k_eval_basis<1, float>), grid, block, 0, s, dg->eitems, dg->groups,
                          dg->fnl, dg->bas, dg->px, dg->py, dg->pz, dg->phiT, 1);
     } else {
       float* v = static_cast<float*>(dg->vals);
-      if (dg->npm > 0) {
-        if (dg->chunked)
-          hipLaunchKernelGGL(dg->gga ? k_eval_tl<10> : k_eval_tl<4>, dim3(dg->npm), dim3(512), 0,
-                             s, dg->pmitems, dg->groups, dg->fnl, dg->bas, dg->px, dg->py, dg->pz,
-                             v, dg->phiT, dg->lo16);
-        else if (dg->lo && dg->gga)
-          hipLaunchKernelGGL((k_eval_pm<10, true>), dim3(dg->npm), dim3(512), 0, s,
-                             dg->pmitems, dg->groups, dg->fnl, dg->bas, dg->px, dg->py, dg->pz, v,
-                             dg->phiT, dg->lo16);
-        else if (dg->lo)
-          hipLaunchKernelGGL((k_eval_pm<4, true>), dim3(dg->npm), dim3(512), 0, s, dg->pmitems,
-                             dg->groups, dg->fnl, dg->bas, dg->px, dg->py, dg->pz, v, dg->phiT, dg->lo16);
-        else if (dg->gga && !dg->radial)
-          hipLaunchKernelGGL((k_eval_pm<10>), dim3(dg->npm), dim3(512), 0, s,
-                             dg->pmitems, dg->groups, dg->fnl, dg->bas, dg->px, dg->py, dg->pz, v,
-                             dg->phiT, dg->lo16);
-        else
-          hipLaunchKernelGGL(k_eval_pm<4>, dim3(dg->npm), dim3(512), 0, s, dg->pmitems, dg->groups,
-                             dg->fnl, dg->bas, dg->px, dg->py, dg->pz, v, dg->phiT, dg->lo16);
+      if (dg->ntile > 0) {
+        const auto kernel = dg->chunked              ? (dg->gga ? k_eval_tl<10> : k_eval_tl<4>)
+                            : dg->lo && dg->gga      ? k_eval_pm<10, true>
+                            : dg->lo                 ? k_eval_pm<4, true>
+                            : dg->gga && !dg->radial ? k_eval_pm<10, false>
+                                                     : k_eval_pm<4, false>;
+        hipLaunchKernelGGL(kernel, tgrid, dim3(512), 0, s, dg->tfirst, dg->torder, G, dg->groups,
+                           dg->fnl, dg->bas, dg->px, dg->py, dg->pz, v, dg->phiT, dg->lo16);
       }
       if (dg->presplit && dg->ndensity > 0)
         hipLaunchKernelGGL(k_split_pm, dim3(dg->ndensity), dim3(256), 0, s, dg->ditems,
@@ -5614,9 +5629,9 @@ static void launch_density(DeviceGrid& g, hipStream_t s, const double* d_rho, in
                            hipEvent_t* ev, void* yb) {
   T* pg = static_cast<T*>(spin == 2 ? g.pg2 : g.pg);
   const double* rho = spin == 2 ? d_rho + g.packed : d_rho;
-  if (g.ngather > 0)
-    hipLaunchKernelGGL(k_gather_density<T>, dim3(g.ngather), dim3(256), 0, s, g.gitems, g.groups,
-                       g.mols, g.fnl, rho, pg);
+  if (g.ngroups > 0)
+    hipLaunchKernelGGL(k_gather_density<T>, g.gather_grid(), dim3(256), 0, s, g.groups, g.mols,
+                       g.fnl, rho, pg);
   if (spin < 2) mark(ev, 1, s);
   if (g.nchunk > 0)
     hipLaunchKernelGGL((g.gga ? k_density_dc<4, T> : k_density_dc<1, T>), dim3(g.nchunk),
@@ -5633,9 +5648,9 @@ static void launch_density_bf(DeviceGrid& g, hipStream_t s, const double* d_rho,
   const double* rho = spin == 2 ? d_rho + g.packed : d_rho;
   const float* vals = static_cast<const float*>(g.vals);
   if (g.inkernel) {  // variants 6 (128-function row chunks) and 7 (64)
-    if (g.ngather > 0)
-      hipLaunchKernelGGL(k_gather_density_bf<4>, dim3(g.ngather), dim3(256), 0, s, g.gitems,
-                         g.groups, g.mols, g.fnl, rho, pg3);
+    if (g.ngroups > 0)
+      hipLaunchKernelGGL(k_gather_density_bf<4>, g.gather_grid(), dim3(256), 0, s, g.groups, g.mols,
+                         g.fnl, rho, pg3);
     if (spin < 2) mark(ev, 1, s);
     float* y = yb ? yb + (spin == 2 ? g.phi_elems : 0) : nullptr;
     if (g.ndensity > 0) {
@@ -5659,15 +5674,11 @@ static void launch_density_bf(DeviceGrid& g, hipStream_t s, const double* d_rho,
   }
   if (g.lo) {  // variants 8 and 9: phi's remainder plane (8: four-piece P_g)
     const bool four = g.density_variant == 8 || g.chunked;
-    if (g.ngather > 0) {
-      if (four)
-        hipLaunchKernelGGL((g.chunked ? k_gather_density_bf<4, true> : k_gather_density_bf<4, false>),
-                           dim3(g.ngather), dim3(256), 0, s, g.gitems, g.groups, g.mols, g.fnl,
-                           rho, pg3);
-      else
-        hipLaunchKernelGGL(k_gather_density_bf<3>, dim3(g.ngather), dim3(256), 0, s, g.gitems,
-                           g.groups, g.mols, g.fnl, rho, pg3);
-    }
+    if (g.ngroups > 0)
+      hipLaunchKernelGGL((g.chunked ? k_gather_density_bf<4, true>
+                          : four    ? k_gather_density_bf<4, false>
+                                    : k_gather_density_bf<3, false>),
+                         g.gather_grid(), dim3(256), 0, s, g.groups, g.mols, g.fnl, rho, pg3);
     if (spin < 2) mark(ev, 1, s);
     float* y = yb ? yb + (spin == 2 ? g.phi_elems : 0) : nullptr;
 
@@ -5695,9 +5706,9 @@ static void launch_density_bf(DeviceGrid& g, hipStream_t s, const double* d_rho,
     XCQ_HIP(hipGetLastError());
     return;
   }
-  if (g.ngather > 0)
-    hipLaunchKernelGGL(k_gather_density_bf<3>, dim3(g.ngather), dim3(256), 0, s, g.gitems,
-                       g.groups, g.mols, g.fnl, rho, pg3);
+  if (g.ngroups > 0)
+    hipLaunchKernelGGL(k_gather_density_bf<3>, g.gather_grid(), dim3(256), 0, s, g.groups, g.mols,
+                       g.fnl, rho, pg3);
   if (spin < 2) mark(ev, 1, s);
   if (g.ndensity > 0) {
     if (g.density_variant == 1) {

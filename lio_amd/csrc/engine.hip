@@ -3413,17 +3413,38 @@ __device__ inline double dist3(double x, double y, double z, double ax, double a
   return sqrt(dx * dx + dy * dy + dz * dz);
 }
 
+// The Becke cell function of the scaled difference u: the size term, then three
+// rounds of 1.5 u - 0.5 u^3.  Halving is exact, so each fma below rounds once
+// where the host's product by 0.5 and difference do, with the same bits.
+__device__ inline double becke_step(double u, double aw) {
+#pragma clang fp contract(off)
+  u += aw * (1.0 - u * u);
+  u = __builtin_fma(-0.5, u * u * u, 1.5 * u);
+  u = __builtin_fma(-0.5, u * u * u, 1.5 * u);
+  u = __builtin_fma(-0.5, u * u * u, 1.5 * u);
+  return __builtin_fma(-0.5, u, 0.5);
+}
+
 // Becke cell function with the pair's size term aw = chi / (chi^2 - 1)
 // taken from a table (the host computes it with the same operations), so a
 // factor costs one division instead of three.
 __device__ inline double becke_cell_w(double dj, double dk, double rjk, double aw) {
 #pragma clang fp contract(off)
-  double u = (dj - dk) / rjk;
-  u += aw * (1.0 - u * u);
-  u = 1.5 * u - 0.5 * (u * u * u);
-  u = 1.5 * u - 0.5 * (u * u * u);
-  u = 1.5 * u - 0.5 * (u * u * u);
-  return 0.5 * (1.0 - u);
+  return becke_step((dj - dk) / rjk, aw);
+}
+
+// The same factor with the quotient formed from the pair's reciprocal rinv =
+// RN(1 / rjk): after one correction by the exact residual q lies within an ulp
+// of the quotient, so the second one rounds it correctly (Markstein, IBM J.
+// Res. Dev. 34, 1990) and the factor has becke_cell_w's bits.  Five operations
+// in place of the division's dozen.
+__device__ inline double becke_cell_r(double dj, double dk, double rjk, double rinv, double aw) {
+#pragma clang fp contract(off)
+  const double a = dj - dk;
+  double q = a * rinv;
+  q = __builtin_fma(__builtin_fma(-q, rjk, a), rinv, q);
+  q = __builtin_fma(__builtin_fma(-q, rjk, a), rinv, q);
+  return becke_step(q, aw);
 }
 
 // Staged points per Becke block; the block has kBeckeLanes waves, one per
@@ -3438,8 +3459,9 @@ constexpr int kBeckePts = 64, kBeckeNear = 64;
 // order the host's becke_order forms with the same operations.  gord holds
 // the nucleus indices in that order, gpos the rank of each list position, and
 // the group's tables in that order follow: the nuclei's coordinates (ox, oy,
-// oz) and, for every list position j and rank t, the pair distance and size
-// term of nuclei j and gord[t] (td, tw, rows of natoms from sq_off), so that
+// oz) and, for every list position j and rank t, the pair distance, its
+// reciprocal and the size term of nuclei j and gord[t] (td, tr, tw, rows of
+// natoms from sq_off; j = gord[t] is never read), so that
 // the Becke products load by rank, with no index load in between.  One block
 // per group.
 __global__ __launch_bounds__(256) void k_becke_order(
@@ -3450,7 +3472,7 @@ __global__ __launch_bounds__(256) void k_becke_order(
     const double* __restrict__ sx, const double* __restrict__ sy,
     const double* __restrict__ sz, int* __restrict__ gord, int* __restrict__ gpos,
     double* __restrict__ ox, double* __restrict__ oy, double* __restrict__ oz,
-    double* __restrict__ td, double* __restrict__ tw) {
+    double* __restrict__ td, double* __restrict__ tr, double* __restrict__ tw) {
   const StGroup G = groups[blockIdx.x];
   if (G.npts == 0) return;
   const StMol m = mols[G.mol];
@@ -3484,6 +3506,7 @@ __global__ __launch_bounds__(256) void k_becke_order(
     const int j = e / k, t = e % k;
     const long long src = (long long)at[j] * na + ord[t];
     td[(long long)G.sq_off + e] = D[src];
+    tr[(long long)G.sq_off + e] = 1.0 / D[src];
     tw[(long long)G.sq_off + e] = W[src];
   }
 }
@@ -3583,15 +3606,24 @@ __global__ __launch_bounds__(kBeckePts) void k_becke_exact(
 // sum and the bound; a zero P_own ends the point.  The group is uniform in
 // the block, so the loops over j and the nuclei's loads are wave-uniform;
 // distances are recomputed instead of stored per point, with the host's
-// values.  The host's weigh (grid.cpp) does the same arithmetic, so the
-// weights are bitwise its weights.
-__global__ __launch_bounds__(kBeckePts * kBeckeLanes) void k_becke(
+// values.  The reference's zero test against n needs no pass of its own: n is
+// among the nuclei of the product, and a zero factor drops it.  The host's
+// weigh (grid.cpp) has the same results of every operation, so the weights
+// are bitwise its weights.
+//
+// Bound by FP64 vector issue, and by the latency of the tables' scalar loads
+// between the factors.  So the quotient comes from a stored reciprocal, two
+// factors are in flight at a time, and the registers are held at 64, so that
+// a block's 8 waves leave room for three other blocks on the unit (two
+// factors need no spills at that; four need eight and measured the same).
+// Against one factor at a time with a division in each and the zero test
+// ahead: 104 -> 75 us for 25 atoms, 2.1 -> 1.62 ms for 110, and 1.4 ms less
+// of 7.0 for 195.
+__global__ __launch_bounds__(kBeckePts * kBeckeLanes, 8) void k_becke(
     const StGroup* __restrict__ groups, const int2* __restrict__ items,
-    const StMol* __restrict__ mols, const int* __restrict__ gatoms,
     const int* __restrict__ gpos, const double* __restrict__ ox, const double* __restrict__ oy,
-    const double* __restrict__ oz, const double* __restrict__ td, const double* __restrict__ tw,
-    const double* __restrict__ ax, const double* __restrict__ ay, const double* __restrict__ az,
-    const double* __restrict__ aw, const double* __restrict__ rij,
+    const double* __restrict__ oz, const double* __restrict__ td, const double* __restrict__ tr,
+    const double* __restrict__ tw,
     const double* __restrict__ sx, const double* __restrict__ sy,
     const double* __restrict__ sz, const double2* __restrict__ bterm,
     const int2* __restrict__ bnuc, double* __restrict__ sw) {
@@ -3606,11 +3638,6 @@ __global__ __launch_bounds__(kBeckePts * kBeckeLanes) void k_becke(
   const StGroup G = groups[gi];
   const bool live = p < G.pt_off + G.npts;
   const int k = G.natoms, kn = min(k, kBeckeNear);
-  const StMol m = mols[G.mol];
-  const int* at = gatoms + G.atom_off;
-  const double* A = ax + m.atom_base;
-  const double* B = ay + m.atom_base;
-  const double* C = az + m.atom_base;
   const double* Xo = ox + G.atom_off;  // the nuclei's coordinates by rank
   const double* Yo = oy + G.atom_off;
   const double* Zo = oz + G.atom_off;
@@ -3624,13 +3651,9 @@ __global__ __launch_bounds__(kBeckePts * kBeckeLanes) void k_becke(
   __syncthreads();
   double mine = 0.0, sum = 0.0;
   if (live && k > 0) {
-    const int na = m.natom;
-    const double* W = aw + m.rij_off;
-    const double* D = rij + m.rij_off;
     const double2 tm = bterm[p];
     const int2 nq = bnuc[p];
-    const int qo = nq.x, qn = nq.y, an = at[qn];
-    const double dn = dist3(x, y, z, A[an], B[an], C[an]);
+    const int qo = nq.x, qn = nq.y;
     const double pn = tm.y;
     mine = tm.x;
     if (mine != 0.0) {
@@ -3644,23 +3667,49 @@ __global__ __launch_bounds__(kBeckePts * kBeckeLanes) void k_becke(
           sum += pn;
           continue;
         }
-        const int aj = at[j];
-        const double dj = dist3(x, y, z, A[aj], B[aj], C[aj]);
-        const double* Dj = D + (long long)aj * na;
-        const double* Wj = W + (long long)aj * na;
-        if (becke_cell_w(dj, dn, Dj[an], Wj[an]) == 0.0) continue;
         const int tj = gpos[G.atom_off + j];  // j's own rank, skipped
+        const double dj = tj < kBeckeNear ? dnear[tj][lane] : dist3(x, y, z, Xo[tj], Yo[tj], Zo[tj]);
         const double* Dr = td + G.sq_off + (long long)j * k;
+        const double* Rr = tr + G.sq_off + (long long)j * k;
         const double* Wr = tw + G.sq_off + (long long)j * k;
         double prod = 1.0;
-        for (int t = 0; t < k; ++t) {
-          if (t == tj) continue;
-          const double dk = t < kBeckeNear ? dnear[t][lane] : dist3(x, y, z, Xo[t], Yo[t], Zo[t]);
-          prod *= becke_cell_w(dj, dk, Dr[t], Wr[t]);
-          if (prod < thr) {
-            prod = 0.0;
-            break;
+        bool low = false;
+        auto factors = [&](int t, const double* dk, auto n) {
+          double s[n];
+#pragma unroll
+          for (int u = 0; u < n; ++u)
+            s[u] = becke_cell_r(dj, dk[u], Dr[t + u], Rr[t + u], Wr[t + u]);
+#pragma unroll
+          for (int u = 0; u < n; ++u) {
+            prod *= t + u == tj ? 1.0 : s[u];
+            low = low || prod < thr;
           }
+        };
+        int t = 0;
+        double dk[2];
+        for (; t + 2 <= kn && !low; t += 2) {
+#pragma unroll
+          for (int u = 0; u < 2; ++u) dk[u] = dnear[t + u][lane];
+          factors(t, dk, std::integral_constant<int, 2>());
+        }
+        for (; t < kn && !low; ++t) {
+          dk[0] = dnear[t][lane];
+          factors(t, dk, std::integral_constant<int, 1>());
+        }
+        for (; t + 2 <= k && !low; t += 2) {
+#pragma unroll
+          for (int u = 0; u < 2; ++u) dk[u] = dist3(x, y, z, Xo[t + u], Yo[t + u], Zo[t + u]);
+          factors(t, dk, std::integral_constant<int, 2>());
+        }
+        for (; t < k && !low; ++t) {
+          dk[0] = dist3(x, y, z, Xo[t], Yo[t], Zo[t]);
+          factors(t, dk, std::integral_constant<int, 1>());
+        }
+        if (low) prod = 0.0;
+        if (prod != prod) {  // coincident nuclei: only now is the zero test against n needed
+          const int tn = gpos[G.atom_off + qn];
+          const double dn = dist3(x, y, z, Xo[tn], Yo[tn], Zo[tn]);
+          if (becke_cell_r(dj, dn, Dr[tn], Rr[tn], Wr[tn]) == 0.0) prod = 0.0;
         }
         sum += prod;
       }
@@ -3678,63 +3727,92 @@ __global__ __launch_bounds__(kBeckePts * kBeckeLanes) void k_becke(
     sw[p] *= (total == 0.0 ? 0.0 : mine / total);
 }
 
+// Threads of the kernels that walk a staged group's points.
+constexpr int kWalkThreads = 1024;
+
 // Points a staged group keeps (all, or those of non-zero weight).
-__global__ __launch_bounds__(256) void k_group_count(const StGroup* __restrict__ groups,
-                                                     const double* __restrict__ sw, int drop_zero,
-                                                     int* __restrict__ count) {
-  __shared__ int sc[4];
+__global__ __launch_bounds__(kWalkThreads) void k_group_count(const StGroup* __restrict__ groups,
+                                                              const double* __restrict__ sw,
+                                                              int drop_zero,
+                                                              int* __restrict__ count) {
+  __shared__ int sc[kWalkThreads / 64];
   const StGroup G = groups[blockIdx.x];
   int c = 0;
-  for (int i = threadIdx.x; i < G.npts; i += 256) c += (!drop_zero || sw[G.pt_off + i] != 0.0);
+  for (int i = threadIdx.x; i < G.npts; i += kWalkThreads)
+    c += (!drop_zero || sw[G.pt_off + i] != 0.0);
   for (int o = 32; o >= 1; o >>= 1) c += __shfl_xor(c, o);
   if ((threadIdx.x & 63) == 0) sc[threadIdx.x >> 6] = c;
   __syncthreads();
-  if (threadIdx.x == 0) count[blockIdx.x] = sc[0] + sc[1] + sc[2] + sc[3];
+  if (threadIdx.x == 0) {
+    int n = 0;
+    for (int w = 0; w < kWalkThreads / 64; ++w) n += sc[w];
+    count[blockIdx.x] = n;
+  }
 }
 
 // Final group f takes the kept points of staged group src[f] in staged
 // order into [pt_off, pt_off + n), then pads to npts_pad with copies of its
-// first point of zero weight (the host layout).
+// first point of zero weight (the host layout).  One block walks the group in
+// steps of kWalkThreads points, bound by the latency of each step's loads and
+// barrier, so the steps are few and long, the next step's points are loaded
+// before this one's ranks are known, and the waves' counts alternate between
+// two rows so that one barrier a step is enough: 77 -> 33 us for 25 atoms,
+// 155 -> 62 us for 110 against 256 threads and a step's loads after its
+// ranks (k_group_count, likewise, 30 -> 11 and 50 -> 16 us).
 struct CompactItem {
   int src, pt_off, n, npts_pad;
 };
-__global__ __launch_bounds__(256) void k_compact(const CompactItem* __restrict__ items,
-                                                 const StGroup* __restrict__ groups,
-                                                 const double* __restrict__ sx,
-                                                 const double* __restrict__ sy,
-                                                 const double* __restrict__ sz,
-                                                 const double* __restrict__ sw, int drop_zero,
-                                                 double* __restrict__ px, double* __restrict__ py,
-                                                 double* __restrict__ pz, double* __restrict__ pw) {
-  __shared__ int swave[4];
+__global__ __launch_bounds__(kWalkThreads) void k_compact(
+    const CompactItem* __restrict__ items, const StGroup* __restrict__ groups,
+    const double* __restrict__ sx, const double* __restrict__ sy,
+    const double* __restrict__ sz, const double* __restrict__ sw, int drop_zero,
+    double* __restrict__ px, double* __restrict__ py, double* __restrict__ pz,
+    double* __restrict__ pw) {
+  constexpr int NW = kWalkThreads / 64;
+  __shared__ int swave[2][NW];
   __shared__ int sfirst;
   const CompactItem it = items[blockIdx.x];
   const StGroup G = groups[it.src];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  if (threadIdx.x == 0) sfirst = -1;
-  int base = 0;
-  for (int c0 = 0; c0 < G.npts; c0 += 256) {
+  double4 cur = make_double4(0.0, 0.0, 0.0, 0.0), nxt = cur;  // x, y, z, weight
+  auto load = [&](int i, double4& v) {
+    if (i < G.npts) {
+      const int q = G.pt_off + i;
+      v = make_double4(sx[q], sy[q], sz[q], sw[q]);
+    }
+  };
+  load(threadIdx.x, cur);
+  int base = 0, row = 0;
+  for (int c0 = 0; c0 < G.npts; c0 += kWalkThreads, row ^= 1) {
     const int i = c0 + threadIdx.x;
-    const bool keep = i < G.npts && (!drop_zero || sw[G.pt_off + i] != 0.0);
+    load(i + kWalkThreads, nxt);
+    const bool keep = i < G.npts && (!drop_zero || cur.w != 0.0);
     const unsigned long long mask = __ballot(keep);
     const int rank = __popcll(mask & ((1ull << lane) - 1ull));
-    if (lane == 0) swave[wave] = __popcll(mask);
+    if (lane == 0) swave[row][wave] = __popcll(mask);
     __syncthreads();
-    int before = base;
-    for (int w = 0; w < wave; ++w) before += swave[w];
+    int before = base, all = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const int n = swave[row][w];
+      before += w < wave ? n : 0;
+      all += n;
+    }
     if (keep) {
       const int q = it.pt_off + before + rank;
-      px[q] = sx[G.pt_off + i];
-      py[q] = sy[G.pt_off + i];
-      pz[q] = sz[G.pt_off + i];
-      pw[q] = sw[G.pt_off + i];
+      px[q] = cur.x;
+      py[q] = cur.y;
+      pz[q] = cur.z;
+      pw[q] = cur.w;
       if (before + rank == 0) sfirst = i;
     }
-    base += swave[0] + swave[1] + swave[2] + swave[3];
-    __syncthreads();
+    base += all;
+    cur = nxt;
   }
+  __syncthreads();
+  if (it.n == it.npts_pad) return;
   const int f = sfirst;
-  for (int q = it.n + threadIdx.x; q < it.npts_pad; q += 256) {
+  for (int q = it.n + threadIdx.x; q < it.npts_pad; q += kWalkThreads) {
     px[it.pt_off + q] = sx[G.pt_off + f];
     py[it.pt_off + q] = sy[G.pt_off + f];
     pz[it.pt_off + q] = sz[G.pt_off + f];
@@ -5012,8 +5090,8 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
     XCQ_HIP(hipMallocAsync((void**)&dci, std::max<size_t>(1, G) * sizeof(CompactItem), s));
     up(dci, ci.data(), ci.size() * sizeof(CompactItem));
     if (G > 0)
-      hipLaunchKernelGGL(k_compact, dim3(G), dim3(256), 0, s, dci, dpts->groups, dpts->x, dpts->y,
-                         dpts->z, dpts->w, dpts->drop_zero, dg->px, dg->py, dg->pz, dg->pw);
+      hipLaunchKernelGGL(k_compact, dim3(G), dim3(kWalkThreads), 0, s, dci, dpts->groups,
+                         dpts->x, dpts->y, dpts->z, dpts->w, dpts->drop_zero, dg->px, dg->py, dg->pz, dg->pw);
     XCQ_HIP(hipGetLastError());
     XCQ_HIP(hipFreeAsync(dci, s));
   }
@@ -5179,10 +5257,11 @@ std::vector<GridPartition> Engine::weigh_and_load(const std::vector<const Molecu
   }
   if (nsq > (1LL << 31) - 256) throw std::runtime_error("g2g: Becke tables too large");
   const size_t nat = h.gatoms.size() + 1;
-  double *td, *tw, *ox, *oy, *oz;
+  double *td, *tr, *tw, *ox, *oy, *oz;
   int* gpos;
   auto carve_becke = [&](Carver& c) {
     td = c.take<double>((size_t)nsq + 1);
+    tr = c.take<double>((size_t)nsq + 1);
     tw = c.take<double>((size_t)nsq + 1);
     ox = c.take<double>(nat);
     oy = c.take<double>(nat);
@@ -5211,18 +5290,19 @@ std::vector<GridPartition> Engine::weigh_and_load(const std::vector<const Molecu
   if (nst > 0)
     hipLaunchKernelGGL(k_becke_order, dim3(nst), dim3(256), 0, s, d.groups, d.mols, d.gatoms,
                        d.ax, d.ay, d.az, d.aw, d.rij, d.x, d.y, d.z, d.gord, gpos, ox, oy, oz,
-                       td, tw);
+                       td, tr, tw);
   if (!h.bitems.empty()) {
     hipLaunchKernelGGL(k_becke_exact, dim3((unsigned)h.bitems.size()), dim3(kBeckePts), 0, s,
                        d.groups, d.bitems, d.mols, d.gatoms, d.owner, d.ax, d.ay, d.az, d.aw,
                        d.rij, d.x, d.y, d.z, d.bterm, d.bnuc);
     hipLaunchKernelGGL(k_becke, dim3((unsigned)h.bitems.size()), dim3(kBeckePts * kBeckeLanes), 0,
-                       s, d.groups, d.bitems, d.mols, d.gatoms, gpos, ox, oy, oz, td, tw, d.ax,
-                       d.ay, d.az, d.aw, d.rij, d.x, d.y, d.z, d.bterm, d.bnuc, d.w);
+                       s, d.groups, d.bitems, gpos, ox, oy, oz, td, tr, tw, d.x, d.y, d.z,
+                       d.bterm, d.bnuc, d.w);
   }
   const int drop = opt.remove_zero_weights ? 1 : 0;
   if (nst > 0)
-    hipLaunchKernelGGL(k_group_count, dim3(nst), dim3(256), 0, s, d.groups, d.w, drop, d.count);
+    hipLaunchKernelGGL(k_group_count, dim3(nst), dim3(kWalkThreads), 0, s, d.groups, d.w, drop,
+                       d.count);
   XCQ_HIP(hipGetLastError());
   std::vector<int> count(nst);
   if (nst > 0) XCQ_HIP(hipMemcpyAsync(count.data(), d.count, nst * sizeof(int),

@@ -4263,6 +4263,73 @@ struct Carver {
 
 }  // namespace
 
+// Host tables on their way to the device, copied by flush() in the order they
+// were named.  Those of at most kMax bytes go through the engine's pinned
+// buffer, and tables that lie behind one another on the device (nothing but
+// the alignment's padding between them) cross in one copy: a copy from
+// pageable memory costs the host 3 to 10 us however small it is, and a grid
+// load has some fifty (the load's own part 0.30 -> 0.02 ms for 25 atoms, 0.09
+// -> 0.03 ms for 60).  Larger tables are copied from where they are, which
+// keeps the pinned buffer small; with the line at 256 KiB a copy of either
+// kind waited for one of the other (0.22 ms for 96 atoms against 0.03).  The
+// sources stay as they are until flush(); the pinned buffer is written again
+// only once its last copies are done.
+class Uploads {
+ public:
+  explicit Uploads(Engine& e) : e_(e) {}
+  void operator()(void* dst, const void* src, size_t bytes) {
+    if (!bytes) return;
+    char* d = static_cast<char*>(dst);
+    if (bytes > kMax) {
+      runs_.push_back({d, 0, bytes, src});
+      return;
+    }
+    if (!runs_.empty() && !runs_.back().direct) {
+      Run& r = runs_.back();
+      if (d >= r.dst + r.bytes && d < r.dst + r.bytes + 256) {
+        const size_t off = r.off + (size_t)(d - r.dst);
+        parts_.push_back({off, src, bytes});
+        r.bytes = (size_t)(d - r.dst) + bytes;
+        used_ = off + bytes;
+        return;
+      }
+    }
+    const size_t off = (used_ + 255) & ~size_t(255);
+    runs_.push_back({d, off, bytes, nullptr});
+    parts_.push_back({off, src, bytes});
+    used_ = off + bytes;
+  }
+  void flush() {
+    char* pin = used_ ? e_.upload_buffer(used_) : nullptr;
+    for (const Part& q : parts_) std::memcpy(pin + q.off, q.src, q.bytes);
+    hipStream_t s = (hipStream_t)e_.stream();
+    for (const Run& r : runs_)
+      XCQ_HIP(hipMemcpyAsync(r.dst, r.direct ? r.direct : pin + r.off, r.bytes,
+                             hipMemcpyHostToDevice, s));
+    if (used_) e_.upload_queued();
+    runs_.clear();
+    parts_.clear();
+    used_ = 0;
+  }
+
+ private:
+  static constexpr size_t kMax = size_t(1) << 20;
+  struct Run {
+    char* dst;
+    size_t off, bytes;
+    const void* direct;
+  };
+  struct Part {
+    size_t off;
+    const void* src;
+    size_t bytes;
+  };
+  Engine& e_;
+  std::vector<Run> runs_;
+  std::vector<Part> parts_;
+  size_t used_ = 0;
+};
+
 Engine::Engine(int device) {
   int n = 0;
   XCQ_HIP(hipGetDeviceCount(&n));
@@ -4282,6 +4349,28 @@ Engine::Engine(int device) {
     XCQ_HIP(hipEventCreate(&ev));
     e = ev;
   }
+  hipEvent_t up;
+  XCQ_HIP(hipEventCreateWithFlags(&up, hipEventDisableTiming));
+  upload_done_ = up;
+}
+
+// The pinned buffer of small uploads, at least `bytes` (grow-only: it holds
+// tables of at most a MiB each), after the copies last queued from it.
+char* Engine::upload_buffer(size_t bytes) {
+  XCQ_HIP(hipEventSynchronize((hipEvent_t)upload_done_));
+  if (upload_cap_ < bytes) {
+    if (upload_) XCQ_HIP(hipHostFree(upload_));
+    upload_ = nullptr;
+    upload_cap_ = 0;
+    const size_t want = (bytes + bytes / 4 + 4095) & ~size_t(4095);
+    XCQ_HIP(hipHostMalloc(&upload_, want, hipHostMallocDefault));
+    upload_cap_ = want;
+  }
+  return static_cast<char*>(upload_);
+}
+
+void Engine::upload_queued() {
+  XCQ_HIP(hipEventRecord((hipEvent_t)upload_done_, (hipStream_t)stream_));
 }
 
 // Device memory comes from the device's stream-ordered pool (hipMallocAsync /
@@ -4405,6 +4494,8 @@ Engine::~Engine() {
   if (stream_) (void)hipStreamSynchronize((hipStream_t)stream_);
   for (auto& e : events_)
     if (e) (void)hipEventDestroy((hipEvent_t)e);
+  if (upload_done_) (void)hipEventDestroy((hipEvent_t)upload_done_);
+  if (upload_) (void)hipHostFree(upload_);
   if (stream_) (void)hipStreamDestroy((hipStream_t)stream_);
 }
 
@@ -4870,22 +4961,52 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
   std::vector<int> membf(memb.size());
   for (size_t k = 0; k < memb.size(); ++k) membf[k] = groups[memb[k].x].fn_off + memb[k].y;
 
+  CompactItem* compact = nullptr;
   auto plan = [&](Carver& c) {
+    // the host's tables first and in upload order, so that they cross in one copy
     dg->bas = c.take<DevFn>(M);
     dg->groups = c.take<DevGroup>(G);
     dg->eitems = c.take<EvalItem>(eitems.size());
     dg->gitems = c.take<GatherItem>(gitems.size());
     dg->tfirst = c.take<int>(tfirst.size());
     dg->torder = c.take<int>(order.size());
-    dg->phiT = c.take<float>(fo);
     dg->ditems = c.take<DensityItem>(ditems.size());
     dg->fitems = c.take<FockItem>(fitems.size());
     dg->gtiles = c.take<int2>(gtiles.size());
     dg->fnl = c.take<int>(fnl.size());
+    dg->memb_off = c.take<int>(M + 1);
+    dg->memb = c.take<int2>(memb.size() + 1);
+    dg->membf = c.take<int>(memb.size() + 1);
+    dg->mols = c.take<DevMol>(nmol);
+    dg->fn_mol = c.take<int>(M);
+    dg->eidx = c.take<int>(eidx.size() + 1);
+    dg->citems = c.take<DensityItem>(citems.size());
+    dg->shells = c.take<int>(shells.size() + 1);
+    dg->fmeta = c.take<FnMeta>(fmeta.size() + 1);
+    dg->ritems = c.take<GatherItem>(ritems.size());
+    dg->tsh = c.take<int2>(tsh.size() + 1);
+    dg->kbsh = c.take<int2>(kbsh.size() + 1);
+    dg->sfn = c.take<int2>(sfn.size() + 1);
+    dg->afn_off = c.take<int>(afn_off.size());
+    dg->afn = c.take<int>(afn.size());
+    dg->chitems = c.take<ChunkItem>(chitems.size());
+    dg->finitems = c.take<ChunkItem>(finitems.size());
+    dg->forder = c.take<int>(forder.size());
+    compact = c.take<CompactItem>(dpts ? G : 0);
+    PersistArgs& pa = dg->pargs;
+    dg->dpargs = c.take<PersistArgs>(1);
+    pa.gneed = c.take<int>(gneed.size() + 1);
+    pa.dneed = c.take<int>(dneed.size() + 1);
+    pa.tbase = c.take<int>(tbase.size() + 1);
+    pa.fperm = c.take<int>(fperm.size() + 1);
+    pa.tperm = c.take<int>(tperm.size() + 1);
+    pa.pitems = c.take<int2>(pitems.size() + 1);
     dg->px = c.take<double>(pt);
     dg->py = c.take<double>(pt);
     dg->pz = c.take<double>(pt);
     dg->pw = c.take<double>(pt);
+    pa.sync = c.take<int>(dg->nsync + 1);
+    dg->phiT = c.take<float>(fo);
     dg->rho = c.take<double>(nspin * packed);
     dg->F = c.take<double>(nspin * packed);
     dg->vals = c.take<char>(vo * vbytes);
@@ -4894,44 +5015,17 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
     dg->factor = c.take<double>(pt);
     dg->epart = c.take<double>(2 * ditems.size());
     dg->fpart = c.take<double>((size_t)fitems.size() * kFnChunk * kFnChunk);
-    dg->memb_off = c.take<int>(M + 1);
-    dg->memb = c.take<int2>(memb.size() + 1);
-    dg->mols = c.take<DevMol>(nmol);
-    dg->fn_mol = c.take<int>(M);
-    dg->eidx = c.take<int>(eidx.size() + 1);
     dg->eout = c.take<double>(2 * nmol);
-    dg->citems = c.take<DensityItem>(citems.size());
     dg->gpart = c.take<double>(go);
     dg->gsum = c.take<double>(3 * fnl.size());
-    dg->membf = c.take<int>(memb.size() + 1);
-    dg->afn_off = c.take<int>(afn_off.size());
-    dg->afn = c.take<int>(afn.size());
     dg->fout = c.take<double>(3 * (size_t)dg->natom);
     dg->pg2 = c.take<char>(dg->open ? po * pbytes : 0);
     dg->factor_b = c.take<double>(dg->open ? pt : 0);
     dg->sums = c.take<double>(dg->open ? 10 * pt : 0);
-    dg->shells = c.take<int>(shells.size() + 1);
-    dg->fmeta = c.take<FnMeta>(fmeta.size() + 1);
     dg->rad = c.take<float>(ro);
-    dg->ritems = c.take<GatherItem>(ritems.size());
-    dg->tsh = c.take<int2>(tsh.size() + 1);
-    dg->kbsh = c.take<int2>(kbsh.size() + 1);
-    dg->sfn = c.take<int2>(sfn.size() + 1);
     dg->lo16 = c.take<unsigned short>(dg->lo ? fo : 0);
-    dg->chitems = c.take<ChunkItem>(chitems.size());
     dg->pcs = c.take<unsigned short>(dg->presplit ? 4 * fo : 0);
     dg->cpart = c.take<double>((size_t)npart * 10 * kDensPts);
-    dg->finitems = c.take<ChunkItem>(finitems.size());
-    dg->forder = c.take<int>(forder.size());
-    PersistArgs& pa = dg->pargs;
-    dg->dpargs = c.take<PersistArgs>(1);
-    pa.sync = c.take<int>(dg->nsync + 1);
-    pa.gneed = c.take<int>(gneed.size() + 1);
-    pa.dneed = c.take<int>(dneed.size() + 1);
-    pa.tbase = c.take<int>(tbase.size() + 1);
-    pa.fperm = c.take<int>(fperm.size() + 1);
-    pa.tperm = c.take<int>(tperm.size() + 1);
-    pa.pitems = c.take<int2>(pitems.size() + 1);
   };
   Carver sizing{nullptr};
   plan(sizing);
@@ -4999,9 +5093,7 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
   }
 
   hipStream_t s = (hipStream_t)stream_;
-  auto up = [&](void* dst, const void* src, size_t bytes) {
-    if (bytes) XCQ_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s));
-  };
+  Uploads up(*this);
   up(dg->bas, bas.data(), bas.size() * sizeof(DevFn));
   up(dg->groups, groups.data(), groups.size() * sizeof(DevGroup));
   up(dg->eitems, eitems.data(), eitems.size() * sizeof(EvalItem));
@@ -5012,10 +5104,6 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
   up(dg->fitems, fitems.data(), fitems.size() * sizeof(FockItem));
   up(dg->gtiles, gtiles.data(), gtiles.size() * sizeof(int2));
   up(dg->fnl, fnl.data(), fnl.size() * sizeof(int));
-  up(dg->px, hx.data(), hx.size() * sizeof(double));
-  up(dg->py, hy.data(), hy.size() * sizeof(double));
-  up(dg->pz, hz.data(), hz.size() * sizeof(double));
-  up(dg->pw, hw.data(), hw.size() * sizeof(double));
   up(dg->memb_off, moff.data(), moff.size() * sizeof(int));
   up(dg->memb, memb.data(), memb.size() * sizeof(int2));
   up(dg->membf, membf.data(), membf.size() * sizeof(int));
@@ -5034,6 +5122,14 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
   up(dg->chitems, chitems.data(), chitems.size() * sizeof(ChunkItem));
   up(dg->finitems, finitems.data(), finitems.size() * sizeof(ChunkItem));
   up(dg->forder, forder.data(), forder.size() * sizeof(int));
+  std::vector<CompactItem> ci;
+  if (dpts) {  // points come from the device rebuild: compacted into place below
+    if ((int)dpts->src.size() != G) throw std::runtime_error("g2g: staged group map mismatch");
+    ci.resize(G);
+    for (int g = 0; g < G; ++g)
+      ci[g] = CompactItem{dpts->src[g], groups[g].pt_off, groups[g].npts, groups[g].npts_pad};
+    up(compact, ci.data(), ci.size() * sizeof(CompactItem));
+  }
   if (dg->persistent) {
     PersistArgs& pa = dg->pargs;
     up(const_cast<int*>(pa.gneed), gneed.data(), gneed.size() * sizeof(int));
@@ -5081,19 +5177,16 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
     pa.eout = dg->eout;
     up(dg->dpargs, &pa, sizeof(PersistArgs));
   }
-  if (dpts) {  // points come from the device rebuild: compact them into place
-    if ((int)dpts->src.size() != G) throw std::runtime_error("g2g: staged group map mismatch");
-    std::vector<CompactItem> ci(G);
-    for (int g = 0; g < G; ++g)
-      ci[g] = CompactItem{dpts->src[g], groups[g].pt_off, groups[g].npts, groups[g].npts_pad};
-    CompactItem* dci = nullptr;
-    XCQ_HIP(hipMallocAsync((void**)&dci, std::max<size_t>(1, G) * sizeof(CompactItem), s));
-    up(dci, ci.data(), ci.size() * sizeof(CompactItem));
-    if (G > 0)
-      hipLaunchKernelGGL(k_compact, dim3(G), dim3(kWalkThreads), 0, s, dci, dpts->groups,
-                         dpts->x, dpts->y, dpts->z, dpts->w, dpts->drop_zero, dg->px, dg->py, dg->pz, dg->pw);
+  up(dg->px, hx.data(), hx.size() * sizeof(double));
+  up(dg->py, hy.data(), hy.size() * sizeof(double));
+  up(dg->pz, hz.data(), hz.size() * sizeof(double));
+  up(dg->pw, hw.data(), hw.size() * sizeof(double));
+  up.flush();
+  if (dpts && G > 0) {
+    hipLaunchKernelGGL(k_compact, dim3(G), dim3(kWalkThreads), 0, s, compact, dpts->groups,
+                       dpts->x, dpts->y, dpts->z, dpts->w, dpts->drop_zero, dg->px, dg->py,
+                       dg->pz, dg->pw);
     XCQ_HIP(hipGetLastError());
-    XCQ_HIP(hipFreeAsync(dci, s));
   }
   // basis values of every group, kept for all solves on this grid
   hipEvent_t* ev = reinterpret_cast<hipEvent_t*>(events_);
@@ -5187,18 +5280,19 @@ void stage_atoms(const Molecule& mol, const std::vector<double>& rij, StageHost&
 
 // Carves the tables of h and n_points staged points.
 void carve_stage(Carver& c, const StageHost& h, long long n_points, StageDev& d) {
+  // the host's tables in upload order, those of exact size first
+  d.ax = c.take<double>(h.ax.size());
+  d.ay = c.take<double>(h.ay.size());
+  d.az = c.take<double>(h.az.size());
+  d.aw = c.take<double>(h.aw.size());
+  d.rij = c.take<double>(h.rij.size());
+  d.mols = c.take<StMol>(h.sm.size());
   d.groups = c.take<StGroup>(h.sg.size() + 1);
-  d.mols = c.take<StMol>(h.sm.size() + 1);
   d.bitems = c.take<int2>(h.bitems.size() + 1);
-  d.owner = c.take<int>(n_points + 1);
   d.gatoms = c.take<int>(h.gatoms.size() + 1);
+  d.owner = c.take<int>(n_points + 1);
   d.gord = c.take<int>(h.gatoms.size() + 1);
   d.count = c.take<int>(h.sg.size() + 1);
-  d.ax = c.take<double>(h.ax.size() + 1);
-  d.ay = c.take<double>(h.ay.size() + 1);
-  d.az = c.take<double>(h.az.size() + 1);
-  d.aw = c.take<double>(h.aw.size() + 1);
-  d.rij = c.take<double>(h.rij.size() + 1);
   d.x = c.take<double>(n_points + 1);
   d.y = c.take<double>(n_points + 1);
   d.z = c.take<double>(n_points + 1);
@@ -5244,9 +5338,7 @@ std::vector<GridPartition> Engine::weigh_and_load(const std::vector<const Molecu
   const int nmol = (int)mols.size();
   const int nst = (int)h.sg.size();
   hipStream_t s = (hipStream_t)stream_;
-  auto up = [&](void* dst, const void* src, size_t bytes) {
-    if (bytes) XCQ_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s));
-  };
+  Uploads up(*this);
   // each group's natoms x natoms Becke tables in near-first order, in their
   // own grow-only buffer (sized now that the groups are known)
   std::vector<StGroup> sg = h.sg;
@@ -5272,21 +5364,22 @@ std::vector<GridPartition> Engine::weigh_and_load(const std::vector<const Molecu
   carve_becke(bsize);
   Carver bc{becke_buffer(bsize.used)};
   carve_becke(bc);
-  up(d.groups, sg.data(), sg.size() * sizeof(StGroup));
-  up(d.mols, h.sm.data(), h.sm.size() * sizeof(StMol));
   // the Becke blocks heaviest first (cost ~ natoms^2), so that the longest
   // ones do not start last
   std::vector<int2> bitems = h.bitems;
   std::stable_sort(bitems.begin(), bitems.end(), [&](const int2& a, const int2& b) {
     return h.sg[a.x].natoms > h.sg[b.x].natoms;
   });
-  up(d.bitems, bitems.data(), bitems.size() * sizeof(int2));
-  up(d.gatoms, h.gatoms.data(), h.gatoms.size() * sizeof(int));
   up(d.ax, h.ax.data(), h.ax.size() * sizeof(double));
   up(d.ay, h.ay.data(), h.ay.size() * sizeof(double));
   up(d.az, h.az.data(), h.az.size() * sizeof(double));
   up(d.aw, h.aw.data(), h.aw.size() * sizeof(double));
   up(d.rij, h.rij.data(), h.rij.size() * sizeof(double));
+  up(d.mols, h.sm.data(), h.sm.size() * sizeof(StMol));
+  up(d.groups, sg.data(), sg.size() * sizeof(StGroup));
+  up(d.bitems, bitems.data(), bitems.size() * sizeof(int2));
+  up(d.gatoms, h.gatoms.data(), h.gatoms.size() * sizeof(int));
+  up.flush();
   if (nst > 0)
     hipLaunchKernelGGL(k_becke_order, dim3(nst), dim3(256), 0, s, d.groups, d.mols, d.gatoms,
                        d.ax, d.ay, d.az, d.aw, d.rij, d.x, d.y, d.z, d.gord, gpos, ox, oy, oz,
@@ -5524,14 +5617,14 @@ std::vector<GridPartition> Engine::load_generated(const std::vector<const Molecu
     g.ez = c.take<double>(ez.size());
     g.ew = c.take<double>(ew.size());
     g.srad = c.take<double>(srad.size());
-    g.sh_a = c.take<double>(sh_a.size() + 1);
-    g.sh_thr = c.take<double>(sh_thr.size() + 1);
-    g.sh_first = c.take<int>(sh_first.size() + 1);
-    g.sh_len = c.take<int>(sh_len.size() + 1);
-    g.sh_atom = c.take<int>(sh_atom.size() + 1);
+    g.sh_a = c.take<double>(sh_a.size());
+    g.sh_thr = c.take<double>(sh_thr.size());
+    g.sh_first = c.take<int>(sh_first.size());
+    g.sh_len = c.take<int>(sh_len.size());
+    g.sh_atom = c.take<int>(sh_atom.size());
     g.bin_mol = c.take<int>(nbins);
-    g.count = c.take<int>(2 * nbins);
-    g.err = c.take<int>(1);
+    g.count = c.take<int>(2 * nbins + 1);
+    g.err = g.count + 2 * nbins;
     g.slots = c.take<int>(nslot + 1);
     g.aslots = c.take<int>(naslot + 1);
     g.pk = c.take<int>(nslot + 1);
@@ -5550,9 +5643,7 @@ std::vector<GridPartition> Engine::load_generated(const std::vector<const Molecu
   Carver c{stage_buffer(plan.used)};
   carve(c);
   hipStream_t s = (hipStream_t)stream_;
-  auto up = [&](void* dst, const void* src, size_t bytes) {
-    if (bytes) XCQ_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s));
-  };
+  Uploads up(*this);
   up(g.atoms, gatom.data(), gatom.size() * sizeof(GenAtom));
   up(g.mols, gmol.data(), gmol.size() * sizeof(GenMol));
   up(g.r1, r1.data(), r1.size() * sizeof(double));
@@ -5568,10 +5659,11 @@ std::vector<GridPartition> Engine::load_generated(const std::vector<const Molecu
   up(g.sh_len, sh_len.data(), sh_len.size() * sizeof(int));
   up(g.sh_atom, sh_atom.data(), sh_atom.size() * sizeof(int));
   up(g.bin_mol, bin_mol.data(), bin_mol.size() * sizeof(int));
+  up(d.rij, h.rij.data(), h.rij.size() * sizeof(double));
+  up.flush();
   // run bounds and the error flag start at zero (a fill kernel, no memset)
-  hipLaunchKernelGGL(k_fill_int, dim3((2 * nbins + 255) / 256), dim3(256), 0, s, g.count,
-                     2 * nbins, 0);
-  hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(256), 0, s, g.err, 1, 0);
+  hipLaunchKernelGGL(k_fill_int, dim3((2 * nbins + 256) / 256), dim3(256), 0, s, g.count,
+                     2 * nbins + 1, 0);
   const int natoms = (int)gatom.size();
   if (nraw > 0)
     hipLaunchKernelGGL(k_gen_keys, dim3((unsigned)((nraw + 255) / 256)), dim3(256), 0, s,
@@ -5583,20 +5675,17 @@ std::vector<GridPartition> Engine::load_generated(const std::vector<const Molecu
   if (nraw > 0)
     hipLaunchKernelGGL(k_gen_bounds, dim3((unsigned)((nraw + 255) / 256)), dim3(256), 0, s,
                        g.skeys, nraw, (unsigned)nbins, g.count);
-  up(d.rij, h.rij.data(), h.rij.size() * sizeof(double));
   hipLaunchKernelGGL(k_gen_screen, dim3(nbins), dim3(256), 0, s, g.mols, g.bin_mol, g.atoms,
                      g.srad, d.rij, g.sh_first, g.sh_len, g.sh_atom, g.sh_a, g.sh_thr,
                      opt.assign_all_functions ? 1 : 0, g.slots, g.aslots, g.info);
   XCQ_HIP(hipGetLastError());
-  std::vector<int> count(2 * nbins);
+  std::vector<int> count(2 * nbins + 1);
   std::vector<BinInfo> info(nbins);
-  int err = 0;
-  XCQ_HIP(hipMemcpyAsync(count.data(), g.count, 2 * nbins * sizeof(int), hipMemcpyDeviceToHost,
-                         s));
+  XCQ_HIP(hipMemcpyAsync(count.data(), g.count, count.size() * sizeof(int),
+                         hipMemcpyDeviceToHost, s));
   XCQ_HIP(hipMemcpyAsync(info.data(), g.info, nbins * sizeof(BinInfo), hipMemcpyDeviceToHost, s));
-  XCQ_HIP(hipMemcpyAsync(&err, g.err, sizeof(int), hipMemcpyDeviceToHost, s));
   XCQ_HIP(hipStreamSynchronize(s));
-  if (err) throw std::runtime_error("grid point outside the cube lattice of the bounding prism");
+  if (count[2 * nbins]) throw std::runtime_error("grid point outside the cube lattice of the bounding prism");
   for (int b = 0; b < nbins; ++b) count[b] = count[nbins + b] - count[b];
   // the staged groups, as the host keeps them: cubes with significant
   // functions and enough points, in lattice order, then the spheres
@@ -5620,6 +5709,7 @@ std::vector<GridPartition> Engine::load_generated(const std::vector<const Molecu
   std::vector<int> pk(soff), pa(aoff);
   if (!items.empty()) {
     up(g.pitems, items.data(), items.size() * sizeof(PackItem));
+    up.flush();
     hipLaunchKernelGGL(k_gen_pack, dim3((unsigned)items.size()), dim3(256), 0, s, g.pitems,
                        g.mols, g.bin_mol, g.slots, g.aslots, g.pk, g.pa);
     XCQ_HIP(hipGetLastError());

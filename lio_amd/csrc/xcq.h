@@ -345,6 +345,8 @@ class Engine {
     for (int k = 0; k < 4; ++k) ms[k] = load_ms_[k];
   }
   void* stream() const { return stream_; }
+  char* upload_buffer(size_t bytes);
+  void upload_queued();
   const DeviceGrid* grid() const { return grid_; }
 
  private:
@@ -355,6 +357,9 @@ class Engine {
   void* graph_ = nullptr;
   void* stage_ = nullptr;     // device grid rebuild staging (kept, grow-only)
   size_t stage_cap_ = 0;
+  void* upload_ = nullptr;    // pinned, small host tables (kept, grow-only)
+  size_t upload_cap_ = 0;
+  void* upload_done_ = nullptr;  // after the copies last queued from it
   void* becke_ = nullptr;     // Becke tables in near-first order (kept, grow-only)
   size_t becke_cap_ = 0;
   double load_ms_[4] = {};

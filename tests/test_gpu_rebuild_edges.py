@@ -44,3 +44,35 @@ def test_device_weights_equal_the_hosts(natoms, drop):
             assert a[key] == b[key]
         for key in ("wsum", "xsum"):
             assert np.array_equal(a[key], b[key], equal_nan=True)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "bf16x6"])
+def test_reloads_of_changing_size_equal_a_fresh_one(precision):
+    """One engine takes systems of growing and shrinking size in turn, with
+    the host's and the device's grids, so that its kept buffer of pinned host
+    tables grows, is written again while larger than needed, and is passed by
+    for tables too large for it (the 30-atom host grid's points): each solve
+    equals that of an engine that held nothing before, bit for bit."""
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from lio_amd import g2g, systems
+    made = {}
+    for n in (2, 8, 30):
+        Z, pos = systems.random_molecule_ang(n, 70 + n)
+        made[n] = systems.make_system("reload%d" % n, Z, pos, seed=n)
+    kept = g2g.Context(made[2], precision=precision)
+    for n, mode in [(2, "device"), (30, "device"), (8, "host"), (30, "host"), (2, "host"),
+                    (8, "device"), (30, "device")]:
+        print("atoms", n, mode, flush=True)
+        kept.set_grid_mode(mode)
+        kept.set_system(made[n])
+        kept.build_grid()
+        kept.build_grid()  # the tables are written again at once
+        fresh = g2g.Context(made[n], precision=precision, grid_mode=mode)
+        fresh.build_grid()
+        E0, F0, _ = fresh.solve()
+        E1, F1, _ = kept.solve()
+        assert E0 == E1 and np.array_equal(F0, F1)
+        fresh.close()
+    kept.close()

@@ -204,8 +204,10 @@ int xcq_batch_solve_forces(xcq_batch* b, const double* d_rho, double* d_fock, do
  * the reference: it is for callers that cannot allocate device memory during
  * the call (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc).  xcq_batch_solve_forces allocates, at its first call on a
- * split-BF16 grid, a buffer for Y = P_g phi of the force pass; this entry
- * point takes Y from a static device array of the library instead
+ * grid, a buffer for Y = P_g phi of the force pass (FP64 and FP32: only where
+ * it takes at most an eighth of the obtainable memory; the force pass forms Y
+ * again otherwise, with the same results).  This entry point forms Y again in
+ * FP64 and FP32, and in split-BF16 takes it from a static device array
  * (xcq_static_scratch_bytes(), 64 MiB, held by each device the library runs
  * on until the process ends) and fails with an error when the batch needs
  * more.  Every call on one device shares that array: calls that overlap on

@@ -58,7 +58,7 @@ namespace {
 
 constexpr int kPtAlign = 16;     // point padding (one MFMA column tile)
 constexpr int kFnAlign = 16;     // function padding (one MFMA row tile)
-constexpr int kDensPts = 64;     // points per k_density block (16 per wave)
+constexpr int kDensPts = 64;     // points per density block (16 per wave)
 constexpr int kRowSplitMin = 64; // split-BF16 row-split density above this m_pad
 constexpr int kFnChunk = 64;     // functions per density pass / Fock tile side
 constexpr int kXcds = 8;         // MI355X: XCDs, each with its own L2 (block b runs on b % 8)
@@ -987,7 +987,7 @@ __global__ __launch_bounds__(256) void k_gather_density_bf(const DevGroup* __res
     gather_bf_item<NPC, FRAG>(GatherItem{(int)blockIdx.x, e0}, groups, mols, fnl, rho, pgs);
 }
 
-// Density + functional on split-BF16 MFMA: same blocking as k_density (64
+// Density + functional on split-BF16 MFMA: blocks of a whole tile (64
 // points per block, 16 per wave, 64-function row chunks) with K steps of 32
 // functions.  The B operand of a lane is 8 consecutive functions of its point
 // (32 contiguous bytes of the point-major planes), split in registers; the A
@@ -4269,9 +4269,12 @@ struct Carver {
 // the alignment's padding between them) cross in one copy: a copy from
 // pageable memory costs the host 3 to 10 us however small it is, and a grid
 // load has some fifty (the load's own part 0.30 -> 0.02 ms for 25 atoms, 0.09
-// -> 0.03 ms for 60).  Larger tables are copied from where they are, which
-// keeps the pinned buffer small; with the line at 256 KiB a copy of either
-// kind waited for one of the other (0.22 ms for 96 atoms against 0.03).  The
+// -> 0.03 ms for 60).  Larger tables, and those that no longer fit, are copied
+// from where they are, which keeps the pinned buffer small; with the line at
+// 256 KiB a copy of either kind waited for one of the other (0.22 ms for 96
+// atoms against 0.03).  The buffer is made with the engine and never grows:
+// giving pinned memory back waits for every stream of the device (a buffer
+// that grew took 4 ms of a load with eight others running).  The
 // sources stay as they are until flush(); the pinned buffer is written again
 // only once its last copies are done.
 class Uploads {
@@ -4280,27 +4283,22 @@ class Uploads {
   void operator()(void* dst, const void* src, size_t bytes) {
     if (!bytes) return;
     char* d = static_cast<char*>(dst);
-    if (bytes > kMax) {
+    Run* r = runs_.empty() || runs_.back().direct ? nullptr : &runs_.back();
+    if (r && (d < r->dst + r->bytes || d >= r->dst + r->bytes + 256)) r = nullptr;
+    const size_t off = r ? r->off + (size_t)(d - r->dst) : (used_ + 255) & ~size_t(255);
+    if (bytes > kMax || off + bytes > Engine::kUploadBytes) {
       runs_.push_back({d, 0, bytes, src});
       return;
     }
-    if (!runs_.empty() && !runs_.back().direct) {
-      Run& r = runs_.back();
-      if (d >= r.dst + r.bytes && d < r.dst + r.bytes + 256) {
-        const size_t off = r.off + (size_t)(d - r.dst);
-        parts_.push_back({off, src, bytes});
-        r.bytes = (size_t)(d - r.dst) + bytes;
-        used_ = off + bytes;
-        return;
-      }
-    }
-    const size_t off = (used_ + 255) & ~size_t(255);
-    runs_.push_back({d, off, bytes, nullptr});
+    if (r)
+      r->bytes = (size_t)(d - r->dst) + bytes;
+    else
+      runs_.push_back({d, off, bytes, nullptr});
     parts_.push_back({off, src, bytes});
     used_ = off + bytes;
   }
   void flush() {
-    char* pin = used_ ? e_.upload_buffer(used_) : nullptr;
+    char* pin = used_ ? e_.upload_buffer() : nullptr;
     for (const Part& q : parts_) std::memcpy(pin + q.off, q.src, q.bytes);
     hipStream_t s = (hipStream_t)e_.stream();
     for (const Run& r : runs_)
@@ -4352,20 +4350,13 @@ Engine::Engine(int device) {
   hipEvent_t up;
   XCQ_HIP(hipEventCreateWithFlags(&up, hipEventDisableTiming));
   upload_done_ = up;
+  XCQ_HIP(hipHostMalloc(&upload_, kUploadBytes, hipHostMallocDefault));
 }
 
-// The pinned buffer of small uploads, at least `bytes` (grow-only: it holds
-// tables of at most a MiB each), after the copies last queued from it.
-char* Engine::upload_buffer(size_t bytes) {
+// The pinned buffer of small uploads (kUploadBytes), after the copies last
+// queued from it.
+char* Engine::upload_buffer() {
   XCQ_HIP(hipEventSynchronize((hipEvent_t)upload_done_));
-  if (upload_cap_ < bytes) {
-    if (upload_) XCQ_HIP(hipHostFree(upload_));
-    upload_ = nullptr;
-    upload_cap_ = 0;
-    const size_t want = (bytes + bytes / 4 + 4095) & ~size_t(4095);
-    XCQ_HIP(hipHostMalloc(&upload_, want, hipHostMallocDefault));
-    upload_cap_ = want;
-  }
   return static_cast<char*>(upload_);
 }
 

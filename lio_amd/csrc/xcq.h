@@ -167,7 +167,8 @@ int radix_sort_pairs(void* temp, size_t* temp_bytes, const unsigned* keys_in,
 //   FP64: FP64 values, FP64 MFMA.
 //   FP32: FP32 values (half the bytes), FP32 MFMA, Fock products summed in
 //         the matrix unit over at most 32 points before FP64 accumulation.
-//   BF16X6: FP32 values stored point-major; every operand is split exactly
+//   BF16X6: FP32 values (tiles of 16 points x 32 functions in variants 10 and
+//         11, point-major in the others); every operand is split exactly
 //         into three BF16 pieces (8 significant bits each) and a tile
 //         product is the six piece products of weight >= 2^-16 relative
 //         (hi*hi, hi*mid, mid*hi, hi*lo, mid*mid, lo*hi) on BF16 MFMA with
@@ -345,7 +346,8 @@ class Engine {
     for (int k = 0; k < 4; ++k) ms[k] = load_ms_[k];
   }
   void* stream() const { return stream_; }
-  char* upload_buffer(size_t bytes);
+  static constexpr size_t kUploadBytes = size_t(4) << 20;
+  char* upload_buffer();
   void upload_queued();
   const DeviceGrid* grid() const { return grid_; }
 
@@ -357,8 +359,7 @@ class Engine {
   void* graph_ = nullptr;
   void* stage_ = nullptr;     // device grid rebuild staging (kept, grow-only)
   size_t stage_cap_ = 0;
-  void* upload_ = nullptr;    // pinned, small host tables (kept, grow-only)
-  size_t upload_cap_ = 0;
+  void* upload_ = nullptr;    // pinned, small host tables (kUploadBytes)
   void* upload_done_ = nullptr;  // after the copies last queued from it
   void* becke_ = nullptr;     // Becke tables in near-first order (kept, grow-only)
   size_t becke_cap_ = 0;

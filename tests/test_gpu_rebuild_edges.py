@@ -49,10 +49,10 @@ def test_device_weights_equal_the_hosts(natoms, drop):
 @pytest.mark.parametrize("precision", ["fp64", "bf16x6"])
 def test_reloads_of_changing_size_equal_a_fresh_one(precision):
     """One engine takes systems of growing and shrinking size in turn, with
-    the host's and the device's grids, so that its kept buffer of pinned host
-    tables grows, is written again while larger than needed, and is passed by
-    for tables too large for it (the 30-atom host grid's points): each solve
-    equals that of an engine that held nothing before, bit for bit."""
+    the host's and the device's grids, so that its pinned buffer of host
+    tables is written again after other sizes and is passed by for tables too
+    large for it (the 30-atom host grid's points): each solve equals that of
+    an engine that held nothing before, bit for bit."""
     torch = pytest.importorskip("torch")
     if not torch.cuda.is_available():
         pytest.skip("no GPU")

@@ -1675,11 +1675,18 @@ __global__ __launch_bounds__(256) void k_density_cs_finish(const ChunkItem* __re
   if (active) {
     const double* ps = cpart + (long long)it.pbase * NS * kDensPts + lane;
     double s[NS];
+    // chunk by chunk, so that a chunk's loads are in flight together: latency
+    // bounds this launch, and sum by sum it waited for every chunk ten times
+    // ((H2O)32 47 -> 35 us, the same sums)
+    double t[NS];
 #pragma unroll
-    for (int k = 0; k < NS; ++k) {
-      double t = ps[k * kDensPts];
-      for (int c = 1; c < it.nch; ++c) t += ps[((long long)c * NS + k) * kDensPts];
-      s[k] = t;
+    for (int k = 0; k < NS; ++k) s[k] = ps[k * kDensPts];
+    for (int c = 1; c < it.nch; ++c) {
+      ps += NS * kDensPts;
+#pragma unroll
+      for (int k = 0; k < NS; ++k) t[k] = ps[k * kDensPts];
+#pragma unroll
+      for (int k = 0; k < NS; ++k) s[k] += t[k];
     }
     point_stage<NT>(s, g.pt_off + it.p0 + lane, iexch, spin, pw, factor, factor_b, sums, sstride,
                     e_w, n_w);

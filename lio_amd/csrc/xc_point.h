@@ -370,10 +370,19 @@ __device__ __host__ __noinline__ void gga_point_other(double rho, const double g
 __device__ __host__ inline void gga_point_x(double rho, const double g[3], const double h1[3],
                                             const double h2[3], int iexch, double& ex,
                                             double& ec, double& y2a) {
-  if (iexch >= 4 && iexch <= 8)
-    gga_point_other(rho, g, h1, h2, iexch, ex, ec, y2a);
-  else
+  if (iexch >= 4 && iexch <= 8) {
+    // copies of its own for the call, which takes addresses: on the device the
+    // caller's values stay in registers on the PBE path
+    const double gc[3] = {g[0], g[1], g[2]}, h1c[3] = {h1[0], h1[1], h1[2]},
+                 h2c[3] = {h2[0], h2[1], h2[2]};
+    double x, c, y;
+    gga_point_other(rho, gc, h1c, h2c, iexch, x, c, y);
+    ex = x;
+    ec = c;
+    y2a = y;
+  } else {
     gga_point(rho, g, h1, h2, ex, ec, y2a);
+  }
 }
 
 // ---------------------------------------------------------------------------

@@ -163,7 +163,8 @@ int xcq_query(xcq_context* ctx);
 int xcq_collect(xcq_context* ctx, double* fock_accum, xcq_solve_info* info);
 /* Waits for the context stream and returns the HIP-event durations (ms) of
  * the last solve's phases: [0] density expansion, [1] density + functional,
- * [2] Fock tiles + slice sums, [3] Fock packing + energy reduction. */
+ * [2] Fock tiles + slice sums, [3] Fock packing + energy reduction; a build
+ * with forces has them in [2] in FP64 and FP32, in [3] in split-BF16. */
 int xcq_kernel_times(xcq_context* ctx, double ms[4]);
 /* HIP stream (hipStream_t) the context launches on. */
 void* xcq_stream(xcq_context* ctx);
@@ -204,18 +205,23 @@ int xcq_batch_solve_forces(xcq_batch* b, const double* d_rho, double* d_fock, do
  * the reference: it is for callers that cannot allocate device memory during
  * the call (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc).  xcq_batch_solve_forces allocates, at its first call on a
- * grid, a buffer for Y = P_g phi of the force pass (FP64 and FP32: only where
- * it takes at most an eighth of the obtainable memory; the force pass forms Y
- * again otherwise, with the same results).  This entry point forms Y again in
- * FP64 and FP32, and in split-BF16 takes it from a static device array
+ * split-BF16 grid, a buffer for Y = P_g phi of the force pass (FP64 and FP32
+ * keep Y where the grid's allocation has room and form it again where it has
+ * not, with the same results); this entry point
+ * takes Y from a static device array of the library instead
  * (xcq_static_scratch_bytes(), 64 MiB, held by each device the library runs
  * on until the process ends) and fails with an error when the batch needs
- * more.  Every call on one device shares that array: calls that overlap on
+ * more (FP64 and FP32 form Y again).  Every call on one device shares that array: calls that overlap on
  * one device (several batches' streams at once) race.  Same results as
  * xcq_batch_solve_forces. */
 int xcq_batch_solve_forces_static(xcq_batch* b, const double* d_rho, double* d_fock,
                                   double* d_forces);
 long long xcq_static_scratch_bytes(void);
+/* Values of Y = P_g phi of a forces build on the current grid: *held those
+ * that the force pass takes from the density kernel, *all of them.  No
+ * reference counterpart. */
+int xcq_force_y(xcq_context* ctx, long long* held, long long* all);
+int xcq_batch_force_y(xcq_batch* b, long long* held, long long* all);
 int xcq_batch_atoms(xcq_batch* b, int* first_atom);
 int xcq_batch_capture(xcq_batch* b, const double* d_rho, double* d_fock);
 int xcq_batch_replay(xcq_batch* b);

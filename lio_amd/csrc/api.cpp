@@ -538,6 +538,14 @@ long long xcq_batch_arena_bytes(xcq_batch* b) {
   return b ? (long long)b->engine->arena_bytes() : -1;
 }
 
+int xcq_force_y(xcq_context* ctx, long long* held, long long* all) {
+  return guarded([&] { ctx->engine->force_y(held, all); });
+}
+
+int xcq_batch_force_y(xcq_batch* b, long long* held, long long* all) {
+  return guarded([&] { b->engine->force_y(held, all); });
+}
+
 int xcq_batch_load_ms(xcq_batch* b, double ms[4]) {
   return guarded([&] { b->engine->load_phases(ms); });
 }

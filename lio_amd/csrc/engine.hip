@@ -1735,7 +1735,7 @@ __global__ __launch_bounds__(256, 2) void k_density_dc(const ChunkItem* __restri
                                                        const DevGroup* __restrict__ groups,
                                                        const T* __restrict__ pg,
                                                        const T* __restrict__ vals,
-                                                       T* __restrict__ ybuf,
+                                                       T* __restrict__ ybuf, long long ylen,
                                                        double* __restrict__ cpart) {
   constexpr int NS = (NT == 4) ? 10 : 1;
   constexpr int RT = 4;
@@ -1828,7 +1828,9 @@ __global__ __launch_bounds__(256, 2) void k_density_dc(const ChunkItem* __restri
     if (kt + 1 < nk) slab(kt + 1, by, bx);
   }
   if (!active) return;
-  if (ybuf) {  // Y for the force pass, in the planes' layout (one plane per group)
+  // Y for the force pass, in the planes' layout (one plane per group), where
+  // the buffer holds the group's whole
+  if (g.val_off / (NT == 4 ? 10 : 4) + plane <= ylen) {
     T* Y = ybuf + g.val_off / (NT == 4 ? 10 : 4) + (V - (vals + g.val_off));
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
@@ -2620,15 +2622,18 @@ __device__ inline void force_rows(const double (&w)[12], int lrow, double (*slot
   }
 }
 
-// FP64 / FP32 values (tiled planes).  YS: Y from the density kernel's buffer
-// (8 or 4 bytes per point and function written and read again instead of
-// 2 n m^2 flops: HBM-bound); else recomputed from P_g as k_gather_density
-// leaves it, the same operations in the same order, for callers that allow no
-// allocation (or where none is left).  The sums are the same bit for bit.
-template <class T, bool YS>
+// FP64 / FP32 values (tiled planes).  Y comes from the density kernel's buffer
+// for the groups that lie whole in its first ylen values (8 or 4 bytes per
+// point and function written and read again instead of 2 n m^2 flops:
+// HBM-bound), and is recomputed from P_g as k_gather_density leaves it for the
+// others, the same operations in the same order.  The sums are the same bit
+// for bit.  ALL: it holds every group (60 atoms: 0.08 ms less than with the
+// product's code beside the loads).
+template <class T, bool ALL>
 __global__ __launch_bounds__(256, 2) void k_force(const DensityItem* __restrict__ items,
                                                   const DevGroup* __restrict__ groups,
                                                   const T* __restrict__ pg,
+                                                  const T* __restrict__ ybuf, long long ylen,
                                                   const T* __restrict__ vals, int nval,
                                                   const double* __restrict__ factor,
                                                   double* __restrict__ gpart) {
@@ -2644,7 +2649,8 @@ __global__ __launch_bounds__(256, 2) void k_force(const DensityItem* __restrict_
   const long long plane = (long long)mp * g.npts_pad;
   const long long tile = (long long)((active ? p0 : 0) >> 4) * (16 * mp);
   const T* V = vals + g.val_off + tile;
-  const T* Yp = YS ? pg + g.val_off / nval + tile : nullptr;
+  const bool stored = ALL || g.val_off / nval + plane <= ylen;
+  const T* Yp = ybuf + g.val_off / nval + tile;
   const T* Pm = pg + g.pg_off;
   const unsigned ve = 16 * Mma<T>::row(lk, 0) + lrow;
   const double f = active ? factor[g.pt_off + p0 + lrow] : 0.0;
@@ -2655,7 +2661,7 @@ __global__ __launch_bounds__(256, 2) void k_force(const DensityItem* __restrict_
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt) acc[rt] = typename Mma<T>::acc{0, 0, 0, 0};
     if (active) {
-      if constexpr (YS) {
+      if (stored) {
 #pragma unroll
         for (int rt = 0; rt < 4; ++rt)
           if (rt < nrt)
@@ -4174,23 +4180,33 @@ struct DeviceGrid {
   int *tfirst = nullptr, *torder = nullptr;  // tile evaluation blocks (tile_block)
   int ntile = 0;
   float* phiT = nullptr;          // function-major phi (split-BF16 Fock operand)
-  void* ybuf = nullptr;           // Y = P_g phi per point and function (force pass), in the
-                                  // planes' layout and type; allocated at the first forces
-                                  // build (not in the arena)
+  float* ybuf = nullptr;          // Y = P_g phi per point (split-BF16 forces), in the planes'
+                                  // layout; allocated at the first forces build (not in the
+                                  // arena)
   size_t ybuf_cap = 0;            // its bytes
-  bool y_denied = false;          // no memory for it: FP64 and FP32 forces recompute Y
+  bool ystored = true;            // FP64, FP32: keep Y where the arena has room (y_room)
   // P_g expansion: up to 256 blocks per group, each looping
   dim3 gather_grid() const {
     return dim3((unsigned)ngroups, (unsigned)std::max(
                                        1LL, std::min(256LL, ((long long)max_mpad * max_mpad + 255) / 256)));
   }
-  // values of Y per spin
-  long long yelems() const {
-    return prec == Precision::BF16X6 ? phi_elems : val_elems / nval;
-  }
-  size_t ybytes() const {
-    return (size_t)(open ? 2 : 1) * (size_t)yelems() *
-           (prec == Precision::FP64 ? sizeof(double) : sizeof(float));
+  // values of Y per spin (FP64, FP32)
+  long long yelems() const { return val_elems / nval; }
+  // Y of spin sp (0 or 1) for the FP64 and FP32 force passes, from the density
+  // launches to the force launches, which come before the Fock ones: at the
+  // arena's end, in the Fock matrix's buffers and the bytes asked for as
+  // headroom for larger grids.  *n gets how many of the spin's values they
+  // hold; the force pass recomputes those of the other groups, to the same
+  // bits.  So no memory is taken for Y and no call allocates any.  (A closed
+  // shell's Y is a tenth of its planes and fits beside a headroom of an
+  // eighth.  With buffers of their own the open shell's forces of (H2O)32 in
+  // FP64 took 5.7 ms, with this 5.8, with nothing kept 7.9.)
+  template <class T>
+  T* y_room(int sp, long long* n) const {
+    char* a = reinterpret_cast<char*>(fg);
+    const long long all = ystored ? (long long)((arena + arena_cap - a) / sizeof(T)) : 0;
+    *n = std::max(0LL, std::min(yelems(), all - sp * yelems()));
+    return reinterpret_cast<T*>(a) + sp * yelems();
   }
   DensityItem* ditems = nullptr;
   FockItem* fitems = nullptr;
@@ -4444,19 +4460,6 @@ static size_t pool_alloc(void** p, size_t want, size_t need, hipStream_t s, int 
   (void)hipGetLastError();
   XCQ_HIP(hipMallocAsync(p, need, s));
   return need;
-}
-
-// Device memory a new allocation could have: free, or cached unused in the
-// stream-ordered pool.
-static size_t obtainable_bytes(int device) {
-  size_t free_b = 0, total_b = 0;
-  XCQ_HIP(hipMemGetInfo(&free_b, &total_b));
-  hipMemPool_t pool;
-  uint64_t reserved = 0, used = 0;
-  XCQ_HIP(hipDeviceGetDefaultMemPool(&pool, device));
-  XCQ_HIP(hipMemPoolGetAttribute(pool, hipMemPoolAttrReservedMemCurrent, &reserved));
-  XCQ_HIP(hipMemPoolGetAttribute(pool, hipMemPoolAttrUsedMemCurrent, &used));
-  return free_b + (reserved > used ? reserved - used : 0);
 }
 
 // Returns an arena to the slab it came from (after the stream's work on it
@@ -5009,10 +5012,8 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
     dg->F = c.take<double>(nspin * packed);
     dg->vals = c.take<char>(vo * vbytes);
     dg->pg = c.take<char>(po * pbytes);
-    dg->fg = c.take<double>(po);
     dg->factor = c.take<double>(pt);
     dg->epart = c.take<double>(2 * ditems.size());
-    dg->fpart = c.take<double>((size_t)fitems.size() * kFnChunk * kFnChunk);
     dg->eout = c.take<double>(2 * nmol);
     dg->gpart = c.take<double>(go);
     dg->gsum = c.take<double>(3 * fnl.size());
@@ -5024,6 +5025,9 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
     dg->lo16 = c.take<unsigned short>(dg->lo ? fo : 0);
     dg->pcs = c.take<unsigned short>(dg->presplit ? 4 * fo : 0);
     dg->cpart = c.take<double>((size_t)npart * 10 * kDensPts);
+    // last: the Fock matrix's own buffers, which Y may take first (y_room)
+    dg->fg = c.take<double>(po);
+    dg->fpart = c.take<double>((size_t)fitems.size() * kFnChunk * kFnChunk);
   };
   Carver sizing{nullptr};
   plan(sizing);
@@ -5037,8 +5041,17 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
     // headroom (12.5 %, 25 % for a grid that outgrew its arena) so that the
     // grids of the next steps of a moving molecule fit the same arena
     const size_t want = dg->arena_bytes + (reclaim ? dg->arena_bytes / 4 : dg->arena_bytes / 8);
-    const size_t free_b = obtainable_bytes(device_);
+    size_t free_b = 0, total_b = 0;
     const bool slab = g_slab[device_].active();
+    XCQ_HIP(hipMemGetInfo(&free_b, &total_b));
+    {  // memory freed into the pool is available again
+      hipMemPool_t pool;
+      uint64_t reserved = 0, used = 0;
+      XCQ_HIP(hipDeviceGetDefaultMemPool(&pool, device_));
+      XCQ_HIP(hipMemPoolGetAttribute(pool, hipMemPoolAttrReservedMemCurrent, &reserved));
+      XCQ_HIP(hipMemPoolGetAttribute(pool, hipMemPoolAttrUsedMemCurrent, &used));
+      if (reserved > used) free_b += reserved - used;
+    }
     if (!slab && dg->arena_bytes > free_b + reclaim) {
       const size_t need = dg->arena_bytes;
       throw std::runtime_error("g2g: grid needs " + std::to_string(need >> 20) +
@@ -5068,7 +5081,7 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
   Carver carve{dg->arena};
   plan(carve);
   // the previous grid's Y buffer serves this one when large enough
-  if (old.g && old.g->ybuf && old.g->ybuf_cap >= dg->ybytes()) {
+  if (old.g && old.g->ybuf && old.g->ybuf_cap >= (size_t)(dg->open ? 2 : 1) * fo * sizeof(float)) {
     dg->ybuf = old.g->ybuf;
     dg->ybuf_cap = old.g->ybuf_cap;
     old.g->ybuf = nullptr;
@@ -5794,17 +5807,19 @@ static void launch_density_finish(DeviceGrid& g, hipStream_t s, int spin) {
 
 template <class T>
 static void launch_density(DeviceGrid& g, hipStream_t s, const double* d_rho, int spin,
-                           hipEvent_t* ev, void* yb) {
+                           hipEvent_t* ev, bool forces) {
   T* pg = static_cast<T*>(spin == 2 ? g.pg2 : g.pg);
   const double* rho = spin == 2 ? d_rho + g.packed : d_rho;
   if (g.ngroups > 0)
     hipLaunchKernelGGL(k_gather_density<T>, g.gather_grid(), dim3(256), 0, s, g.groups, g.mols,
                        g.fnl, rho, pg);
   if (spin < 2) mark(ev, 1, s);
+  long long ylen = 0;
+  T* y = g.y_room<T>(spin == 2 ? 1 : 0, &ylen);
   if (g.nchunk > 0)
     hipLaunchKernelGGL((g.gga ? k_density_dc<4, T> : k_density_dc<1, T>), dim3(g.nchunk),
-                       dim3(256), 0, s, g.chitems, g.groups, pg, static_cast<const T*>(g.vals),
-                       yb ? static_cast<T*>(yb) + (spin == 2 ? g.yelems() : 0) : nullptr, g.cpart);
+                       dim3(256), 0, s, g.chitems, g.groups, pg, static_cast<const T*>(g.vals), y,
+                       forces ? ylen : 0, g.cpart);
   launch_density_finish(g, s, spin);
   XCQ_HIP(hipGetLastError());
 }
@@ -5965,7 +5980,6 @@ static void launch_fock(DeviceGrid& g, hipStream_t s, const double* factor) {
 // Closed-shell split-BF16 builds whose density kernel is k_density_bf2
 // (variants 1, 2, 5) leave Y for the forces in ybuf.
 static bool ystore_forces(const DeviceGrid& g) {
-  if (g.prec != Precision::BF16X6) return g.ybuf != nullptr;  // both spins when open
   if (g.inkernel || g.lo) return g.ybuf != nullptr;  // both spins when open
   return g.prec == Precision::BF16X6 && !g.open && g.ybuf &&
          (g.density_variant == 1 || g.density_variant == 2 || g.density_variant == 5);
@@ -5974,14 +5988,11 @@ static bool ystore_forces(const DeviceGrid& g) {
 template <class T>
 static void launch_force_planes(DeviceGrid& g, hipStream_t s, const void* pg, int sp,
                                 const double* factor) {
-  const T* vals = static_cast<const T*>(g.vals);
-  if (ystore_forces(g))
-    hipLaunchKernelGGL((k_force<T, true>), dim3(g.nforce), dim3(256), 0, s, g.citems, g.groups,
-                       static_cast<const T*>(g.ybuf) + (sp == 1 ? g.yelems() : 0), vals, g.nval,
-                       factor, g.gpart);
-  else
-    hipLaunchKernelGGL((k_force<T, false>), dim3(g.nforce), dim3(256), 0, s, g.citems, g.groups,
-                       static_cast<const T*>(pg), vals, g.nval, factor, g.gpart);
+  long long ylen = 0;
+  const T* y = g.y_room<T>(sp, &ylen);
+  hipLaunchKernelGGL((ylen == g.yelems() ? k_force<T, true> : k_force<T, false>), dim3(g.nforce),
+                     dim3(256), 0, s, g.citems, g.groups, static_cast<const T*>(pg), y, ylen,
+                     static_cast<const T*>(g.vals), g.nval, factor, g.gpart);
 }
 
 static void launch_forces(DeviceGrid& g, hipStream_t s, double* d_forces) {
@@ -5996,12 +6007,12 @@ static void launch_forces(DeviceGrid& g, hipStream_t s, double* d_forces) {
         launch_force_planes<float>(g, s, pg, sp, factor);
       else if (g.inkernel)
         hipLaunchKernelGGL(k_force_ev, dim3(g.nforce), dim3(256), 0, s, g.citems, g.groups,
-                           static_cast<const float*>(g.ybuf) + (sp == 1 ? g.phi_elems : 0), g.fmeta, g.shells, g.tsh, g.bas,
+                           g.ybuf + (sp == 1 ? g.phi_elems : 0), g.fmeta, g.shells, g.tsh, g.bas,
                            g.px, g.py, g.pz, factor, g.gpart);
       else if (ystore_forces(g))
         hipLaunchKernelGGL(g.chunked ? k_force_y<true> : k_force_y<false>, dim3(g.nforce),
                            dim3(256), 0, s, g.citems, g.groups,
-                           static_cast<const float*>(g.ybuf) + (sp == 1 ? g.phi_elems : 0),
+                           g.ybuf + (sp == 1 ? g.phi_elems : 0),
                            static_cast<const float*>(g.vals), factor, g.gpart);
       else
         hipLaunchKernelGGL(k_force_bf, dim3(g.nforce), dim3(256), 0, s, g.citems, g.groups,
@@ -6031,7 +6042,7 @@ static void launch_all(DeviceGrid& g, hipStream_t s, const double* d_rho, double
     // not a memset, so the pair can be captured in a graph); the HIP-event
     // phases then read: expand = clearing, density = the whole build
     const PersistArgs& pa = g.pargs;
-    float* yb = d_forces && ystore_forces(g) ? static_cast<float*>(g.ybuf) : nullptr;
+    float* yb = d_forces && ystore_forces(g) ? g.ybuf : nullptr;
     hipLaunchKernelGGL(k_fill_int, dim3((g.nsync + 255) / 256), dim3(256), 0, s, pa.sync, g.nsync,
                        0);
     mark(ev, 1, s);
@@ -6055,13 +6066,16 @@ static void launch_all(DeviceGrid& g, hipStream_t s, const double* d_rho, double
   for (int sp = 0; sp < nspin; ++sp) {
     const int spin = g.open ? sp + 1 : 0;
     if (g.prec == Precision::FP64)
-      launch_density<double>(g, s, d_rho, spin, ev, ystore ? g.ybuf : nullptr);
+      launch_density<double>(g, s, d_rho, spin, ev, d_forces != nullptr);
     else if (g.prec == Precision::FP32)
-      launch_density<float>(g, s, d_rho, spin, ev, ystore ? g.ybuf : nullptr);
+      launch_density<float>(g, s, d_rho, spin, ev, d_forces != nullptr);
     else
-      launch_density_bf(g, s, d_rho, spin, ev, ystore ? static_cast<float*>(g.ybuf) : nullptr);
+      launch_density_bf(g, s, d_rho, spin, ev, ystore ? g.ybuf : nullptr);
   }
   mark(ev, 2, s);
+  // FP64 and FP32 forces first: their Y may lie in the Fock buffers
+  const bool first = g.prec != Precision::BF16X6;
+  if (d_forces && first) launch_forces(g, s, d_forces);
   for (int sp = 0; d_fock && sp < nspin; ++sp) {
     launch_fock(g, s, sp == 1 ? g.factor_b : g.factor);
     if (sp == 0) mark(ev, 3, s);
@@ -6077,28 +6091,20 @@ static void launch_all(DeviceGrid& g, hipStream_t s, const double* d_rho, double
   if (!d_fock) mark(ev, 3, s);
   hipLaunchKernelGGL(k_energy, dim3(g.nmol), dim3(1024), 0, s, g.epart, g.mols, g.eidx, g.eout);
   XCQ_HIP(hipGetLastError());
-  if (d_forces) launch_forces(g, s, d_forces);
+  if (d_forces && !first) launch_forces(g, s, d_forces);
   mark(ev, 4, s);
 }
 
-// The force passes read Y = P_g phi, which the density kernel leaves in a
-// buffer of its own (one value per padded point and function, per spin),
-// allocated at the first forces build of a grid: for split-BF16 from the
-// device slab when one is reserved, else from the stream-ordered pool.  FP64
-// and FP32 can recompute Y (the same bits), so they take the buffer (12.5 %
-// headroom for the grids of the next steps of a moving molecule) only from
-// plenty, at most an eighth of the obtainable memory and never from a slab:
-// no later grid is refused because of it.
+// The split-BF16 force passes read Y = P_g phi, which the density kernel
+// leaves in a buffer of its own (one FP32 value per padded point and function,
+// per spin): allocated at the first forces build of a grid, from the device
+// slab when one is reserved, else from the stream-ordered pool.  (FP64 and
+// FP32 can recompute Y: theirs lies where the arena has room, y_room.)
 static void ensure_ybuf(DeviceGrid& g, hipStream_t s, int device) {
-  if (g.ybuf || g.y_denied) return;
-  const bool must = g.prec == Precision::BF16X6;
-  const size_t need = g.ybytes() + 256, bytes = must ? need : need + need / 8;
+  if (g.prec != Precision::BF16X6 || g.ybuf) return;
+  const size_t bytes = (size_t)(g.open ? 2 : 1) * g.phi_elems * sizeof(float) + 256;
   Slab& sl = g_slab[device];
   void* p = nullptr;
-  if (!must && (sl.active() || bytes > obtainable_bytes(device) / 8)) {
-    g.y_denied = true;
-    return;
-  }
   if (sl.active()) {
     p = sl.take(bytes);
     if (!p)
@@ -6108,7 +6114,7 @@ static void ensure_ybuf(DeviceGrid& g, hipStream_t s, int device) {
   } else {
     g.ybuf_cap = pool_alloc(&p, bytes, bytes, s, device);
   }
-  g.ybuf = p;
+  g.ybuf = static_cast<float*>(p);
 }
 
 SolveResult Engine::solve_device(const double* d_rho, double* d_fock, bool want_energy,
@@ -6145,6 +6151,27 @@ static void* scratch_address(int device) {
   return g_scratch_ptr[device];
 }
 
+void Engine::force_y(long long* held, long long* all) const {
+  if (!grid_) throw std::runtime_error("g2g: no grid");
+  const DeviceGrid& g = *grid_;
+  const int nspin = g.open ? 2 : 1;
+  *held = *all = 0;
+  if (g.prec == Precision::BF16X6) {
+    *all = nspin * g.phi_elems;
+    if (ystore_forces(g)) *held = *all;
+    return;
+  }
+  for (int sp = 0; sp < nspin; ++sp) {
+    long long n = 0;
+    if (g.prec == Precision::FP64)
+      (void)g.y_room<double>(sp, &n);
+    else
+      (void)g.y_room<float>(sp, &n);
+    *held += n;
+    *all += g.yelems();
+  }
+}
+
 size_t Engine::static_scratch_bytes() { return kStaticScratchBytes; }
 
 SolveResult Engine::solve_device_static(const double* d_rho, double* d_fock, double* d_forces) {
@@ -6154,9 +6181,16 @@ SolveResult Engine::solve_device_static(const double* d_rho, double* d_fock, dou
                                                   g.density_variant == 2 ||
                                                   g.density_variant == 5));
   if (!d_forces || g.prec != Precision::BF16X6 || !ystore) {
-    // no Y buffer on these paths: no scratch beyond the grid's arena
-    launch_all(g, (hipStream_t)stream_, d_rho, d_fock, reinterpret_cast<hipEvent_t*>(events_),
-               d_forces);
+    // no Y kept on these paths: no scratch at all
+    g.ystored = false;
+    try {
+      launch_all(g, (hipStream_t)stream_, d_rho, d_fock, reinterpret_cast<hipEvent_t*>(events_),
+                 d_forces);
+    } catch (...) {
+      g.ystored = true;
+      throw;
+    }
+    g.ystored = true;
     return SolveResult{};
   }
   const size_t need = (size_t)(g.open ? 2 : 1) * (size_t)g.phi_elems * sizeof(float);
@@ -6167,7 +6201,7 @@ SolveResult Engine::solve_device_static(const double* d_rho, double* d_fock, dou
                              " MiB (use the allocating entry point)");
   float* y = static_cast<float*>(scratch_address(device_));
   XCQ_HIP(hipSetDevice(device_));
-  void* own = g.ybuf;  // the grid's own buffer (if any) is left untouched
+  float* own = g.ybuf;  // the grid's own buffer (if any) is left untouched
   g.ybuf = y;
   try {
     launch_all(g, (hipStream_t)stream_, d_rho, d_fock, reinterpret_cast<hipEvent_t*>(events_),

@@ -350,6 +350,9 @@ class Engine {
   char* upload_buffer();
   void upload_queued();
   const DeviceGrid* grid() const { return grid_; }
+  // Values of Y = P_g phi of a forces build on this grid: those the force pass
+  // takes from the density kernel (held) and all of them.
+  void force_y(long long* held, long long* all) const;
 
  private:
   int device_ = 0;

@@ -120,6 +120,8 @@ def load_library(path: str = LIB_PATH) -> C.CDLL:
     L.xcq_batch_arena_bytes.argtypes = [vp]
     L.xcq_batch_arena_bytes.restype = C.c_longlong
     L.xcq_batch_load_ms.argtypes = [vp, _dp]
+    L.xcq_force_y.argtypes = [vp, C.POINTER(C.c_longlong), C.POINTER(C.c_longlong)]
+    L.xcq_batch_force_y.argtypes = [vp, C.POINTER(C.c_longlong), C.POINTER(C.c_longlong)]
     L.xcq_batch_tune.argtypes = [vp, vp, vp, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int),
                                  C.c_int, _dp, C.POINTER(C.c_int)]
     L.xcq_set_schedule.argtypes = [vp, C.c_int, C.c_int]
@@ -355,6 +357,13 @@ class Context:
         from the next build_grid; bitwise the results of the phase launches."""
         _check(self.L.xcq_set_persistent(self.h, int(bool(on))), "xcq_set_persistent")
 
+    def force_y(self):
+        """(held, all): values of Y = P_g phi that a forces build on this grid
+        takes from the density kernel, and all of them."""
+        a, b = C.c_longlong(0), C.c_longlong(0)
+        _check(self.L.xcq_force_y(self.h, C.byref(a), C.byref(b)), "xcq_force_y")
+        return a.value, b.value
+
     def release_device(self):
         """Frees the device memory of this molecule; build_grid restores it."""
         _check(self.L.xcq_release_device(self.h), "xcq_release_device")
@@ -555,6 +564,12 @@ class Batch:
 
     def arena_bytes(self) -> int:
         return int(self.L.xcq_batch_arena_bytes(self.h))
+
+    def force_y(self):
+        """(held, all) as Context.force_y."""
+        a, b = C.c_longlong(0), C.c_longlong(0)
+        _check(self.L.xcq_batch_force_y(self.h, C.byref(a), C.byref(b)), "xcq_batch_force_y")
+        return a.value, b.value
 
     def load_ms(self):
         """Host wall time (ms) of the last load's phases: point weights

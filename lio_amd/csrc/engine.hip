@@ -5032,15 +5032,19 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
   Carver sizing{nullptr};
   plan(sizing);
   dg->arena_bytes = sizing.used + 256;
+  const size_t ybytes = (size_t)nspin * fo * sizeof(float);  // Y of split-BF16 forces
   if (old.g && old.g->arena && old.g->arena_cap >= dg->arena_bytes) {
     dg->arena = old.g->arena;
     dg->arena_cap = old.g->arena_cap;
     old.g->arena = nullptr;
   } else {
-    const size_t reclaim = old.g && old.g->arena ? old.g->arena_cap : 0;
+    size_t reclaim = old.g && old.g->arena ? old.g->arena_cap : 0;
     // headroom (12.5 %, 25 % for a grid that outgrew its arena) so that the
     // grids of the next steps of a moving molecule fit the same arena
     const size_t want = dg->arena_bytes + (reclaim ? dg->arena_bytes / 4 : dg->arena_bytes / 8);
+    // a Y buffer that is of no use to the new grid makes room for it
+    const bool drop_y = old.g && old.g->ybuf && (!bf || old.g->ybuf_cap < ybytes);
+    if (drop_y) reclaim += old.g->ybuf_cap;
     size_t free_b = 0, total_b = 0;
     const bool slab = g_slab[device_].active();
     XCQ_HIP(hipMemGetInfo(&free_b, &total_b));
@@ -5062,6 +5066,11 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
       free_arena(old.g->arena, old.g->arena_cap, device_, (hipStream_t)stream_);
       old.g->arena = nullptr;
     }
+    if (drop_y) {
+      free_arena(reinterpret_cast<char*>(old.g->ybuf), old.g->ybuf_cap, device_,
+                 (hipStream_t)stream_);
+      old.g->ybuf = nullptr;
+    }
     Slab& sl = g_slab[device_];
     if (sl.active()) {  // carve from the slab: exact size, no device call
       dg->arena = sl.take(dg->arena_bytes);
@@ -5081,7 +5090,7 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
   Carver carve{dg->arena};
   plan(carve);
   // the previous grid's Y buffer serves this one when large enough
-  if (old.g && old.g->ybuf && old.g->ybuf_cap >= (size_t)(dg->open ? 2 : 1) * fo * sizeof(float)) {
+  if (old.g && old.g->ybuf && old.g->ybuf_cap >= ybytes) {
     dg->ybuf = old.g->ybuf;
     dg->ybuf_cap = old.g->ybuf_cap;
     old.g->ybuf = nullptr;

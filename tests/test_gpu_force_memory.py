@@ -182,6 +182,46 @@ def test_forces_from_a_slab_equal_those_with_more_y_kept():
         assert np.array_equal(np.asarray(f), f0)
 
 
+GROW = r"""
+import json, sys
+sys.path.insert(0, %%(root)r)
+from lio_amd import g2g, systems
+def system(n):
+    Z, pos = systems.random_molecule_ang(n, 50 + n)
+    return systems.make_system("mol", Z, pos, seed=n)
+small, large = system(22), system(30)
+g2g.reserve_slab(%(slab)d)
+ctx = g2g.Context(small, precision="bf16x6")
+ctx.build_grid()
+ctx.solve_forces()
+ctx.set_precision("%(prec)s")
+ctx.set_system(large)
+ctx.build_grid()
+print("RESULT " + json.dumps(ctx.solve()[0]), flush=True)
+"""
+
+
+@pytest.mark.parametrize("prec", ["bf16x6", "fp32"])
+def test_a_larger_grid_takes_the_place_of_an_old_y(prec):
+    """The Y buffer of split-BF16 forces that a larger grid, or one of another
+    precision, cannot use is given back before that grid is placed: a slab
+    that holds the new grid alone takes it."""
+    _torch()
+    from lio_amd import g2g
+    ctx = g2g.Context(_system(22), precision="bf16x6")
+    first = ctx.build_grid()["arena_bytes"] + 4 * ctx.force_y()[1] + 1024
+    ctx.set_precision(prec)
+    middle = ctx.grid_info()["arena_bytes"]
+    ctx.set_system(_system(30))
+    second = ctx.build_grid()["arena_bytes"]
+    E = ctx.solve()[0]
+    ctx.close()
+    slab = max(first, middle, second) + (1 << 20)
+    print("arena and Y %d, then %d and %d, slab %d" % (first, middle, second, slab), flush=True)
+    assert second > first  # so old Y and new grid do not fit together
+    assert _child(GROW % {"slab": slab, "prec": prec}) == E
+
+
 @pytest.mark.parametrize("opened", [False, True])
 def test_captured_forces_replay(opened):
     """An FP64 forces call allocates nothing, so it can be captured: every

@@ -233,8 +233,8 @@ long long xcq_batch_arena_bytes(xcq_batch* b);
 /* Host wall time (ms) of the last load's phases, as xcq_grid_info.load_ms. */
 int xcq_batch_load_ms(xcq_batch* b, double ms[4]);
 /* Autotuner: times `reps` builds for every candidate schedule c < ncand --
- * Fock slice length slices[c] (points, multiple of 128) and, when variants is
- * not NULL, split-BF16 density kernel variants[c] (0: 64-function chunks, 1 and 2:
+ * Fock slice length slices[c] (points, multiple of 128, or XCQ_AUTO_SLICE)
+ * and, when variants is not NULL, split-BF16 density kernel variants[c] (0: 64-function chunks, 1 and 2:
  * 128- and 64-function chunks with LDS-staged density pieces, 3 and 4:
  * row-split 16-point blocks for groups above 64 functions, 5: 2 in the
  * radial-Hessian layout, 4 value planes instead of 10, 6 and 7: the basis
@@ -252,12 +252,18 @@ int xcq_batch_tune(xcq_batch* b, const double* d_rho, double* d_fock, int reps,
                    const int* slices, const int* variants, int ncand, double* ms_out,
                    int* best);
 /* Sets the schedule directly (a zero slice or a negative variant keeps that
- * knob): for a context it takes effect at the next xcq_build_grid, a batch
+ * knob, a slice of XCQ_AUTO_SLICE, the initial state, leaves the slice to the
+ * library): for a context it takes effect at the next xcq_build_grid, a batch
  * reloads at once.  No reference counterpart. */
+enum { XCQ_AUTO_SLICE = -1 };
+/* The slice length that XCQ_AUTO_SLICE gives groups of m_pad padded functions
+ * in this precision (XCQ_FP64, ...). */
+int xcq_auto_slice(int precision, int m_pad);
 int xcq_set_schedule(xcq_context* ctx, int fock_slice, int density_variant);
 int xcq_batch_set_schedule(xcq_batch* b, int fock_slice, int density_variant);
-/* The batch's schedule knobs (any pointer may be NULL).  No reference
- * counterpart. */
+/* The batch's schedule knobs (any pointer may be NULL); *fock_slice is
+ * XCQ_AUTO_SLICE where it depends on the group's size, so that the knobs read
+ * can be set again.  No reference counterpart. */
 int xcq_batch_get_schedule(xcq_batch* b, int* fock_slice, int* density_variant, int* persistent);
 /* on = 1: a closed-shell split-BF16 build with density variant 8 runs as one
  * persistent launch over an ordered queue of every phase's items (expansion,
@@ -271,7 +277,8 @@ int xcq_set_persistent(xcq_context* ctx, int on);
 /* Fock slice per group size bucket (the autotuner's schedule): groups of at
  * most m_hi[i] padded functions (m_hi ascending; the first bucket that holds
  * the group) take slices[i] points per Fock slice (multiples of 128), larger
- * groups the batch's fock_slice; nb = 0 clears the buckets.  Reloads. */
+ * groups the batch's fock_slice (automatic where that is XCQ_AUTO_SLICE);
+ * nb = 0 clears the buckets.  Reloads. */
 int xcq_batch_set_bucket_slices(xcq_batch* b, int nb, const int* m_hi, const int* slices);
 /* Padded function and point counts of every group of the batch (molecule
  * order); *ngroups gets the count, at most max entries are written. */

@@ -551,10 +551,7 @@ int xcq_batch_load_ms(xcq_batch* b, double ms[4]) {
 }
 
 static xcq::Tuning schedule(xcq::Tuning t, int fock_slice, int density_variant) {
-  if (fock_slice > 0) {
-    t.fock_slice = fock_slice;
-    t.default_slice = false;
-  }
+  if (fock_slice > 0 || fock_slice == xcq::kAutoSlice) t.fock_slice = fock_slice;
   if (density_variant >= 0) t.density_variant = density_variant;
   return t;
 }
@@ -581,6 +578,10 @@ int xcq_batch_set_bucket_slices(xcq_batch* b, int nb, const int* m_hi, const int
     b->engine->set_tuning(t);
     load_batch(b);
   });
+}
+
+int xcq_auto_slice(int precision, int m_pad) {
+  return xcq::Tuning::auto_slice(m_pad, precision == XCQ_BF16X6);
 }
 
 int xcq_batch_group_sizes(xcq_batch* b, int* m_pad, long long* npts_pad, int max, int* ngroups) {
@@ -618,7 +619,11 @@ int xcq_batch_set_persistent(xcq_batch* b, int on) {
 int xcq_batch_get_schedule(xcq_batch* b, int* fock_slice, int* density_variant, int* persistent) {
   return guarded([&] {
     const xcq::Tuning& t = b->engine->tuning();
-    if (fock_slice) *fock_slice = t.fock_slice;
+    // split-BF16's automatic slice is the same for every group: its length
+    if (fock_slice)
+      *fock_slice = t.fock_slice == xcq::kAutoSlice && b->prec == xcq::Precision::BF16X6
+                        ? xcq::Tuning::auto_slice(0, true)
+                        : t.fock_slice;
     if (density_variant) *density_variant = t.density_variant;
     if (persistent) *persistent = t.persistent;
   });
@@ -633,7 +638,6 @@ int xcq_batch_tune(xcq_batch* b, const double* d_rho, double* d_fock, int reps, 
     for (int c = 0; c < ncand; ++c) {
       xcq::Tuning t = b->engine->tuning();
       t.fock_slice = slices[c];
-      t.default_slice = false;
       if (variants) t.density_variant = variants[c];
       b->engine->set_tuning(t);
       load_batch(b);
@@ -652,7 +656,6 @@ int xcq_batch_tune(xcq_batch* b, const double* d_rho, double* d_fock, int reps, 
     }
     xcq::Tuning t = b->engine->tuning();
     t.fock_slice = slices[ibest];
-    t.default_slice = false;
     if (variants) t.density_variant = variants[ibest];
     b->engine->set_tuning(t);
     load_batch(b);

@@ -62,7 +62,6 @@ constexpr int kDensPts = 64;     // points per density block (16 per wave)
 constexpr int kRowSplitMin = 64; // split-BF16 row-split density above this m_pad
 constexpr int kFnChunk = 64;     // functions per density pass / Fock tile side
 constexpr int kXcds = 8;         // MI355X: XCDs, each with its own L2 (block b runs on b % 8)
-constexpr int kSliceDefault = 1024;  // points per Fock slice (split-K over blocks)
 constexpr int kPackMapMax = 8192;  // groups per molecule the packing kernel maps in LDS (64 KB)
 constexpr int kEvalPts = 256;    // threads per evaluation block
 constexpr int kEvalSpan = 4096;  // points (or elements) one evaluation block covers
@@ -4155,7 +4154,6 @@ double wall() {
 struct DeviceGrid {
   int M = 0, natom = 0, iexch = 9, nval = 10;  // M, natom: whole batch
   int nmol = 1, max_M = 0, max_ng = 0, max_mpad = 0;
-  int fock_slice = kSliceDefault;
   int density_variant = 10;
   int nrowsplit = 0;  // leading density items on the row-split kernel
   long long packed = 0;                 // packed entries of the whole batch
@@ -4546,7 +4544,8 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
   for (const Molecule* m : mols)
     if (m->gga != mols[0]->gga || m->iexch != mols[0]->iexch)
       throw std::runtime_error("g2g: the molecules of a batch must share the functional");
-  if (tuning_.fock_slice < 128 || tuning_.fock_slice % 128 != 0)
+  if (tuning_.fock_slice != kAutoSlice &&
+      (tuning_.fock_slice < 128 || tuning_.fock_slice % 128 != 0))
     throw std::runtime_error("g2g: the Fock slice must be a positive multiple of 128 points");
   if (tuning_.bucket_mhi.size() != tuning_.bucket_slice.size())
     throw std::runtime_error("g2g: one Fock slice per size bucket");
@@ -4565,7 +4564,6 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
     ~Guard() { release(g, s, device); }
   } guard{dg, (hipStream_t)stream_, device_};
   dg->nmol = nmol;
-  dg->fock_slice = tuning_.fock_slice;
   dg->density_variant = tuning_.density_variant;
 
   if (dg->density_variant < 0 || dg->density_variant > 11)

@@ -214,24 +214,27 @@ enum class Precision : int { FP64 = 0, FP32 = 1, BF16X6 = 2 };
 //               of at most bucket_mhi[i] padded functions (ascending; the
 //               first bucket that holds the group) take bucket_slice[i];
 //               larger groups, and every group when the lists are empty,
-//               take fock_slice.
+//               take fock_slice, or what the group's size gives where
+//               fock_slice is kAutoSlice.
+constexpr int kAutoSlice = -1;
 struct Tuning {
-  int fock_slice = 1024;
+  int fock_slice = kAutoSlice;
   int density_variant = 10;
   int persistent = 0;
   std::vector<int> bucket_mhi, bucket_slice;
-  // No slice was asked for: FP64 and FP32 groups take 256 points up to 128
+  // kAutoSlice: FP64 and FP32 groups take 256 points up to 128
   // functions (one to three blocks a slice, whose 64 steps of a 1024-point
   // slice would run alone: one water 24 us against 61, 25 atoms 215 against
   // 251), 512 up to 384 ((H2O)32 389 us against 418 with 256 and 406 with 1024
-  // throughout) and fock_slice above (100 atoms 2.71 ms against 2.80 with 512).
-  // Split-BF16's slices also decide where its FP32 sums end: always fock_slice.
-  bool default_slice = true;
+  // throughout) and 1024 above (100 atoms 2.71 ms against 2.80 with 512).
+  // Split-BF16's slices also decide where its FP32 sums end: always 1024.
+  static int auto_slice(int m_pad, bool split_bf16) {
+    return split_bf16 || m_pad > 384 ? 1024 : m_pad > 128 ? 512 : 256;
+  }
   int slice_for(int m_pad, bool split_bf16) const {
     for (size_t i = 0; i < bucket_mhi.size(); ++i)
       if (m_pad <= bucket_mhi[i]) return bucket_slice[i];
-    if (!default_slice || split_bf16) return fock_slice;
-    return m_pad <= 128 ? 256 : m_pad <= 384 ? 512 : fock_slice;
+    return fock_slice == kAutoSlice ? auto_slice(m_pad, split_bf16) : fock_slice;
   }
 };
 

@@ -28,6 +28,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 # built with AddressSanitizer by `make -C lio_amd/csrc asan`)
 LIB_PATH = os.environ.get("LIO_AMD_LIBRARY") or os.path.join(HERE, "libg2g.so")
 
+AUTO_SLICE = -1  # the Fock slice by the group's size, as the library chooses it
+
 _dp = C.POINTER(C.c_double)
 _up = C.POINTER(C.c_uint)
 _bp = C.POINTER(C.c_bool)
@@ -126,6 +128,7 @@ def load_library(path: str = LIB_PATH) -> C.CDLL:
                                  C.c_int, _dp, C.POINTER(C.c_int)]
     L.xcq_set_schedule.argtypes = [vp, C.c_int, C.c_int]
     L.xcq_reserve_slab.argtypes = [C.c_int, C.c_ulonglong]
+    L.xcq_auto_slice.argtypes = [C.c_int, C.c_int]
     L.xcq_batch_set_schedule.argtypes = [vp, C.c_int, C.c_int]
     L.xcq_set_persistent.argtypes = [vp, C.c_int]
     L.xcq_batch_set_persistent.argtypes = [vp, C.c_int]
@@ -192,6 +195,11 @@ def make_problem(system, **options):
     for k, v in opt.items():
         setattr(p, k, v)
     return p, keep
+
+
+def auto_slice(precision: str, m_pad: int) -> int:
+    """Points per Fock slice that AUTO_SLICE gives groups of m_pad functions."""
+    return int(load_library().xcq_auto_slice(PRECISION[precision], int(m_pad)))
 
 
 def _groups_to_dicts(arr):
@@ -349,7 +357,8 @@ class Context:
         return info.energy, F, dict(electrons=info.electrons)
 
     def set_schedule(self, fock_slice=0, density_variant=-1):
-        """Kernel schedule for the next build_grid (0 / -1 keep a knob)."""
+        """Kernel schedule for the next build_grid (0 / -1 keep a knob;
+        fock_slice AUTO_SLICE, the initial state, leaves it to the library)."""
         _check(self.L.xcq_set_schedule(self.h, fock_slice, density_variant), "xcq_set_schedule")
 
     def set_persistent(self, on: bool):
@@ -579,7 +588,8 @@ class Batch:
         return ms.tolist()
 
     def set_schedule(self, fock_slice=0, density_variant=-1):
-        """Sets the kernel schedule and reloads (0 / -1 keep a knob)."""
+        """Sets the kernel schedule and reloads (0 / -1 keep a knob;
+        fock_slice AUTO_SLICE, the initial state, leaves it to the library)."""
         _check(self.L.xcq_batch_set_schedule(self.h, fock_slice, density_variant),
                "xcq_batch_set_schedule")
 
@@ -590,14 +600,15 @@ class Batch:
         _check(self.L.xcq_batch_set_persistent(self.h, int(bool(on))), "xcq_batch_set_persistent")
 
     def schedule(self) -> dict:
-        """The batch's schedule knobs: fock_slice, density_variant, persistent."""
+        """The batch's schedule knobs: fock_slice (AUTO_SLICE where it depends
+        on the group's size), density_variant, persistent."""
         a, b, c = C.c_int(0), C.c_int(0), C.c_int(0)
         _check(self.L.xcq_batch_get_schedule(self.h, C.byref(a), C.byref(b), C.byref(c)),
                "xcq_batch_get_schedule")
         return {"fock_slice": a.value, "density_variant": b.value, "persistent": bool(c.value)}
 
-    def tune(self, d_rho: int, d_fock: int, slices=(256, 512, 1024, 2048), variants=None,
-             reps: int = 5):
+    def tune(self, d_rho: int, d_fock: int, slices=(AUTO_SLICE, 256, 512, 1024, 2048),
+             variants=None, reps: int = 5):
         """Autotunes the schedule on these buffers over the candidates
         (slices[c], variants[c]) -- or every slice with the current density
         variant when variants is None; returns (best (slice, variant or None),
@@ -660,7 +671,8 @@ class Batch:
         buckets[i] padded functions; larger groups form the last bucket) is
         chosen by timing whole builds on these buffers, one bucket at a time,
         heaviest bucket (sum of n m^2) first, the others held at their best so
-        far; then, in split-BF16 mode, one persistent launch (density variant
+        far, from the faster of two starts, the automatic slice of each
+        bucket's bound and 1024 points throughout; then, in split-BF16 mode, one persistent launch (density variant
         8) against one launch per phase with the batch's density variant.
         The result is written to ``path`` (when given) and returned: bucket
         bounds and slices, the launch form and density variant, the ms per
@@ -683,13 +695,18 @@ class Batch:
         which = np.searchsorted(np.array(edges), m, side="left")
         work = np.zeros(nb)
         np.add.at(work, which, p.astype(np.float64) * m.astype(np.float64) ** 2)
-        choice = [1024] * nb
         table = {}
         self.set_persistent(False)
         variant = self.schedule()["density_variant"]
-        self.set_bucket_slices(edges, choice)
-        best = self._time_builds(d_rho, d_fock, reps)
-        table["start"] = best
+        best, choice = np.inf, None
+        for name, start in (("automatic", [auto_slice(self.precision, e) for e in edges]),
+                            ("1024 throughout", [1024] * nb)):
+            if start == choice:
+                continue
+            self.set_bucket_slices(edges, start)
+            table[name] = ms = self._time_builds(d_rho, d_fock, reps)
+            if ms < best:
+                best, choice = ms, start
         for b in np.argsort(-work):
             if work[b] == 0:
                 continue

@@ -33,6 +33,7 @@
 #include <chrono>
 #include <map>
 #include <atomic>
+#include <climits>
 #include <mutex>
 #include <cstdio>
 #include <cstring>
@@ -62,7 +63,9 @@ constexpr int kDensPts = 64;     // points per density block (16 per wave)
 constexpr int kRowSplitMin = 64; // split-BF16 row-split density above this m_pad
 constexpr int kFnChunk = 64;     // functions per density pass / Fock tile side
 constexpr int kXcds = 8;         // MI355X: XCDs, each with its own L2 (block b runs on b % 8)
-constexpr int kPackMapMax = 8192;  // groups per molecule the packing kernel maps in LDS (64 KB)
+// groups the packing kernel maps in LDS at a time (64 KB): as rows of F_g, as
+// local indices
+constexpr int kPackRows = 8192, kPackIndices = 16384;
 constexpr int kEvalPts = 256;    // threads per evaluation block
 constexpr int kEvalSpan = 4096;  // points (or elements) one evaluation block covers
 
@@ -3055,8 +3058,13 @@ __global__ __launch_bounds__(256) void k_fock_group(const DevGroup* __restrict__
 // kPackLanes-th entry, and a butterfly adds them: the walk is a few loads deep
 // instead of one or two per group (latency bounds it: (H2O)32 42 -> 26 us,
 // one water 16 -> 6, 195 atoms 660 -> 400 with one thread per J and the
-// group looked up for every entry).
+// group looked up for every entry).  For a molecule of more than kPackRows
+// groups the map holds I's local indices (Row = int), half the bytes, of
+// kPackIndices groups at a time, and the group is looked up for every entry
+// after all (four waters in 9932 groups: 1.5 ms, merging the two lists in one
+// thread per J 9.4; in 18476 groups 2.9 against 17.5).
 constexpr int kPackLanes = 8, kPackCols = 256 / kPackLanes;
+template <class Row>
 __global__ __launch_bounds__(256) void k_fock_pack(const int* __restrict__ memb_off,
                                                    const int2* __restrict__ memb,
                                                    const DevGroup* __restrict__ groups,
@@ -3064,7 +3072,9 @@ __global__ __launch_bounds__(256) void k_fock_pack(const int* __restrict__ memb_
                                                    const int* __restrict__ fn_mol,
                                                    const double* __restrict__ fg,
                                                    double* __restrict__ F) {
-  extern __shared__ long long srow[];
+  extern __shared__ long long smap[];
+  Row* srow = reinterpret_cast<Row*>(smap);
+  constexpr bool kRows = sizeof(Row) == 8;
   const int I = blockIdx.y;
   const DevMol mol = mols[fn_mol[I]];
   const int j0 = blockIdx.x * kPackCols;
@@ -3073,19 +3083,51 @@ __global__ __launch_bounds__(256) void k_fock_pack(const int* __restrict__ memb_
   const bool in = J < mol.fn_base + mol.M && J >= I;
   const int l = threadIdx.x % kPackLanes;
   const int b0 = in ? memb_off[J] : 0, be = in ? memb_off[J + 1] : 0;
-  for (int q = threadIdx.x; q < mol.ng; q += 256) srow[q] = -1;
-  __syncthreads();
-  for (int a = memb_off[I] + threadIdx.x; a < memb_off[I + 1]; a += 256) {
-    const int2 u = memb[a];
-    srow[u.x - mol.g0] = groups[u.x].pg_off + (long long)u.y * groups[u.x].m_pad;
-  }
-  __syncthreads();
   double s = 0.0;
+  int b = b0 + l;
+  // groups [g0, g0 + n) of the batch in the map
+  auto map_groups = [&](int g0, int n) {
+    for (int q = threadIdx.x; q < n; q += 256) srow[q] = -1;
+    __syncthreads();
+    for (int a = memb_off[I] + threadIdx.x; a < memb_off[I + 1]; a += 256) {
+      const int2 u = memb[a];
+      if (!kRows && (unsigned)(u.x - g0) >= (unsigned)n) continue;
+      srow[u.x - g0] = kRows ? (Row)(groups[u.x].pg_off + (long long)u.y * groups[u.x].m_pad)
+                             : (Row)u.y;
+    }
+    __syncthreads();
+  };
+  // this lane's entries below e
+  auto add = [&](int g0, int e) {
 #pragma unroll 4
-  for (int b = b0 + l; b < be; b += kPackLanes) {
-    const int2 v = memb[b];
-    const long long r = srow[v.x - mol.g0];
-    if (r >= 0) s += fg[r + v.y];
+    for (; b < e; b += kPackLanes) {
+      const int2 v = memb[b];
+      const Row r = srow[v.x - g0];
+      if (r < 0) continue;
+      if constexpr (kRows)
+        s += fg[r + v.y];
+      else
+        s += fg[groups[v.x].pg_off + (long long)r * groups[v.x].m_pad + v.y];
+    }
+  };
+  if constexpr (kRows) {
+    map_groups(mol.g0, mol.ng);
+    add(mol.g0, be);
+  } else {
+    int e = b0;
+    for (int w = 0; w < mol.ng; w += kPackIndices) {
+      const int n = min(kPackIndices, mol.ng - w), end = mol.g0 + w + n;
+      if (w) __syncthreads();  // every lane is done with the map before
+      map_groups(mol.g0 + w, n);
+      for (int hi = be; e < hi;) {  // J's first entry past these groups
+        const int mid = (e + hi) >> 1;
+        if (memb[mid].x < end)
+          e = mid + 1;
+        else
+          hi = mid;
+      }
+      add(mol.g0 + w, e);
+    }
   }
 #pragma unroll
   for (int o = 1; o < kPackLanes; o <<= 1) s += __shfl_xor(s, o);
@@ -3093,52 +3135,31 @@ __global__ __launch_bounds__(256) void k_fock_pack(const int* __restrict__ memb_
     F[mol.rho_off + packed_index(I - mol.fn_base, J - mol.fn_base, mol.M)] = s;
 }
 
-// The sum of k_fock_pack in one thread: entry i of J's list belongs to lane
-// i % kPackLanes, the lanes added as the butterfly does.
-struct PackSum {
+// The sum of k_fock_pack in one thread, for the persistent build: entry i of
+// J's list [b, be) belongs to lane i % kPackLanes, the lanes added as the
+// butterfly does, so J's list is walked kPackLanes entries at a time beside I's
+// [a, ae).
+__device__ inline double merge_sum(const int2* memb, int a, int ae, int b, int be,
+                                   const DevGroup* groups, const double* fg) {
   double s[kPackLanes] = {};
-  __device__ inline void add(int i, double x) {
+  int2 u = a < ae ? memb[a] : make_int2(INT_MAX, 0);
+  for (; b < be; b += kPackLanes) {
 #pragma unroll
-    for (int k = 0; k < kPackLanes; ++k) s[k] += (i % kPackLanes) == k ? x : 0.0;
-  }
-  __device__ inline double total() {
-#pragma unroll
-    for (int o = 1; o < kPackLanes; o <<= 1)
-#pragma unroll
-      for (int k = 0; k < kPackLanes; k += 2 * o) s[k] += s[k + o];
-    return s[0];
-  }
-};
-
-// The same by merging the two sorted lists, for molecules with more groups
-// than the LDS map holds.
-__global__ void k_fock_pack_merge(const int* __restrict__ memb_off, const int2* __restrict__ memb,
-                            const DevGroup* __restrict__ groups, const DevMol* __restrict__ mols,
-                            const int* __restrict__ fn_mol, const double* __restrict__ fg,
-                            double* __restrict__ F) {
-  const int I = blockIdx.y;
-  const DevMol mol = mols[fn_mol[I]];
-  const int J = mol.fn_base + blockIdx.x * blockDim.x + threadIdx.x;
-  if (J >= mol.fn_base + mol.M || J < I) return;
-  int a = memb_off[I], ae = memb_off[I + 1];
-  int b = memb_off[J], be = memb_off[J + 1];
-  const int b0 = b;
-  PackSum s;
-  while (a < ae && b < be) {
-    const int2 u = memb[a], v = memb[b];
-    if (u.x < v.x) {
-      ++a;
-    } else if (v.x < u.x) {
-      ++b;
-    } else {
-      const DevGroup g = groups[u.x];
-      const int li = min(u.y, v.y), lj = max(u.y, v.y);
-      s.add(b - b0, fg[g.pg_off + (long long)li * g.m_pad + lj]);
-      ++a;
-      ++b;
+    for (int k = 0; k < kPackLanes; ++k) {
+      if (b + k >= be) break;
+      const int2 v = memb[b + k];
+      while (u.x < v.x) u = ++a < ae ? memb[a] : make_int2(INT_MAX, 0);
+      if (u.x == v.x) {
+        const DevGroup& g = groups[u.x];
+        s[k] += fg[g.pg_off + (long long)min(u.y, v.y) * g.m_pad + max(u.y, v.y)];
+      }
     }
   }
-  F[mol.rho_off + packed_index(I - mol.fn_base, J - mol.fn_base, mol.M)] = s.total();
+#pragma unroll
+  for (int o = 1; o < kPackLanes; o <<= 1)
+#pragma unroll
+    for (int k = 0; k < kPackLanes; k += 2 * o) s[k] += s[k + o];
+  return s[0];
 }
 
 // Fixed-order reduction of the per-block (Exc, N) pairs of each molecule
@@ -3341,26 +3362,10 @@ __global__ __launch_bounds__(256, 2) void k_build_persist(PersistArgs* pargs, in
       const int I = pi.x;
       const DevMol mol = a.mols[a.fn_mol[I]];
       const int J = mol.fn_base + pi.y * 256 + (int)threadIdx.x;
-      if (J < mol.fn_base + mol.M && J >= I) {
-        int u0 = a.memb_off[I], ue = a.memb_off[I + 1];
-        int v0 = a.memb_off[J], ve = a.memb_off[J + 1];
-        PackSum sum;
-        while (u0 < ue && v0 < ve) {
-          const int2 u = a.memb[u0], v = a.memb[v0];
-          if (u.x < v.x) {
-            ++u0;
-          } else if (v.x < u.x) {
-            ++v0;
-          } else {
-            const DevGroup gg = a.groups[u.x];
-            const int li = min(u.y, v.y), lj = max(u.y, v.y);
-            sum.add(v0 - a.memb_off[J], a.fg[gg.pg_off + (long long)li * gg.m_pad + lj]);
-            ++u0;
-            ++v0;
-          }
-        }
-        F[mol.rho_off + packed_index(I - mol.fn_base, J - mol.fn_base, mol.M)] = sum.total();
-      }
+      if (J < mol.fn_base + mol.M && J >= I)
+        F[mol.rho_off + packed_index(I - mol.fn_base, J - mol.fn_base, mol.M)] =
+            merge_sum(a.memb, a.memb_off[I], a.memb_off[I + 1], a.memb_off[J], a.memb_off[J + 1],
+                      a.groups, a.fg);
     } else {
       // energies: the 1024-lane fixed-order reduction of the phase launch,
       // four lanes per thread
@@ -6086,14 +6091,12 @@ static void launch_all(DeviceGrid& g, hipStream_t s, const double* d_rho, double
   for (int sp = 0; d_fock && sp < nspin; ++sp) {
     launch_fock(g, s, sp == 1 ? g.factor_b : g.factor);
     if (sp == 0) mark(ev, 3, s);
-    if (g.max_ng <= kPackMapMax)
-      hipLaunchKernelGGL(k_fock_pack, dim3((g.max_M + kPackCols - 1) / kPackCols, g.M), dim3(256),
-                         (size_t)g.max_ng * sizeof(long long), s, g.memb_off, g.memb, g.groups, g.mols,
-                         g.fn_mol, g.fg, d_fock + sp * g.packed);
-    else
-      hipLaunchKernelGGL(k_fock_pack_merge, dim3((g.max_M + 127) / 128, g.M), dim3(128), 0, s,
-                         g.memb_off, g.memb, g.groups, g.mols, g.fn_mol, g.fg,
-                         d_fock + sp * g.packed);
+    const bool rows = g.max_ng <= kPackRows;
+    hipLaunchKernelGGL((rows ? k_fock_pack<long long> : k_fock_pack<int>),
+                       dim3((g.max_M + kPackCols - 1) / kPackCols, g.M), dim3(256),
+                       std::min(g.max_ng, kPackIndices) * (rows ? sizeof(long long) : sizeof(int)),
+                       s, g.memb_off, g.memb, g.groups, g.mols, g.fn_mol, g.fg,
+                       d_fock + sp * g.packed);
   }
   if (!d_fock) mark(ev, 3, s);
   hipLaunchKernelGGL(k_energy, dim3(g.nmol), dim3(1024), 0, s, g.epart, g.mols, g.eidx, g.eout);

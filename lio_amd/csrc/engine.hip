@@ -4247,7 +4247,7 @@ struct DeviceGrid {
   unsigned short* pcs = nullptr;  // those pieces: 4 planes of phi_elems BF16
   ChunkItem* chitems = nullptr;   // its blocks in dispatch order (XCD-interleaved)
   int nchunk = 0;
-  double* cpart = nullptr;        // per (point tile, chunk): 10 x 64 row-dot sums
+  double* cpart = nullptr;        // per (point tile, chunk): 10 (LDA 1) x 64 row-dot sums
   ChunkItem* finitems = nullptr;  // per point tile (k_density_cs_finish)
   int* forder = nullptr;          // Fock blocks: item per block (XCD-interleaved)
   int nfock_order = 0;
@@ -5027,7 +5027,7 @@ void Engine::load_batch_impl(const std::vector<const Molecule*>& mols,
     dg->rad = c.take<float>(ro);
     dg->lo16 = c.take<unsigned short>(dg->lo ? fo : 0);
     dg->pcs = c.take<unsigned short>(dg->presplit ? 4 * fo : 0);
-    dg->cpart = c.take<double>((size_t)npart * 10 * kDensPts);
+    dg->cpart = c.take<double>((size_t)npart * (dg->gga ? 10 : 1) * kDensPts);
     // last: the Fock matrix's own buffers, which Y may take first (y_room)
     dg->fg = c.take<double>(po);
     dg->fpart = c.take<double>((size_t)fitems.size() * kFnChunk * kFnChunk);

@@ -182,6 +182,33 @@ def test_forces_from_a_slab_equal_those_with_more_y_kept():
         assert np.array_equal(np.asarray(f), f0)
 
 
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("iexch", [9, 2])
+def test_bytes_of_a_grid(precision, iexch):
+    """A grid's bytes are its planes, P_g and F_g per group, the slices'
+    partial Fock tiles, the density's partial sums (ten per point and chunk of
+    64 functions, one in LDA), the force sums, six values per point, and lists
+    of under 32 MB."""
+    _torch()
+    from lio_amd import g2g
+    b = g2g.Batch([_system(45, iexch=iexch)], precision=precision)
+    m, p = (x.astype(np.int64) for x in b.group_sizes())
+    item = 8 if precision == "fp64" else 4
+    planes = (10 if iexch == 9 else 4) * item * int((m * p).sum())
+    blocks = int((m * m).sum())
+    tiles, chunks = (m + 63) // 64, (p + 63) // 64 * ((m + 63) // 64)
+    sl = np.array([g2g.auto_slice(precision, x) for x in m])
+    fpart = int((tiles * (tiles + 1) // 2 * ((p + sl - 1) // sl)).sum()) * 64 * 64 * 8
+    cpart = int(chunks.sum()) * (10 if iexch == 9 else 1) * 64 * 8
+    force = 24 * int(((p + 63) // 64 * m).sum())
+    bound = planes + item * blocks + 8 * blocks + fpart + cpart + force \
+        + 48 * int(p.sum()) + (32 << 20)
+    print(precision, iexch, "arena", b.arena_bytes(), "bound", bound, "sums", cpart, flush=True)
+    got = b.arena_bytes()
+    b.close()
+    assert got <= bound
+
+
 GROW = r"""
 import json, sys
 sys.path.insert(0, %%(root)r)

@@ -2629,9 +2629,10 @@ __device__ inline void force_rows(const double (&w)[12], int lrow, double (*slot
 // point and function written and read again instead of 2 n m^2 flops:
 // HBM-bound), and is recomputed from P_g as k_gather_density leaves it for the
 // others, the same operations in the same order.  The sums are the same bit
-// for bit.  ALL: it holds every group (60 atoms: 0.08 ms less than with the
-// product's code beside the loads).
-template <class T, bool ALL>
+// for bit.  (Each of the two ways has a walk of its own: with the branch inside
+// one walk Y's loads were kept from those of the planes: 60 atoms, all stored,
+// 0.08 ms more, (H2O)32, none stored, 3.88 ms the call against 3.75.)
+template <class T>
 __global__ __launch_bounds__(256, 2) void k_force(const DensityItem* __restrict__ items,
                                                   const DevGroup* __restrict__ groups,
                                                   const T* __restrict__ pg,
@@ -2651,63 +2652,68 @@ __global__ __launch_bounds__(256, 2) void k_force(const DensityItem* __restrict_
   const long long plane = (long long)mp * g.npts_pad;
   const long long tile = (long long)((active ? p0 : 0) >> 4) * (16 * mp);
   const T* V = vals + g.val_off + tile;
-  const bool stored = ALL || g.val_off / nval + plane <= ylen;
   const T* Yp = ybuf + g.val_off / nval + tile;
   const T* Pm = pg + g.pg_off;
   const unsigned ve = 16 * Mma<T>::row(lk, 0) + lrow;
   const double f = active ? factor[g.pt_off + p0 + lrow] : 0.0;
   double* out = gpart + g.force_off + (long long)(it.p0 / kDensPts) * mp * 3;
-  for (int c0 = 0; c0 < mp; c0 += kFnChunk) {
-    const int nrt = min(4, (mp - c0) / 16);
-    typename Mma<T>::acc acc[4];
+  auto walk = [&](auto ys) {
+    for (int c0 = 0; c0 < mp; c0 += kFnChunk) {
+      const int nrt = min(4, (mp - c0) / 16);
+      typename Mma<T>::acc acc[4];
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) acc[rt] = typename Mma<T>::acc{0, 0, 0, 0};
-    if (active) {
-      if (stored) {
+      for (int rt = 0; rt < 4; ++rt) acc[rt] = typename Mma<T>::acc{0, 0, 0, 0};
+      if (active) {
+        if constexpr (decltype(ys)::value) {
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt)
-          if (rt < nrt)
+          for (int rt = 0; rt < 4; ++rt)
+            if (rt < nrt)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-              acc[rt][i] = (Yp + 16 * (c0 + 16 * rt + Mma<T>::row(0, i)))[ve];
-      } else {
-        const T* Bk = V + 16 * lk + lrow;  // phi[k][p]
-        for (int k0 = 0; k0 < mp; k0 += 4) {
-          const T b = Bk[16 * k0];
+              for (int i = 0; i < 4; ++i)
+                acc[rt][i] = (Yp + 16 * (c0 + 16 * rt + Mma<T>::row(0, i)))[ve];
+        } else {
+          const T* Bk = V + 16 * lk + lrow;  // phi[k][p]
+          for (int k0 = 0; k0 < mp; k0 += 4) {
+            const T b = Bk[16 * k0];
 #pragma unroll
-          for (int rt = 0; rt < 4; ++rt) {
-            if (rt >= nrt) continue;
-            const T a = Pm[((long long)(c0 / 16 + rt) * (mp >> 3) + (k0 >> 3)) * 128 + 2 * lane +
-                           ((k0 >> 2) & 1)];
-            Mma<T>::op(a, b, acc[rt]);
+            for (int rt = 0; rt < 4; ++rt) {
+              if (rt >= nrt) continue;
+              const T a = Pm[((long long)(c0 / 16 + rt) * (mp >> 3) + (k0 >> 3)) * 128 + 2 * lane +
+                             ((k0 >> 2) & 1)];
+              Mma<T>::op(a, b, acc[rt]);
+            }
           }
         }
       }
-    }
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-      double w[12];
-      int jj[4];
+      for (int rt = 0; rt < 4; ++rt) {
+        double w[12];
+        int jj[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        jj[i] = 16 * rt + Mma<T>::row(lk, i);
-        const T* vj = V + 16 * (c0 + 16 * rt + Mma<T>::row(0, i));
-        const double y = f * (double)acc[rt][i];
+        for (int i = 0; i < 4; ++i) {
+          jj[i] = 16 * rt + Mma<T>::row(lk, i);
+          const T* vj = V + 16 * (c0 + 16 * rt + Mma<T>::row(0, i));
+          const double y = f * (double)acc[rt][i];
 #pragma unroll
-        for (int a = 0; a < 3; ++a)
-          w[3 * i + a] = active && rt < nrt ? y * (double)(vj + (a + 1) * plane)[ve] : 0.0;
+          for (int a = 0; a < 3; ++a)
+            w[3 * i + a] = active && rt < nrt ? y * (double)(vj + (a + 1) * plane)[ve] : 0.0;
+        }
+        force_rows(w, lrow, sG[wave], jj);
       }
-      force_rows(w, lrow, sG[wave], jj);
+      __syncthreads();
+      if (threadIdx.x < 3 * kFnChunk) {
+        const int jj = threadIdx.x / 3, a = threadIdx.x % 3;
+        if (c0 + jj < mp)
+          out[(long long)(c0 + jj) * 3 + a] =
+              ((sG[0][jj][a] + sG[1][jj][a]) + sG[2][jj][a]) + sG[3][jj][a];
+      }
+      __syncthreads();
     }
-    __syncthreads();
-    if (threadIdx.x < 3 * kFnChunk) {
-      const int jj = threadIdx.x / 3, a = threadIdx.x % 3;
-      if (c0 + jj < mp)
-        out[(long long)(c0 + jj) * 3 + a] =
-            ((sG[0][jj][a] + sG[1][jj][a]) + sG[2][jj][a]) + sG[3][jj][a];
-    }
-    __syncthreads();
-  }
+  };
+  if (g.val_off / nval + plane <= ylen)
+    walk(std::true_type());
+  else
+    walk(std::false_type());
 }
 
 // Split-BF16 values (point-major FP32 planes, P_g as three BF16 pieces): Y on
@@ -4203,7 +4209,8 @@ struct DeviceGrid {
   // bits.  So no memory is taken for Y and no call allocates any.  (A closed
   // shell's Y is a tenth of its planes and fits beside a headroom of an
   // eighth.  With buffers of their own the open shell's forces of (H2O)32 in
-  // FP64 took 5.7 ms, with this 5.8, with nothing kept 7.9.)
+  // FP64 took 5.71 ms, with this 5.78, with nothing kept 7.5; LDA of 45 atoms
+  // 1.29, 1.37, 2.14.)
   template <class T>
   T* y_room(int sp, long long* n) const {
     char* a = reinterpret_cast<char*>(fg);
@@ -6002,9 +6009,9 @@ static void launch_force_planes(DeviceGrid& g, hipStream_t s, const void* pg, in
                                 const double* factor) {
   long long ylen = 0;
   const T* y = g.y_room<T>(sp, &ylen);
-  hipLaunchKernelGGL((ylen == g.yelems() ? k_force<T, true> : k_force<T, false>), dim3(g.nforce),
-                     dim3(256), 0, s, g.citems, g.groups, static_cast<const T*>(pg), y, ylen,
-                     static_cast<const T*>(g.vals), g.nval, factor, g.gpart);
+  hipLaunchKernelGGL(k_force<T>, dim3(g.nforce), dim3(256), 0, s, g.citems, g.groups,
+                     static_cast<const T*>(pg), y, ylen, static_cast<const T*>(g.vals), g.nval,
+                     factor, g.gpart);
 }
 
 static void launch_forces(DeviceGrid& g, hipStream_t s, double* d_forces) {

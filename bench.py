@@ -59,8 +59,8 @@ DENSITY_KERNEL = "k_density_cs<4, false> + k_density_cs_finish<4>"
 # WRITE_SIZE x 1.0 in KiB (copy-kernel calibrated) of both launches, measured
 # on the tree named in DENSITY_TRAFFIC_TREE (profiles/xc_fock_h2o32.md gives
 # the command)
-DENSITY_TRAFFIC = ((2358634 + 57239) * 2.0 + (106171 + 59226) * 1.0) * 1024
-DENSITY_TRAFFIC_TREE = "57a446f"
+DENSITY_TRAFFIC = ((2357470 + 56190) * 2.0 + (106171 + 5543) * 1.0) * 1024
+DENSITY_TRAFFIC_TREE = "9be3b1b"
 
 
 def log(*a):

@@ -84,6 +84,8 @@ typedef struct {
 
 const char* xcq_last_error(void);
 
+/* A context or batch holds 4 MiB of pinned host memory for the tables of its
+ * grid loads until it is destroyed. */
 int xcq_create(int device, xcq_context** out);
 int xcq_destroy(xcq_context* ctx);
 int xcq_set_problem(xcq_context* ctx, const xcq_problem* problem);

@@ -14,7 +14,7 @@
 //                      rho, Hessian of rho
 //   k_density_cs_finish  the chunks' shares added, PBE/LDA
 //                      -> factor_p = w_p v_p and per-tile (Exc, N)
-//   k_fock             F_g tile (64 x 64) over a 512-point slice,
+//   k_fock             F_g tile (64 x 64) over a slice of the points,
 //                      phi^T diag(factor) phi on FP64 MFMA, one partial/slice
 //   k_fock_group       sums the slices of each tile in fixed order
 //   k_fock_pack        packed F_IJ = sum over groups holding I and J, in
@@ -1459,8 +1459,9 @@ __global__ __launch_bounds__(256) void k_split_pm(const DensityItem* __restrict_
 // the functional with one lane per point (the density blocks hold each point
 // on four lanes, a quarter of the wave).
 //
-// What bounds it: the SIMDs' issue.  A K step is about 600 VALU instructions
-// (the split of the B operand) of 4 cycles and 112 MFMA of 16, and the two
+// What bounds it: the SIMDs' issue.  A K step is about 520 VALU instructions
+// (391 of them the split of the B operand) of 4 cycles and 112 MFMA of 16 ((H2O)32,
+// epilogue included: VALU 52 % of the cycles, MFMA 31 %), and the two
 // overlap little on this GPU (two waves a SIMD alternating 384 FMA and 96
 // MFMA take 4.7 ms where the sum is 5.3, fully interleaved 4.1), so the time
 // is near their sum as long as the operands arrive.  The tiled planes and the
@@ -1723,8 +1724,8 @@ __global__ __launch_bounds__(256) void k_density_cs_finish(const ChunkItem* __re
 // cpart and k_density_cs_finish adds the chunks and evaluates the functional.
 //
 // What bounds it: the FP64 unit for large groups (the matrix products keep it
-// busy 69 % of the time at 60 atoms, the epilogue's FMAs, which it shares with
-// them, another 7 %), HBM for small ones ((H2O)32: 9.1 GB at 5.1 TB/s, the
+// busy 68 % of the cycles at 60 atoms, the other vector instructions, which
+// do not overlap them, another 5 %), HBM for small ones ((H2O)32: 9.1 GB at 5.1 TB/s, the
 // epilogue's ten planes and the K loop's four).  Against one block per tile
 // walking the chunks with four full products: (H2O)32 2.47 -> 1.83 ms, 60
 // atoms 8.9 -> 5.6 ms, 45 atoms LDA 0.89 -> 0.60 ms.  Taking the diagonal
@@ -2818,8 +2819,8 @@ __global__ __launch_bounds__(256, 2) void k_force_bf(const DensityItem* __restri
   }
 }
 
-// Split-BF16 forces from the Y = P_g phi the density kernel left in ybuf
-// (point-major, exact FP32 sums): the same per-function sums as k_force_bf,
+// Split-BF16 forces from the Y = P_g phi the density kernel left in ybuf (in
+// the planes' layout, tiled or point-major; exact FP32 sums): the same per-function sums as k_force_bf,
 // in the same lane and wave order, without recomputing the product.
 template <bool TL>
 __global__ __launch_bounds__(256) void k_force_y(const DensityItem* __restrict__ items,
@@ -2954,13 +2955,12 @@ __global__ __launch_bounds__(256) void k_force_ev(const DensityItem* __restrict_
   }
 }
 
-// gsum[fn_off + j][a] = sum over the group's blocks (in order) of gpart; one
-// block per group.
+// gsum[fn_off + j][a] = sum over the group's point blocks of gpart; blockIdx.x
+// the group, blockIdx.y 64 of its elements.
 // accumulate: add onto gsum (the second spin of an open shell).
-// One thread per (group, element), blockIdx.x the group; the loads of
-// several blocks are in flight together, the sum stays in block order.
-// (Four threads per element, each a quarter of the blocks by turns, added in
-// thread order: a sphere's 73 blocks are 19 loads in a row, not 73.)
+// Four threads per element, each taking every fourth point block in order with
+// several loads in flight, added in thread order: a sphere's 73 blocks are 19
+// loads in a row, not 73.
 __global__ __launch_bounds__(256) void k_force_group(const DevGroup* __restrict__ groups,
                                                      const double* __restrict__ gpart,
                                                      double* __restrict__ gsum, int accumulate) {
@@ -4259,7 +4259,7 @@ struct DeviceGrid {
   int* forder = nullptr;          // Fock blocks: item per block (XCD-interleaved)
   int nfock_order = 0;
   int nfin = 0;
-  unsigned short* lo16 = nullptr; // phi's remainder in BF16, point-major (phi_elems)
+  unsigned short* lo16 = nullptr; // phi's remainder in BF16, in the planes' layout (phi_elems)
   bool persistent = false;        // one persistent launch per build (k_build_persist)
   PersistArgs pargs{};            // its queue and tables (device pointers)
   PersistArgs* dpargs = nullptr;  // device copy of pargs, read by the kernel
@@ -5996,8 +5996,9 @@ static void launch_fock(DeviceGrid& g, hipStream_t s, const double* factor) {
 // XC forces after the density launches (P_g blocks and factors in place):
 // per-block partials and group sums per spin, then per-atom sums into
 // d_forces (natom x 3, atom-major).
-// Closed-shell split-BF16 builds whose density kernel is k_density_bf2
-// (variants 1, 2, 5) leave Y for the forces in ybuf.
+// Split-BF16: whether the density launch leaves Y for the forces in ybuf (the
+// in-kernel variants and 8 to 11 for both spins; variants 1, 2 and 5 for a
+// closed shell).
 static bool ystore_forces(const DeviceGrid& g) {
   if (g.inkernel || g.lo) return g.ybuf != nullptr;  // both spins when open
   return g.prec == Precision::BF16X6 && !g.open && g.ybuf &&
@@ -6080,7 +6081,7 @@ static void launch_all(DeviceGrid& g, hipStream_t s, const double* d_rho, double
     return;
   }
   const int nspin = g.open ? 2 : 1;
-  // closed-shell split-BF16 forces take Y = P_g phi from the density pass
+  // split-BF16 forces that take Y = P_g phi from the density pass
   const bool ystore = d_forces && ystore_forces(g);
   for (int sp = 0; sp < nspin; ++sp) {
     const int spin = g.open ? sp + 1 : 0;
